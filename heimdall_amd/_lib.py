@@ -38,6 +38,10 @@ SIGNATURES = {
     "bf_gate_project_workspace_size": (_c_int, [_c_i64, _c_int, _c_int, ctypes.POINTER(_c_sz)]),
     "bf_gate_project": (_c_int, [_vp, _c_i64, _c_int, _c_i64, _vp, _vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp,
                                  _c_sz, _vp]),
+    "bf_student_inputs_max_tokens": (_c_i64, []),
+    "bf_student_inputs_workspace_size": (_c_int, [_c_i64] + [_c_int] * 4 + [ctypes.POINTER(_c_sz)]),
+    "bf_student_inputs": (_c_int, [_vp, _c_i64] + [_vp, _c_i64, _c_i64] * 2 + [_c_i64, _c_i64] + [_c_int] * 4 + [_vp] * 9
+                          + [_c_i64, _c_int, _vp, _vp, _c_int] + [_vp] * 4 + [_c_sz, _vp]),
     "bf_gdn_conv_inputs": (_c_int, [_vp, _c_i64, _vp, _c_int, _vp, _c_int] + [_vp] * 5 + [_c_int, _c_i64]
                            + [_c_int] * 3 + [_fp, _fp] + [_vp] * 5 + [_c_int, _vp]),
     "bf_gated_norm": (_c_int, [_vp, _c_int, _vp, _vp, _c_i64, _c_int, _fp, _vp, _c_int, _vp]),

@@ -169,6 +169,50 @@ __device__ __forceinline__ int tfrag_index(int row, int col) {
     return ((ks * 4 + tt) * 64 + 16 * lg + l16) * VEC + e;
 }
 
+// p[0] + p[stride] + .. over the n split partials of a sum, added in split order. The loads of 16 partials go out
+// together: one at a time, the 40 partials of a decode step's gate sums took 10 us of memory round trips.
+__device__ __forceinline__ float split_sum(const float* p, long stride, int n) {
+    float s = 0.f;
+    for (int i = 0; i < n; i += 16) {
+        float v[16];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) v[j] = p[(long)(i + j < n ? i + j : n - 1) * stride];
+#pragma unroll
+        for (int j = 0; j < 16; ++j) s = i + j < n ? s + v[j] : s;
+    }
+    return s;
+}
+
+// The memory gates from the logits of the ab projection: g = -exp(A_log) softplus(a + dt_bias) decay_mask (softplus
+// with torch's default threshold), beta = sigmoid(b).
+__device__ __forceinline__ float mem_gate_g(float a, float dt_bias, float A_log, float mask) {
+    const float x = a + dt_bias;
+    const float sp = x > 20.f ? x : log1pf(expf(x));
+    return -expf(A_log) * sp * mask;
+}
+__device__ __forceinline__ float mem_gate_beta(float b) { return 1.f / (1.f + expf(-b)); }
+
+// Sum of squares of a row of D floats by 4 consecutive lanes (lane & 3 = part), the same value in each. Lane part
+// takes elements 16 j + 4 part .. + 3, j ascending, and the parts are added as (0 + 1) + (2 + 3): the order of
+// mem_project_kernel's norm, so a row normalised here has its bits.
+template <int D>
+__device__ __forceinline__ float row_square_sum(const float* row, int part) {
+    float4 v[D / 16];
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) v[j] = *reinterpret_cast<const float4*>(row + 16 * j + 4 * part);
+    float ss = 0.f;
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) {
+        ss += v[j].x * v[j].x;
+        ss += v[j].y * v[j].y;
+        ss += v[j].z * v[j].z;
+        ss += v[j].w * v[j].w;
+    }
+    ss += __shfl_xor(ss, 1);
+    ss += __shfl_xor(ss, 2);
+    return ss;
+}
+
 __device__ __forceinline__ int lane_id() { return threadIdx.x & (WAVE - 1); }
 // Wave index inside the workgroup, marked wave-uniform (readfirstlane) so that values derived from it (buffer
 // descriptors, LDS bases, loop bounds) live in SGPRs; plain threadIdx.x / 64 is treated as divergent and descriptors

@@ -86,6 +86,12 @@ struct DecodeArgs {
     float* state;             // [B][G][D][D]
     float* o;                 // [B][H][D]
     float* lse;               // [B][H] or null
+    // The memory inputs as student_front leaves them (gp_part null: as above): qm and km hold the unnormalised
+    // projections, and g_new, beta_new and z are the sums of the gate partials [gp_ns][B][2 G + H] with the biases.
+    const float* gp_part;
+    int gp_ns;
+    float q_scale;
+    const float *b_ab, *b_mix, *A_log, *dt_bias, *decay_mask;
     int nsplit, slots;        // window splits of `slots` ring slots (decode_split)
     float* ws_om;             // [B][H][D] memory read
     float* ws_part;           // [B][G][nsplit][R][D + 2] window partials
@@ -285,6 +291,12 @@ inline int gate_project_nsplit(long n_tok, int d) {
     long ns = 1024 / (tiles > 0 ? tiles : 1);
     return (int)(ns < 1 ? 1 : (ns > steps ? steps : ns));
 }
+// splits that hold at least one 128-wide step, *per steps each
+inline int gate_project_splits(long n_tok, int d, int* per) {
+    const int ns = gate_project_nsplit(n_tok, d), steps = (d + 127) / 128;
+    *per = (steps + ns - 1) / ns;
+    return (steps + *per - 1) / *per;
+}
 inline int gate_project_wsplit_substeps(int d) { return 2 * ((d + 255) / 256); }
 inline size_t gate_project_workspace(long n_tok, int d, int nout) {
     if (n_tok > GP_SPLIT_MAX_TOK)
@@ -293,6 +305,26 @@ inline size_t gate_project_workspace(long n_tok, int d, int nout) {
 }
 int gate_project_dispatch(const GateProjArgs& a, hipStream_t stream);
 int mem_project_dispatch(const MemProjArgs& a, hipStream_t stream);
+
+// The memory inputs of a few tokens (student_front). Above FRONT_MAX_TOK the tiled kernels are the faster ones.
+constexpr long FRONT_MAX_TOK = 256;
+struct FrontArgs {
+    GateProjArgs gp;                // x, W, the split partials (part), n_tok; out0 / out1 unused
+    int gp_ns, gp_per;              // set by student_front
+    const void *q, *k;              // bf16 rows: token t, head h at q + t * q_st + h * q_sh (elements), D contiguous
+    long q_st, q_sh, k_st, k_sh;
+    const float *fq, *fk;           // [H][D][D], [G][D][D]
+    int H, G, D;
+    float *yq, *yk;                 // [n_tok][H][D], [n_tok][G][D]: the unnormalised projections
+    // the finish pass (chunks)
+    void *qm, *km;                  // [n_tok][H][D], [n_tok][G][D] in out_dtype
+    int out_dtype, sinks;
+    float q_scale;
+    long start, T;                  // position of each sequence's first token, tokens per sequence
+    const float *A_log, *dt_bias, *decay_mask;
+    float *g, *beta, *z;            // [n_tok][G], [n_tok][G], [n_tok][H]
+};
+int student_front(FrontArgs& a, bool finish, hipStream_t stream);
 int window_fa_dispatch(const WinArgs& a, hipStream_t stream);
 
 struct KvArgs {
@@ -371,6 +403,11 @@ struct LayerArgs {
     const float* s_new;
     float* state;
 };
+// The memory branch of a chunk of up to FEW_MAX_T tokens: the write stream and the reads token by token (fp32), the
+// state updated in place from s_in (null: zero), the reads into o_mem [B][T][H][D] fp32 (decode.hip).
+constexpr int FEW_MAX_T = 16;
+int few_mem_dispatch(const LayerArgs& a, const float* s_in, hipStream_t stream);
+
 int layer_launch(const LayerArgs& a, int what, hipStream_t s);   // 0 stream, 1 place, 2 write-back, 3 state, 4 query
 
 struct KvAppendArgs {

@@ -236,28 +236,36 @@ int bf_decode_workspace_size(int B, int G, int R, int D, int W, size_t* bytes) {
     return BF_STATUS_OK;
 }
 
-int bf_decode_fwd(int B, int G, int R, int D, int W, int sinks, int64_t pos, int memory, int kv_dtype, int q_dtype,
-                  const void* qr, const float* qm, const void* kr, const void* v, const float* km, const float* g_new,
-                  const float* beta_new, const float* z, const float* mix_lse, const float* mem_scale,
-                  const void* sink_k, const void* sink_v, int n_sinks, void* ring_k, void* ring_v, float* ring_km,
-                  float* ring_g, float* ring_beta, int64_t* ring_pos, float* state, float* o, float* lse,
-                  void* workspace, size_t workspace_bytes, void* stream) {
-    if (B <= 0 || G <= 0 || R <= 0 || W <= 0 || sinks < 0 || pos < 0) return BF_STATUS_INVALID;
+}  // extern "C"
+
+namespace {
+
+// Checks a decode step's arguments and fills `a` (its other fields stay): one shared position `pos`, or per-sequence
+// positions pos_arr on the device (any sequence may then read its memory, so its inputs must be given).
+int decode_args(bf::DecodeArgs& a, int B, int G, int R, int D, int W, int sinks, int64_t pos, const int64_t* pos_arr,
+                int memory, int kv_dtype, int q_dtype, const void* qr, const float* qm, const void* kr, const void* v,
+                const float* km, const float* g_new, const float* beta_new, const float* z, const float* mix_lse,
+                const float* mem_scale, const void* sink_k, const void* sink_v, int n_sinks, void* ring_k,
+                void* ring_v, float* ring_km, float* ring_g, float* ring_beta, int64_t* ring_pos, float* state,
+                float* o, float* lse, void* workspace, size_t workspace_bytes) {
+    if (B <= 0 || G <= 0 || R <= 0 || W <= 0 || sinks < 0 || (!pos_arr && pos < 0) || (pos_arr && sinks > 63))
+        return BF_STATUS_INVALID;
     if (!supported_dim(D) || R > 8 || !supported_dtype(kv_dtype) || !supported_dtype(q_dtype))
         return BF_STATUS_UNSUPPORTED;
+    if (pos_arr) n_sinks = sinks;                       // a fixed sink block per sequence
     if (n_sinks < 0 || n_sinks > 63 || n_sinks > sinks || (n_sinks > 0 && (!sink_k || !sink_v)))
         return BF_STATUS_INVALID;
     if (!qr || !kr || !v || !km || !g_new || !beta_new || !ring_k || !ring_v || !ring_km || !ring_g || !ring_beta ||
         !ring_pos || !o)
         return BF_STATUS_INVALID;
-    const int mem_on = memory && pos >= W;
+    const int mem_on = memory && (pos_arr || pos >= W);
     if (mem_on && (!qm || !z || !mix_lse || !mem_scale || !state)) return BF_STATUS_INVALID;
     size_t need = 0;
     const int st = bf_decode_workspace_size(B, G, R, D, W, &need);
     if (st) return st;
     if (!workspace || workspace_bytes < need) return BF_STATUS_WORKSPACE;
-    bf::DecodeArgs a{};
-    a.B = B; a.G = G; a.R = R; a.D = D; a.W = W; a.sinks = sinks; a.pos = pos; a.mem_on = mem_on;
+    a.B = B; a.G = G; a.R = R; a.D = D; a.W = W; a.sinks = sinks; a.pos = pos_arr ? 0 : pos; a.pos_arr = pos_arr;
+    a.mem_on = mem_on;
     a.kv_dtype = kv_dtype; a.q_dtype = q_dtype;
     a.qr = qr; a.qm = qm; a.kr = kr; a.v = v; a.km = km; a.g_new = g_new; a.beta_new = beta_new;
     a.z = z; a.mix_lse = mix_lse; a.mem_scale = mem_scale;
@@ -270,7 +278,24 @@ int bf_decode_fwd(int B, int G, int R, int D, int W, int sinks, int64_t pos, int
     a.ws_part = reinterpret_cast<float*>(ws + align256((size_t)B * G * R * D * sizeof(float)));
     a.ws_ev = reinterpret_cast<float*>(reinterpret_cast<char*>(a.ws_part) +
                                        align256((size_t)B * G * a.nsplit * R * (D + 2) * sizeof(float)));
-    return bf::decode_dispatch(a, static_cast<hipStream_t>(stream));
+    return BF_STATUS_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int bf_decode_fwd(int B, int G, int R, int D, int W, int sinks, int64_t pos, int memory, int kv_dtype, int q_dtype,
+                  const void* qr, const float* qm, const void* kr, const void* v, const float* km, const float* g_new,
+                  const float* beta_new, const float* z, const float* mix_lse, const float* mem_scale,
+                  const void* sink_k, const void* sink_v, int n_sinks, void* ring_k, void* ring_v, float* ring_km,
+                  float* ring_g, float* ring_beta, int64_t* ring_pos, float* state, float* o, float* lse,
+                  void* workspace, size_t workspace_bytes, void* stream) {
+    bf::DecodeArgs a{};
+    const int st = decode_args(a, B, G, R, D, W, sinks, pos, nullptr, memory, kv_dtype, q_dtype, qr, qm, kr, v, km,
+                               g_new, beta_new, z, mix_lse, mem_scale, sink_k, sink_v, n_sinks, ring_k, ring_v, ring_km,
+                               ring_g, ring_beta, ring_pos, state, o, lse, workspace, workspace_bytes);
+    return st ? st : bf::decode_dispatch(a, static_cast<hipStream_t>(stream));
 }
 
 int bf_decode_fwd_batch(int B, int G, int R, int D, int W, int sinks, const int64_t* pos, int memory, int kv_dtype,
@@ -279,34 +304,66 @@ int bf_decode_fwd_batch(int B, int G, int R, int D, int W, int sinks, const int6
                         const float* mem_scale, void* sink_k, void* sink_v, void* ring_k, void* ring_v, float* ring_km,
                         float* ring_g, float* ring_beta, int64_t* ring_pos, float* state, float* o, float* lse,
                         void* workspace, size_t workspace_bytes, void* stream) {
-    if (B <= 0 || G <= 0 || R <= 0 || W <= 0 || sinks < 0 || sinks > 63 || !pos) return BF_STATUS_INVALID;
-    if (!supported_dim(D) || R > 8 || !supported_dtype(kv_dtype) || !supported_dtype(q_dtype))
-        return BF_STATUS_UNSUPPORTED;
-    if (sinks > 0 && (!sink_k || !sink_v)) return BF_STATUS_INVALID;
-    if (!qr || !kr || !v || !km || !g_new || !beta_new || !ring_k || !ring_v || !ring_km || !ring_g || !ring_beta ||
-        !ring_pos || !o)
-        return BF_STATUS_INVALID;
-    // the positions live on the device: any sequence may read its memory, so its inputs must be given
-    if (memory && (!qm || !z || !mix_lse || !mem_scale || !state)) return BF_STATUS_INVALID;
-    size_t need = 0;
-    const int st = bf_decode_workspace_size(B, G, R, D, W, &need);
-    if (st) return st;
-    if (!workspace || workspace_bytes < need) return BF_STATUS_WORKSPACE;
+    if (!pos) return BF_STATUS_INVALID;
     bf::DecodeArgs a{};
-    a.B = B; a.G = G; a.R = R; a.D = D; a.W = W; a.sinks = sinks; a.pos = 0; a.pos_arr = pos; a.mem_on = memory != 0;
-    a.kv_dtype = kv_dtype; a.q_dtype = q_dtype;
-    a.qr = qr; a.qm = qm; a.kr = kr; a.v = v; a.km = km; a.g_new = g_new; a.beta_new = beta_new;
-    a.z = z; a.mix_lse = mix_lse; a.mem_scale = mem_scale;
-    a.sink_k = sink_k; a.sink_v = sink_v; a.n_sinks = sinks;
-    a.ring_k = ring_k; a.ring_v = ring_v; a.ring_km = ring_km; a.ring_g = ring_g; a.ring_beta = ring_beta;
-    a.ring_pos = ring_pos; a.state = state; a.o = o; a.lse = lse;
-    bf::decode_split(B, G, W, a.nsplit, a.slots);
+    const int st = decode_args(a, B, G, R, D, W, sinks, 0, pos, memory, kv_dtype, q_dtype, qr, qm, kr, v, km, g_new,
+                               beta_new, z, mix_lse, mem_scale, sink_k, sink_v, sinks, ring_k, ring_v, ring_km, ring_g,
+                               ring_beta, ring_pos, state, o, lse, workspace, workspace_bytes);
+    return st ? st : bf::decode_dispatch(a, static_cast<hipStream_t>(stream));
+}
+
+// The memory inputs of a chunk of a few tokens (bf16 activations).
+static void student_inputs_layout(int64_t n_tok, int H, int G, int D, int d_model, size_t (&at)[4]) {
+    at[0] = 0;
+    at[1] = at[0] + align256((size_t)n_tok * H * D * sizeof(float));
+    at[2] = at[1] + align256((size_t)n_tok * G * D * sizeof(float));
+    at[3] = at[2] + align256(bf::gate_project_workspace(n_tok, d_model, 2 * G + H));
+}
+
+int64_t bf_student_inputs_max_tokens(void) { return bf::FRONT_MAX_TOK; }
+
+int bf_student_inputs_workspace_size(int64_t n_tok, int H, int G, int D, int d_model, size_t* bytes) {
+    if (!bytes || n_tok <= 0 || n_tok > bf::FRONT_MAX_TOK || H <= 0 || G <= 0 || d_model <= 0) return BF_STATUS_INVALID;
+    if (!supported_dim(D)) return BF_STATUS_UNSUPPORTED;
+    size_t at[4];
+    student_inputs_layout(n_tok, H, G, D, d_model, at);
+    *bytes = at[3];
+    return BF_STATUS_OK;
+}
+
+int bf_student_inputs(const void* x, int64_t x_st, const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_st,
+                      int64_t k_sh, int64_t n_tok, int64_t T, int H, int G, int D, int d_model, const float* fq,
+                      const float* fk, const float* w_ab, const float* b_ab, const float* w_mix, const float* b_mix,
+                      const float* A_log, const float* dt_bias, const float* decay_mask, int64_t start, int sinks,
+                      void* qm, void* km, int out_dtype, float* g, float* beta, float* z, void* workspace,
+                      size_t workspace_bytes, void* stream) {
+    size_t need = 0;
+    const int st = bf_student_inputs_workspace_size(n_tok, H, G, D, d_model, &need);
+    if (st) return st;
+    if (!supported_dtype(out_dtype)) return BF_STATUS_UNSUPPORTED;
+    if (T <= 0 || n_tok % T || d_model % 8 || x_st % 8 || x_st < d_model || 2 * G + H > bf::GP_MAX_OUT || start < 0 ||
+        sinks < 0 || q_st <= 0 || q_sh < 0 || k_st <= 0 || k_sh < 0 || q_st > (1 << 26) || k_st > (1 << 26))
+        return BF_STATUS_INVALID;
+    if (!x || !q || !k || !fq || !fk || !w_ab || !w_mix || !A_log || !dt_bias || !decay_mask || !qm || !km || !g ||
+        !beta || !z)
+        return BF_STATUS_INVALID;
+    for (const void* p : {x, (const void*)w_ab, (const void*)w_mix, (const void*)qm, (const void*)km})
+        if ((uintptr_t)p & 15) return BF_STATUS_INVALID;
+    if (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 255)) return BF_STATUS_WORKSPACE;
+    size_t at[4];
+    student_inputs_layout(n_tok, H, G, D, d_model, at);
     char* ws = static_cast<char*>(workspace);
-    a.ws_om = reinterpret_cast<float*>(ws);
-    a.ws_part = reinterpret_cast<float*>(ws + align256((size_t)B * G * R * D * sizeof(float)));
-    a.ws_ev = reinterpret_cast<float*>(reinterpret_cast<char*>(a.ws_part) +
-                                       align256((size_t)B * G * a.nsplit * R * (D + 2) * sizeof(float)));
-    return bf::decode_dispatch(a, static_cast<hipStream_t>(stream));
+    bf::FrontArgs f{};
+    f.gp.x = static_cast<const uint16_t*>(x); f.gp.n_tok = n_tok; f.gp.x_st = x_st; f.gp.d = d_model;
+    f.gp.w0 = w_ab; f.gp.b0 = b_ab; f.gp.n0 = 2 * G; f.gp.w1 = w_mix; f.gp.b1 = b_mix; f.gp.n1 = H;
+    f.gp.part = reinterpret_cast<float*>(ws + at[2]);
+    f.q = q; f.q_st = q_st; f.q_sh = q_sh; f.k = k; f.k_st = k_st; f.k_sh = k_sh;
+    f.fq = fq; f.fk = fk; f.H = H; f.G = G; f.D = D;
+    f.yq = reinterpret_cast<float*>(ws + at[0]); f.yk = reinterpret_cast<float*>(ws + at[1]);
+    f.qm = qm; f.km = km; f.out_dtype = out_dtype; f.sinks = sinks; f.q_scale = 1.f / sqrtf((float)D);
+    f.start = start; f.T = T; f.A_log = A_log; f.dt_bias = dt_bias; f.decay_mask = decay_mask;
+    f.g = g; f.beta = beta; f.z = z;
+    return bf::student_front(f, true, static_cast<hipStream_t>(stream));
 }
 
 // One decode step of the converted layer from the layer's own inputs (bf16 activations): the gate projections, the
@@ -371,13 +428,30 @@ int bf_student_decode(int B, int H, int G, int D, int W, int sinks, int64_t pos,
     float *qm = reinterpret_cast<float*>(ws + l.qm), *km = reinterpret_cast<float*>(ws + l.km);
     float *g = reinterpret_cast<float*>(ws + l.g), *beta = reinterpret_cast<float*>(ws + l.beta);
     const hipStream_t s = static_cast<hipStream_t>(stream);
-    {
-        bf::GateProjArgs a{};
-        a.x = static_cast<const uint16_t*>(x); a.n_tok = B; a.x_st = d_model; a.d = d_model;
-        a.w0 = w_ab; a.b0 = b_ab; a.n0 = 2 * G; a.out0 = ab; a.w1 = w_mix; a.b1 = b_mix; a.n1 = H; a.out1 = z;
-        a.part = reinterpret_cast<float*>(ws + l.gp);
-        if ((st = bf::gate_project_dispatch(a, s))) return st;
+    bf::GateProjArgs gp{};
+    gp.x = static_cast<const uint16_t*>(x); gp.n_tok = B; gp.x_st = d_model; gp.d = d_model;
+    gp.w0 = w_ab; gp.b0 = b_ab; gp.n0 = 2 * G; gp.out0 = ab; gp.w1 = w_mix; gp.b1 = b_mix; gp.n1 = H; gp.out1 = z;
+    gp.part = reinterpret_cast<float*>(ws + l.gp);
+    void* dws = ws + l.dec;
+    const size_t dn = workspace_bytes - l.dec;
+    if (B <= bf::FRONT_MAX_TOK) {
+        // one launch for both projections; the decode tail finishes their norms and the gate sums
+        bf::FrontArgs f{};
+        f.gp = gp; f.q = q; f.k = k; f.q_st = (long)H * D; f.k_st = (long)G * D; f.q_sh = f.k_sh = D;
+        f.fq = fq; f.fk = fk; f.H = H; f.G = G; f.D = D; f.yq = qm; f.yk = km;
+        bf::DecodeArgs raw{};
+        raw.gp_part = gp.part; raw.q_scale = 1.f / sqrtf((float)D);
+        raw.b_ab = b_ab; raw.b_mix = b_mix; raw.A_log = A_log; raw.dt_bias = dt_bias; raw.decay_mask = decay_mask;
+        // g, beta and z stand for the sums of gp_part: never read
+        if ((st = decode_args(raw, B, G, H / G, D, W, sinks, pos, pos_arr, memory, BF_DTYPE_BF16, BF_DTYPE_BF16, qr, qm,
+                              kr, v, km, g, beta, z, mix_lse, mem_scale, sink_k, sink_v, n_sinks, ring_k, ring_v,
+                              ring_km, ring_g, ring_beta, ring_pos, state, o, nullptr, dws, dn)))
+            return st;
+        if ((st = bf::student_front(f, false, s))) return st;
+        raw.gp_ns = f.gp_ns;
+        return bf::decode_dispatch(raw, s);
     }
+    if ((st = bf::gate_project_dispatch(gp, s))) return st;
     {
         bf::MemProjArgs a{};
         a.x = q; a.n_tok = B; a.nh = H; a.D = D; a.x_st = (long)H * D; a.x_sh = D;
@@ -392,8 +466,6 @@ int bf_student_decode(int B, int H, int G, int D, int W, int sinks, int64_t pos,
         a.pos_arr = pos_arr; a.A_log = A_log; a.dt_bias = dt_bias; a.decay_mask = decay_mask; a.g = g; a.beta = beta;
         if ((st = bf::mem_gates_dispatch(a, s))) return st;
     }
-    void* dws = ws + l.dec;
-    const size_t dn = workspace_bytes - l.dec;
     if (pos_arr)
         return bf_decode_fwd_batch(B, G, H / G, D, W, sinks, pos_arr, memory, BF_DTYPE_BF16, BF_DTYPE_BF16, qr, qm,
                                    kr, v, km, g, beta, z, mix_lse, mem_scale, sink_k, sink_v, ring_k, ring_v, ring_km,
@@ -562,7 +634,7 @@ static bool kv_aligned(const void* p, int64_t s1, int64_t s2) {
 // inner call runs on at most B T tokens with that same segment length, and every buffer of the GDN layout grows
 // monotonically with the token count at a fixed segment length, so the reservation always suffices.
 struct LayerWs {
-    size_t wq, wk, wv, wg, wb, om, o_mem, s_new, part, gdn, total;
+    size_t wq, wk, wv, wg, wb, om, o_mem, few, s_new, part, gdn, total;
     int seg_chunks;
 };
 static LayerWs layer_ws(int B, int G, int R, int D, int T, int in_dtype) {
@@ -577,6 +649,7 @@ static LayerWs layer_ws(int B, int G, int R, int D, int T, int in_dtype) {
     put(w.wb, BT * G * 4);
     put(w.om, BT * H * D * esz);
     put(w.o_mem, BT * H * D * esz);
+    put(w.few, T <= bf::FEW_MAX_T ? BT * H * D * 4 : 0);      // o_mem of the few-token memory branch, fp32
     put(w.s_new, (size_t)B * G * D * D * 4);
     // the item map's slot count does not depend on the window or the position
     put(w.part, in_dtype == BF_DTYPE_BF16 ? bf::window_split_bytes(bf::window_map(B, G, R, T, 1, 0), D) : 0);
@@ -630,7 +703,15 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
     a.s_new = reinterpret_cast<float*>(ws + L.s_new); a.state = state;
     int rc;
     const void* o_mem = nullptr;
-    if (use_mem) {
+    int o_mem_dtype = in_dtype;
+    // a few tokens over a cache: token by token on the state, in place (R <= 8 query heads per KV head)
+    const bool few = use_mem && T <= bf::FEW_MAX_T && R <= 8;
+    if (few) {
+        a.o_mem = ws + L.few;
+        if ((rc = bf::few_mem_dispatch(a, state_valid ? state : nullptr, st))) return rc;
+        o_mem = a.o_mem;
+        o_mem_dtype = BF_DTYPE_F32;
+    } else if (use_mem) {
         // from an empty cache the queries before W never mix the memory in: the stream is the chunk shifted by W
         const bool fresh = start == 0 && !state_valid;
         a.qoff = fresh ? W : 0;
@@ -660,11 +741,11 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
     }
     rc = window_fwd(B, G, R, D, T, W, sinks, start, in_dtype, qr, q_sb, q_sh, q_st, kr, k_sb, k_sh, k_st, v, v_sb,
                     v_sh, v_st, ring_k, ring_v, ring_pos, sink_k, sink_v, n_sinks, use_mem ? 1 : 0, o_mem,
-                    in_dtype, use_mem ? z : nullptr, use_mem ? mix_lse : nullptr, use_mem ? mem_scale : nullptr, o,
+                    o_mem_dtype, use_mem ? z : nullptr, use_mem ? mix_lse : nullptr, use_mem ? mem_scale : nullptr, o,
                     BF_DTYPE_F32, lse, reinterpret_cast<float*>(ws + L.part), stream);
     if (rc) return rc;
     if ((rc = bf::layer_launch(a, 2, st))) return rc;         // ring write-back after every read of the ring
-    if (use_mem && (rc = bf::layer_launch(a, 3, st))) return rc;
+    if (use_mem && !few && (rc = bf::layer_launch(a, 3, st))) return rc;
     return BF_STATUS_OK;
 }
 

@@ -88,16 +88,18 @@ __device__ __forceinline__ void reduce_colgroups(float (&v)[NV], float* red) {
 // State slab pass for one (b, g): columns [j0, j0 + SCOL). Thread tid owns columns j0 + 4 (tid % SCG) .. +3 of rows
 // tid / SCG + (256 / SCG) i. Applies S <- e^{wg} S; delta = wb (wv - S^T wk); S <- S + wk delta^T (skipped when !write), then
 // writes o[r][j] = sum_d qm_r[d] S[d][j] for the R query heads. S is updated in place (s_in == s_out allowed).
-template <int D, int RMAX>
+// `loaded` runs after the slab's loads have been issued and returns the factors of the heads' qm rows (null: 1).
+template <int D, int RMAX, class F>
 __device__ __forceinline__ void state_slab(const float* s_in, float* s_out, const float* wk, const float* wv,
                                            float wg, float wb, bool write, const float* qm, int R, long q_stride,
-                                           float* om, long o_stride, int j0, float* red) {
+                                           float* om, long o_stride, int j0, float* red, F&& loaded) {
     constexpr int RSTEP = 256 / SCG, RPT = D / RSTEP;   // row step, rows per thread
     const int tid = threadIdx.x, cg = tid & (SCG - 1), r0 = tid / SCG;
     const int jc = j0 + 4 * cg;
     float4 s[RPT];
 #pragma unroll
     for (int i = 0; i < RPT; ++i) s[i] = nt_ldf4(s_in + (long)(r0 + RSTEP * i) * D + jc);    // streamed: read once
+    const float* qf = loaded();
     if (write) {
         const float a = __expf(wg);
         float rc[4] = {0.f, 0.f, 0.f, 0.f};
@@ -127,9 +129,10 @@ __device__ __forceinline__ void state_slab(const float* s_in, float* s_out, cons
     for (int r = 0; r < RMAX; ++r) {
         float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
         if (r < R) {
+            const float f = qf ? qf[r] : 1.f;
 #pragma unroll
             for (int i = 0; i < RPT; ++i) {
-                const float qv = qm[r * q_stride + r0 + RSTEP * i];
+                const float qv = qm[r * q_stride + r0 + RSTEP * i] * f;
                 a0 += qv * s[i].x; a1 += qv * s[i].y; a2 += qv * s[i].z; a3 += qv * s[i].w;
             }
         }
@@ -488,7 +491,7 @@ __global__ __launch_bounds__(NT_DEC) void decode_main_kernel(DecodeArgs a) {
         ev[D + d] = kk;
         RKs[d] = NK[d];
         RVs[d] = NV[d];
-        KM[d] = a.km[bg * D + d];
+        if (!a.gp_part) KM[d] = a.km[bg * D + d];       // else the tail writes it, normalised
     }
     if (a.pos_arr && pos < a.n_sinks) {                 // the new token becomes sink row pos (no split reads it)
         T* sk = reinterpret_cast<T*>(a.sink_k) + (bg * a.n_sinks + pos) * D;
@@ -503,8 +506,10 @@ __global__ __launch_bounds__(NT_DEC) void decode_main_kernel(DecodeArgs a) {
         ev[2 * D] = a.ring_g[rg];
         ev[2 * D + 1] = a.ring_beta[rg];
         ev[2 * D + 2] = valid ? 1.f : 0.f;
-        a.ring_g[rg] = a.g_new[bg];
-        a.ring_beta[rg] = a.beta_new[bg];
+        if (!a.gp_part) {
+            a.ring_g[rg] = a.g_new[bg];
+            a.ring_beta[rg] = a.beta_new[bg];
+        }
     }
 }
 
@@ -512,13 +517,16 @@ __global__ __launch_bounds__(NT_DEC) void decode_main_kernel(DecodeArgs a) {
 //  - memory on: the write of the ring row that left the window (from ws_ev), then the memory read of the R query
 //    heads for the slab's columns (into ws_om);
 //  - the merge of the window splits for the slab's dims and every query head, the gamma mix, o and lse;
-//  - the ring_pos entry of the new token (its values were written by split 0 of the window kernel).
+//  - the ring_pos entry of the new token (its values were written by split 0 of the window kernel);
+//  - with gp_part, the rest of the memory inputs (the norms of qm and km, the gates and the gamma logits), which is a
+//    few small sums per workgroup under the state's loads instead of two launches of their own.
 template <class KV, int D, int RM>
 __global__ __launch_bounds__(NT_DEC) void decode_tail_kernel(DecodeArgs a) {
     constexpr int MAXS = 64;                            // window splits held in LDS (W <= 65536)
     __shared__ float red[4 * SCG * RM * 4];
     __shared__ float fs[RM][MAXS];
     __shared__ float st2[RM][2];
+    __shared__ float zs[RM], qinv[RM + 1];              // gamma logits; norm factors of qm's rows and (last) km's
     const int x = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
     const int G = a.G, R = a.R, H = G * R, W = a.W, NS = a.nsplit;
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -527,12 +535,39 @@ __global__ __launch_bounds__(NT_DEC) void decode_tail_kernel(DecodeArgs a) {
     const long pos = a.pos_arr ? a.pos_arr[b] : a.pos;
     const bool mem_on = a.mem_on && (!a.pos_arr || pos >= W);
     float* om = a.ws_om + ((long)b * H + g * R) * D;
+    const float* QM = a.qm + ((long)b * H + g * R) * D;
+    auto inputs = [&]() -> const float* {
+        if (!a.gp_part) return nullptr;
+        const long stride = (long)a.B * (2 * G + H);
+        const float* gp = a.gp_part + (long)b * (2 * G + H);
+        if (wv == 0 && tid < 4 * (R + 1)) {             // 4 lanes per row: the R rows of qm, then km's
+            const int r = tid >> 2;
+            const bool isq = r < R;
+            const float ss = row_square_sum<D>(isq ? QM + (long)r * D : a.km + bg * D, tid & 3);
+            if ((tid & 3) == 0) qinv[isq ? r : RM] = (isq ? a.q_scale : 1.f) / fmaxf(sqrtf(ss), 1e-12f);
+        }
+        if (wv == 1 && lane < R) {
+            const int h = g * R + lane;
+            zs[lane] = split_sum(gp + 2 * G + h, stride, a.gp_ns) + (a.b_mix ? a.b_mix[h] : 0.f);
+        }
+        if (x == 0 && wv == 2 && lane == 0) {
+            const float la = split_sum(gp + g, stride, a.gp_ns) + (a.b_ab ? a.b_ab[g] : 0.f);
+            const float lb = split_sum(gp + G + g, stride, a.gp_ns) + (a.b_ab ? a.b_ab[G + g] : 0.f);
+            const long rg = ((long)b * W + pos % W) * G + g;
+            a.ring_g[rg] = mem_gate_g(la, a.dt_bias[g], a.A_log[g], a.decay_mask[g]);
+            a.ring_beta[rg] = pos >= a.sinks ? mem_gate_beta(lb) : 0.f;
+        }
+        lds_barrier();
+        if (tid < SCOL) a.ring_km[(((long)b * W + pos % W) * G + g) * D + j0 + tid] = a.km[bg * D + j0 + tid] * qinv[RM];
+        return qinv;
+    };
+    if (!mem_on) inputs();
     if (mem_on) {
         const float* ev = a.ws_ev + bg * (2 * D + 4);
         const bool valid = ev[2 * D + 2] != 0.f;
         const float wg = valid ? ev[2 * D] : 0.f, wb = valid ? ev[2 * D + 1] : 0.f;
         float* S = a.state + bg * D * D;
-        state_slab<D, RM>(S, S, ev + D, ev, wg, wb, valid, a.qm + ((long)b * H + g * R) * D, R, D, om, D, j0, red);
+        state_slab<D, RM>(S, S, ev + D, ev, wg, wb, valid, QM, R, D, om, D, j0, red, inputs);
     }
     // split statistics per head (wave w takes heads w, w + 4): M = max m_s, f_s = e^{m_s - M}, L = sum f_s l_s
     const float* part = a.ws_part + bg * NS * R * (D + 2);
@@ -555,18 +590,150 @@ __global__ __launch_bounds__(NT_DEC) void decode_tail_kernel(DecodeArgs a) {
         const int r = i / SCOL, d = j0 + i % SCOL, h = g * R + r;
         const float M = st2[r][0], L = st2[r][1];
         float ow = 0.f;
-        for (int s_ = 0; s_ < NS; ++s_) ow += fs[r][s_] * part[(s_ * R + r) * (D + 2) + 2 + d];
+        for (int s0 = 0; s0 < NS; s0 += 8) {            // 8 rows' loads together
+            float p[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) p[j] = part[(min(s0 + j, NS - 1) * R + r) * (D + 2) + 2 + d];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ow = s0 + j < NS ? fmaf(fs[r][s0 + j], p[j], ow) : ow;
+        }
         ow /= L;
         const float lse = M + logf(L);
         float o = ow;
         if (mem_on) {
-            const float gam = 1.f / (1.f + __expf(-(a.z[(long)b * H + h] + a.mix_lse[h] * (lse - lnW))));
+            const float z = a.gp_part ? zs[r] : a.z[(long)b * H + h];
+            const float gam = 1.f / (1.f + __expf(-(z + a.mix_lse[h] * (lse - lnW))));
             o = ow + gam * (a.mem_scale[h] * om[r * D + d] - ow);
         }
         a.o[((long)b * H + h) * D + d] = o;
         if (x == 0 && i % SCOL == 0 && a.lse) a.lse[(long)b * H + h] = lse;
     }
     if (x == 0 && g == 0 && tid == 0 && (a.pos_arr || b == 0)) a.ring_pos[(a.pos_arr ? (long)b * W : 0L) + pos % W] = pos;
+}
+
+// The memory branch of a chunk of a few tokens over a cache (an MTP verification; T <= FEW_MAX_T): workgroup (x, g, b)
+// holds 64 columns of the state in registers and takes the tokens in turn: the row of position p - W leaves the window
+// (a ring row if ring_pos holds that position, or a row of this chunk) and is written into the state, then the R query
+// heads read it. Each token costs two sums over the slab's rows (~2 us), where the chunked scan pays for 64 tokens,
+// five launches and bf16 copies of the stream: at T = 2, H = 24, G = 4, D = 256 this pass replaced stream, prep, scan
+// and state copy. Above 16 tokens the scan is the faster one.
+template <int D, int RM>
+__global__ __launch_bounds__(NT_DEC) void few_mem_kernel(LayerArgs a, const float* s_in) {
+    constexpr int RSTEP = 256 / SCG, RPT = D / RSTEP;
+    __shared__ float red[4 * SCG * RM * 4];
+    __shared__ float ks[FEW_MAX_T][D];                  // the leaving keys, their values (this slab's columns), gates
+    __shared__ float vs[FEW_MAX_T][SCOL];
+    __shared__ float gs[FEW_MAX_T], bs[FEW_MAX_T];
+    __shared__ int on[FEW_MAX_T];
+    __shared__ float qs[2][RM * D];
+    const int x = blockIdx.x, g = blockIdx.y, b = blockIdx.z;
+    const int G = a.G, R = a.R, H = G * R, W = a.W, T = a.T;
+    const int tid = threadIdx.x, cg = tid & (SCG - 1), r0 = tid / SCG, j0 = x * SCOL, jc = j0 + 4 * cg;
+    const long bg = (long)b * G + g;
+    auto ldx = [](const void* p, long i, int dt) {
+        return dt == DT_BF16 ? bf2f(reinterpret_cast<const uint16_t*>(p)[i]) : reinterpret_cast<const float*>(p)[i];
+    };
+    float4 s[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i)
+        s[i] = s_in ? nt_ldf4(s_in + (bg * D + r0 + RSTEP * i) * D + jc) : make_float4(0.f, 0.f, 0.f, 0.f);
+    // the rows leaving the window
+    for (int i = 0; i < T; ++i) {
+        const long p = a.start + i - W;
+        const bool chunk = p >= a.start;
+        const long t = p - a.start, slot = p >= 0 ? p % W : 0;
+        const bool ok = chunk || (p >= 0 && a.ring_pos[slot] == p);
+        const long rk = ((long)b * W + slot) * G + g, ck = ((long)b * T + t) * G + g;
+        for (int d = tid; d < D; d += NT_DEC)
+            ks[i][d] = !ok ? 0.f : (chunk ? ldx(a.km, ck * D + d, a.km_dtype) : a.ring_km[rk * D + d]);
+        if (tid < SCOL)
+            vs[i][tid] = !ok ? 0.f : (chunk ? ldx(a.v, b * a.v_sb + g * a.v_sh + t * a.v_st + j0 + tid, a.in_dtype)
+                                            : ldx(a.ring_v, (bg * W + slot) * D + j0 + tid, a.in_dtype));
+        if (tid == NT_DEC - 1) {
+            on[i] = ok;
+            gs[i] = !ok ? 0.f : (chunk ? a.g[ck] : a.ring_g[rk]);
+            bs[i] = !ok ? 0.f : (chunk ? a.beta[ck] : a.ring_beta[rk]);
+        }
+    }
+    // token i's queries, loaded a token ahead
+    constexpr int QPT = RM * D / NT_DEC;
+    auto ldq = [&](int i, float (&q)[QPT]) {
+        const long base = (((long)b * T + min(i, T - 1)) * H + g * R) * D;
+#pragma unroll
+        for (int j = 0; j < QPT; ++j) q[j] = ldx(a.qm, base + min(tid + NT_DEC * j, R * D - 1), a.qm_dtype);
+    };
+    float qn[QPT];
+    ldq(0, qn);
+    float* om = reinterpret_cast<float*>(a.o_mem) + ((long)b * T * H + g * R) * D;
+    for (int i = 0; i < T; ++i) {
+        float* q = qs[i & 1];
+#pragma unroll
+        for (int j = 0; j < QPT; ++j) q[tid + NT_DEC * j] = qn[j];
+        ldq(i + 1, qn);
+        __syncthreads();                                // q, and before token 0 the leaving rows
+        if (on[i]) {                                    // uniform
+            const float al = __expf(gs[i]), be = bs[i];
+            float rc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int n = 0; n < RPT; ++n) {
+                const float k = ks[i][r0 + RSTEP * n];
+                rc[0] += k * s[n].x; rc[1] += k * s[n].y; rc[2] += k * s[n].z; rc[3] += k * s[n].w;
+            }
+            reduce_colgroups<4>(rc, red);
+            float dl[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) dl[e] = be * (vs[i][4 * cg + e] - al * rc[e]);
+#pragma unroll
+            for (int n = 0; n < RPT; ++n) {
+                const float k = ks[i][r0 + RSTEP * n];
+                s[n].x = al * s[n].x + k * dl[0];
+                s[n].y = al * s[n].y + k * dl[1];
+                s[n].z = al * s[n].z + k * dl[2];
+                s[n].w = al * s[n].w + k * dl[3];
+            }
+        }
+        if (a.start + i < W) continue;                  // uniform: no memory read before position W
+        float acc[RM * 4];
+#pragma unroll
+        for (int r = 0; r < RM; ++r) {
+            float a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+            if (r < R) {
+#pragma unroll
+                for (int n = 0; n < RPT; ++n) {
+                    const float qv = q[r * D + r0 + RSTEP * n];
+                    a0 += qv * s[n].x; a1 += qv * s[n].y; a2 += qv * s[n].z; a3 += qv * s[n].w;
+                }
+            }
+            acc[4 * r] = a0; acc[4 * r + 1] = a1; acc[4 * r + 2] = a2; acc[4 * r + 3] = a3;
+        }
+        reduce_colgroups<RM * 4>(acc, red);
+        if (r0 == 0) {
+#pragma unroll
+            for (int r = 0; r < RM; ++r)
+                if (r < R) *reinterpret_cast<float4*>(om + ((long)i * H + r) * D + jc) =
+                    make_float4(acc[4 * r], acc[4 * r + 1], acc[4 * r + 2], acc[4 * r + 3]);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) nt_stf4(a.state + (bg * D + r0 + RSTEP * i) * D + jc, s[i]);
+}
+
+template <int D>
+static int launch_few(const LayerArgs& a, const float* s_in, hipStream_t stream) {
+    const dim3 grid(D / SCOL, a.G, a.B), block(NT_DEC);
+    if (a.R <= 4) hipLaunchKernelGGL((few_mem_kernel<D, 4>), grid, block, 0, stream, a, s_in);
+    else hipLaunchKernelGGL((few_mem_kernel<D, 8>), grid, block, 0, stream, a, s_in);
+    return (int)hipGetLastError();
+}
+
+int few_mem_dispatch(const LayerArgs& a, const float* s_in, hipStream_t stream) {
+    if (a.T > FEW_MAX_T || a.R > RMAX) return BF_ERR_UNSUPPORTED;
+    switch (a.D) {
+        case 64: return launch_few<64>(a, s_in, stream);
+        case 128: return launch_few<128>(a, s_in, stream);
+        case 256: return launch_few<256>(a, s_in, stream);
+        default: return BF_ERR_UNSUPPORTED;
+    }
 }
 
 // ----------------------------------------------------------------------------------------------- single-token GDN
@@ -577,7 +744,8 @@ __global__ __launch_bounds__(NT_DEC) void gdn_step_kernel(StepArgs a) {
     const int G = a.G, R = a.R, H = G * R;
     const long bg = (long)b * G + g;
     state_slab<D, RMAX>(a.s_in + bg * D * D, a.s_out + bg * D * D, a.k + bg * D, a.v + bg * D, a.g[bg], a.beta[bg], true,
-                  a.q + ((long)b * H + g * R) * D, R, D, a.o + ((long)b * H + g * R) * D, D, x * SCOL, red);
+                  a.q + ((long)b * H + g * R) * D, R, D, a.o + ((long)b * H + g * R) * D, D, x * SCOL, red,
+                  [] { return (const float*)nullptr; });
 }
 
 // ------------------------------------------------------------------------------------------------ host launchers

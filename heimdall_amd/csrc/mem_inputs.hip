@@ -188,11 +188,9 @@ __global__ __launch_bounds__(256) void mem_gates_kernel(MemGatesArgs a) {
     const long t = e / a.G;
     const int j = (int)(e % a.G);
     const float* row = a.ab + t * a.ab_st;
-    const float x = row[j] + a.dt_bias[j];
-    const float sp = x > 20.f ? x : log1pf(expf(x));            // softplus, torch's default threshold
-    a.g[e] = -expf(a.A_log[j]) * sp * a.decay_mask[j];
+    a.g[e] = mem_gate_g(row[j], a.dt_bias[j], a.A_log[j], a.decay_mask[j]);
     const long pos = (a.pos_arr ? a.pos_arr[t / a.T] : a.start) + t % a.T;
-    a.beta[e] = pos >= a.sinks ? 1.f / (1.f + expf(-row[a.G + j])) : 0.f;
+    a.beta[e] = pos >= a.sinks ? mem_gate_beta(row[a.G + j]) : 0.f;
 }
 
 int mem_gates_dispatch(const MemGatesArgs& a, hipStream_t stream) {
@@ -350,10 +348,8 @@ __global__ __launch_bounds__(64 * GP_WAVES) void gate_project_kernel(GateProjArg
 // while the current one multiplies (the lane / MFMA mapping of gate_project_kernel), and writes its partial sums to
 // part[s][token][n0 + n1]; gate_project_reduce_kernel adds the splits in a fixed order (s = 0, 1, ..) and the bias.
 template <int NT>
-__global__ __launch_bounds__(64) void gate_project_split_kernel(GateProjArgs a, int steps_per) {
+__device__ __forceinline__ void gate_split_wave(const GateProjArgs& a, int steps_per, int sp, long tok0) {
     const int lane = lane_id(), l16 = lane & 15, lg = lane >> 4;
-    const int sp = blockIdx.x;
-    const long tok0 = (long)blockIdx.y * 16;
     const int nout = a.n0 + a.n1;
     const long tok = tok0 + l16;
     const bool tok_ok = tok < a.n_tok;
@@ -434,14 +430,18 @@ __global__ __launch_bounds__(64) void gate_project_split_kernel(GateProjArgs a, 
     }
 }
 
+template <int NT>
+__global__ __launch_bounds__(64) void gate_project_split_kernel(GateProjArgs a, int steps_per) {
+    gate_split_wave<NT>(a, steps_per, blockIdx.x, (long)blockIdx.y * 16);
+}
+
 __global__ __launch_bounds__(256) void gate_project_reduce_kernel(GateProjArgs a, int nsplit) {
     const int nout = a.n0 + a.n1;
     const long e = (long)blockIdx.x * 256 + threadIdx.x;
     if (e >= a.n_tok * nout) return;
     const long t = e / nout;
     const int c = (int)(e % nout);
-    float s = 0.f;
-    for (int sp = 0; sp < nsplit; ++sp) s += a.part[(long)sp * a.n_tok * nout + e];
+    const float s = split_sum(a.part + e, a.n_tok * nout, nsplit);
     if (c < a.n0) a.out0[t * a.n0 + c] = s + (a.b0 ? a.b0[c] : 0.f);
     else a.out1[t * a.n1 + (c - a.n0)] = s + (a.b1 ? a.b1[c - a.n0] : 0.f);
 }
@@ -450,8 +450,8 @@ int gate_project_dispatch(const GateProjArgs& a, hipStream_t stream) {
     const int nsplit = gate_project_nsplit(a.n_tok, a.d);
     if (nsplit > 0) {
         if (!a.part) return BF_STATUS_WORKSPACE;
-        const int steps = (a.d + 127) / 128, per = (steps + nsplit - 1) / nsplit;
-        const int ns = (steps + per - 1) / per;               // splits that hold at least one step
+        int per = 0;
+        const int ns = gate_project_splits(a.n_tok, a.d, &per);
         const dim3 grid((unsigned)ns, (unsigned)((a.n_tok + 15) / 16));
         if (a.n0 + a.n1 <= 32) hipLaunchKernelGGL(gate_project_split_kernel<2>, grid, dim3(64), 0, stream, a, per);
         else hipLaunchKernelGGL(gate_project_split_kernel<GP_MAX_OUT / 16>, grid, dim3(64), 0, stream, a, per);
@@ -471,6 +471,127 @@ int gate_project_dispatch(const GateProjArgs& a, hipStream_t stream) {
     if (a.n0 + a.n1 <= 32) hipLaunchKernelGGL((gate_project_kernel<2, 2>), grid, block, 0, stream, a, ws);
     else hipLaunchKernelGGL((gate_project_kernel<GP_MAX_OUT / 16, 1>), grid, block, 0, stream, a, ws);
     return (int)hipGetLastError();
+}
+
+// The memory inputs of a few tokens (a decode step, an MTP verification, a short chunk) in two launches instead of the
+// five of gate_project_split + reduce, two mem_project and mem_gates. One wave per workgroup:
+//  - projection waves, one per (head of q or k, 16 output columns, 64 tokens): the column block of F_h straight from
+//    memory into MFMA A fragments (each instruction reads 64-byte pieces of 4 rows of F_h; no LDS, and the 256 KB of
+//    a head spread over 16 CUs instead of being staged by one), y = x F_h unnormalised, fp32. The products are
+//    mem_project_kernel's, in its order.
+//  - gate waves: gate_split_wave's partial sums.
+// Both read parameters that no workgroup shares with another, so the launch is bound by one memory round trip. The norm
+// of a head's row needs all its columns: student_finish_kernel (chunks) or decode_tail_kernel (decode) applies it.
+constexpr int FR_TILES = 4;                                    // 16-token tiles per projection wave
+template <int D, int NT>
+__global__ __launch_bounds__(64) void student_front_kernel(FrontArgs a) {
+    constexpr int NKD = D / 32, NCT = D / 16;
+    const int heads = a.H + a.G;
+    const long ngrp = (a.gp.n_tok + 16 * FR_TILES - 1) / (16 * FR_TILES), nproj = ngrp * heads * NCT;
+    const long bid = blockIdx.x;
+    if (bid >= nproj) {
+        gate_split_wave<NT>(a.gp, a.gp_per, (int)((bid - nproj) % a.gp_ns), (bid - nproj) / a.gp_ns * 16);
+        return;
+    }
+    const int lane = lane_id(), l16 = lane & 15, lg = lane >> 4;
+    const int ct = (int)(bid % NCT), hh = (int)((bid / NCT) % heads);
+    const long tile0 = bid / NCT / heads * FR_TILES, ntile = min((a.gp.n_tok + 15) / 16, tile0 + FR_TILES);
+    const bool isq = hh < a.H;
+    const int h = isq ? hh : hh - a.H, nh = isq ? a.H : a.G;
+    const float* F = (isq ? a.fq : a.fk) + (long)h * D * D + (long)(8 * lg) * D + 16 * ct + l16;
+    const uint16_t* X = reinterpret_cast<const uint16_t*>(isq ? a.q : a.k) + h * (isq ? a.q_sh : a.k_sh);
+    const long x_st = isq ? a.q_st : a.k_st;
+    float* Y = (isq ? a.yq : a.yk) + (long)h * D + 16 * ct + 4 * lg;
+    float f[NKD][8];
+#pragma unroll
+    for (int ks = 0; ks < NKD; ++ks)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) f[ks][e] = F[(long)(32 * ks + e) * D];
+    uint4 af[NKD];
+#pragma unroll
+    for (int ks = 0; ks < NKD; ++ks)
+        af[ks] = make_uint4(pack_bf16x2(f[ks][0], f[ks][1]), pack_bf16x2(f[ks][2], f[ks][3]),
+                            pack_bf16x2(f[ks][4], f[ks][5]), pack_bf16x2(f[ks][6], f[ks][7]));
+    for (long t = tile0; t < ntile; ++t) {
+        const long n = min((long)16, a.gp.n_tok - 16 * t);
+        const rsrc_t rx = make_rsrc(X + 16 * t * x_st, (uint32_t)(((n - 1) * x_st + D) * 2));    // rows past n read 0
+        uint4 xf[NKD];
+#pragma unroll
+        for (int ks = 0; ks < NKD; ++ks)
+            xf[ks] = buf_ld16(rx, l16 < n ? (uint32_t)((l16 * x_st + 32 * ks + 8 * lg) * 2) : 0xFFFFFFF0u);
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < NKD; ++ks) mma<BF16>(acc, af[ks], xf[ks]);
+        if (l16 < n)
+            *reinterpret_cast<float4*>(Y + (16 * t + l16) * (long)nh * D) = make_float4(acc[0], acc[1], acc[2], acc[3]);
+    }
+}
+
+// The second launch for a chunk: rows of yq / yk normalised into qm / km (4 lanes per row), and the gates and the
+// gamma logit from the gate partials (one thread per (token, KV head) and per (token, head)).
+template <int D>
+__global__ __launch_bounds__(256) void student_finish_kernel(FrontArgs a) {
+    const long n_tok = a.gp.n_tok, rows = n_tok * (a.H + a.G), e = (long)blockIdx.x * 256 + threadIdx.x;
+    const long row_thr = (4 * rows + 255) / 256 * 256;         // whole workgroups take rows
+    if (e < row_thr) {
+        const long r = min(e / 4, rows - 1);
+        const int part = (int)(e & 3);
+        const bool isq = r < n_tok * a.H;
+        const long i = isq ? r : r - n_tok * a.H;
+        const float* y = (isq ? a.yq : a.yk) + i * D;
+        const float inv = (isq ? a.q_scale : 1.f) / fmaxf(sqrtf(row_square_sum<D>(y, part)), 1e-12f);
+        if (e / 4 >= rows) return;
+        void* out = isq ? a.qm : a.km;
+#pragma unroll
+        for (int j = 0; j < D / 16; ++j) {
+            const float4 v = *reinterpret_cast<const float4*>(y + 16 * j + 4 * part);
+            const long at = i * D + 16 * j + 4 * part;
+            if (a.out_dtype == DT_BF16)
+                store4<BF16>(reinterpret_cast<uint16_t*>(out) + at, v.x * inv, v.y * inv, v.z * inv, v.w * inv);
+            else
+                store4<F32>(reinterpret_cast<float*>(out) + at, v.x * inv, v.y * inv, v.z * inv, v.w * inv);
+        }
+        return;
+    }
+    const long i = e - row_thr;
+    const int nout = 2 * a.G + a.H, per = a.G + a.H;
+    if (i >= n_tok * per) return;
+    const long t = i / per, stride = n_tok * nout;
+    const int c = (int)(i % per);
+    const float* p = a.gp.part + t * nout;
+    if (c < a.G) {
+        const float la = split_sum(p + c, stride, a.gp_ns) + (a.gp.b0 ? a.gp.b0[c] : 0.f);
+        const float lb = split_sum(p + a.G + c, stride, a.gp_ns) + (a.gp.b0 ? a.gp.b0[a.G + c] : 0.f);
+        a.g[t * a.G + c] = mem_gate_g(la, a.dt_bias[c], a.A_log[c], a.decay_mask[c]);
+        a.beta[t * a.G + c] = a.start + t % a.T >= a.sinks ? mem_gate_beta(lb) : 0.f;
+    } else {
+        const int h = c - a.G;
+        a.z[t * a.H + h] = split_sum(p + 2 * a.G + h, stride, a.gp_ns) + (a.gp.b1 ? a.gp.b1[h] : 0.f);
+    }
+}
+
+template <int D>
+static int launch_front(FrontArgs& a, bool finish, hipStream_t stream) {
+    a.gp_ns = gate_project_splits(a.gp.n_tok, a.gp.d, &a.gp_per);
+    const long tiles = (a.gp.n_tok + 15) / 16, ngrp = (tiles + FR_TILES - 1) / FR_TILES;
+    const dim3 grid((unsigned)(ngrp * (a.H + a.G) * (D / 16) + a.gp_ns * tiles));
+    if (a.gp.n0 + a.gp.n1 <= 32) hipLaunchKernelGGL((student_front_kernel<D, 2>), grid, dim3(64), 0, stream, a);
+    else hipLaunchKernelGGL((student_front_kernel<D, GP_MAX_OUT / 16>), grid, dim3(64), 0, stream, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !finish) return (int)e;
+    const long wgs = (4 * a.gp.n_tok * (a.H + a.G) + 255) / 256 + (a.gp.n_tok * (a.H + a.G) + 255) / 256;
+    hipLaunchKernelGGL(student_finish_kernel<D>, dim3((unsigned)wgs), dim3(256), 0, stream, a);
+    return (int)hipGetLastError();
+}
+
+int student_front(FrontArgs& a, bool finish, hipStream_t stream) {
+    if (a.gp.n_tok > FRONT_MAX_TOK) return BF_ERR_UNSUPPORTED;
+    switch (a.D) {
+        case 64: return launch_front<64>(a, finish, stream);
+        case 128: return launch_front<128>(a, finish, stream);
+        case 256: return launch_front<256>(a, finish, stream);
+        default: return BF_ERR_UNSUPPORTED;
+    }
 }
 
 }  // namespace bf

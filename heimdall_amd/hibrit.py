@@ -133,6 +133,38 @@ def _mem_inputs_bf16(self, ab, q, k, start: int, out_dtype=torch.bfloat16):
     return qm, km, g, beta
 
 
+def _few_inputs(self, x, q, k, start: int, out_dtype):
+    """The memory inputs and the gamma logit of a short bf16 chunk in one bf_student_inputs call: (qm, km in out_dtype, g,
+    beta, z), the values of ``_gate_logits`` and ``_mem_inputs_bf16``. None where the call does not apply (too many
+    tokens, more than 64 gate columns, rows it cannot address)."""
+    G, H, D = self.c.hkv, self.c.h, self.c.dh
+    b, t, d = x.shape
+    lib = _lib.load()
+    if (b * t > lib.bf_student_inputs_max_tokens() or x.dtype != torch.bfloat16 or d % 8 or 2 * G + H > 64
+            or D not in (64, 128, 256) or x.stride(-1) != 1 or x.stride(1) % 8 or x.data_ptr() % 16
+            or (b > 1 and x.stride(0) != t * x.stride(1)) or (t > 1 and x.stride(1) < d)):
+        return None
+    dense = lambda z_: z_ if (z_.stride(-1) == 1 and z_.stride(1) <= 1 << 26 and
+                              (b == 1 or z_.stride(0) == t * z_.stride(1))) else z_.contiguous()
+    q, k = dense(q), dense(k)
+    dev = x.device
+    qm, km = (torch.empty(b, t, n, D, dtype=out_dtype, device=dev) for n in (H, G))
+    g, beta = (torch.empty(b, t, G, dtype=torch.float32, device=dev) for _ in range(2))
+    z = torch.empty(b, t, H, dtype=torch.float32, device=dev)
+    prm = tuple(_f32(p) for p in (self.fq, self.fk, self.ab.weight, self.ab.bias, self.mix.weight, self.mix.bias,
+                                  self.A_log, self.dt_bias, self.decay_mask))
+    nb = _lib.ctypes.c_size_t(0)
+    check(lib.bf_student_inputs_workspace_size(b * t, H, G, D, d, _lib.ctypes.byref(nb)),
+          "bf_student_inputs_workspace_size")
+    ws = workspace(nb.value, dev)
+    check(lib.bf_student_inputs(x.data_ptr(), max(x.stride(1), d), q.data_ptr(), q.stride(1), q.stride(2), k.data_ptr(),
+                                k.stride(1), k.stride(2), b * t, t, H, G, D, d, *(p.data_ptr() for p in prm), start,
+                                self.sinks, qm.data_ptr(), km.data_ptr(), dtype_code(out_dtype), g.data_ptr(),
+                                beta.data_ptr(), z.data_ptr(), ws.data_ptr(), nb.value, stream_ptr(dev)),
+          "bf_student_inputs")
+    return qm, km, g, beta, z
+
+
 def _new_ring(b, G, w, D, kdt, vdt, dev, overwritten: bool = False):
     """An empty ring (no valid slot). ``overwritten``: the caller's next write fills every slot before anything reads
     the ring (a prefill of at least W tokens from position 0), so the row tensors are left uninitialised; ring_pos
@@ -216,6 +248,7 @@ def _decode(self, x, qr, kr, v, qm, km, g, beta, start, st, sink_k, sink_v, memo
 # G = 4, D = 256, W = 2048 + 4, a t = 2 chunk costs 207 us through the chunk kernels and 261 us as two decode steps,
 # whose time is mostly host launch gaps between their six library calls.
 SMALL_CHUNK = 1
+FEW_MAX_T = 16      # chunks of up to this many tokens take bf_layer_prefill_fwd's token-by-token memory branch (fp32)
 BATCH_KEYS = ("sink_k", "sink_v", "ring_k", "ring_v", "ring_km", "ring_g", "ring_beta", "ring_pos", "S")
 
 
@@ -406,9 +439,15 @@ def student(self, x, q, k, v, qr, kr, start: int, cache: Optional[dict], memory:
         return o
     zmix = None
     if all(z.dtype == torch.bfloat16 for z in (q, k, qr, kr)):
-        # fused: the gate projections, qm / km (bf16 for a chunk's memory branch, fp32 for the decode step), gates
-        ab, zmix = _gate_logits(self, x)
-        qm, km, g, beta = _mem_inputs_bf16(self, ab, q, k, start, torch.bfloat16 if t > 1 else torch.float32)
+        # fused: the gate projections, qm / km (bf16 for a chunk's scan, fp32 for the decode step and the few-token
+        # memory branch), gates
+        odt = torch.bfloat16 if t > FEW_MAX_T else torch.float32
+        few = _few_inputs(self, x, q, k, start, odt) if t > 1 else None
+        if few is not None:
+            qm, km, g, beta, zmix = few
+        else:
+            ab, zmix = _gate_logits(self, x)
+            qm, km, g, beta = _mem_inputs_bf16(self, ab, q, k, start, torch.bfloat16 if t > 1 else torch.float32)
     else:
         qm, km, g, beta = self._mem_inputs(x, q, k, torch.arange(start, start + t, device=dev))
     if "ring_k" not in st:

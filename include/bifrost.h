@@ -153,8 +153,8 @@ int bf_decode_fwd_batch(int B, int G, int R, int D, int W, int sinks, const int6
 /*
  * One decode step of the converted layer from the layer's own inputs, for bf16 activations: _student with t == 1
  * (Heimdall/heimdall/hibrit.py:363-424) including its _mem_inputs (:327-334) and the gamma logit mix(x) (:409), in
- * one call. It runs the kernels of bf_gate_project (ab and mix), bf_mem_project (qm with scale D^-1/2 and km, fp32),
- * bf_mem_gates and then bf_decode_fwd (pos_arr null: all sequences at pos) or bf_decode_fwd_batch (pos_arr [B]
+ * one call. It computes the values of bf_gate_project (ab and mix), bf_mem_project (qm with scale D^-1/2 and km, fp32),
+ * bf_mem_gates and then runs bf_decode_fwd (pos_arr null: all sequences at pos) or bf_decode_fwd_batch (pos_arr [B]
  * int64 on the device: sequence b at pos_arr[b]) on `stream`, so results equal those entry points' chained (bit for
  * bit). The caller keeps the cache bookkeeping of those entry points: with one position, the new token appended to
  * the sinks while pos < sinks (n_sinks counts it) and a zero state before the memory is first written; with
@@ -313,6 +313,25 @@ int bf_gdn_fwd_gated(const void* q, const void* k, const void* v, const float* g
                      float scale, const float* initial_state, const void* norm_z, const float* norm_w,
                      float norm_eps, void* out, float* final_state, int segment_chunks, void* workspace,
                      size_t workspace_bytes, int phases, void* stream);
+
+/*
+ * The memory inputs of a chunk of up to bf_student_inputs_max_tokens() tokens, for bf16 activations
+ * (HybridAttention._mem_inputs, Heimdall/heimdall/hibrit.py:327-334, and the gamma logit mix(x), :409) in two launches:
+ * the values of bf_gate_project, bf_mem_project (qm with scale D^-1/2, and km) and bf_mem_gates.
+ *   x rows x_st elements apart (d_model and x_st multiples of 8, 16-byte aligned); token t, head h of q at
+ *   q + t * q_st + h * q_sh and of k at k + t * k_st + h * k_sh (elements), D contiguous, bf16; parameters as in
+ *   bf_student_decode; n_tok = sequences x T tokens, token t at position start + t mod T. qm [n_tok][H][D] and
+ *   km [n_tok][G][D] in out_dtype (16-byte aligned), g, beta [n_tok][G], z [n_tok][H] f32. 2G + H <= 64.
+ * Workspace: bf_student_inputs_workspace_size bytes, 256-byte aligned.
+ */
+int64_t bf_student_inputs_max_tokens(void);
+int bf_student_inputs_workspace_size(int64_t n_tok, int H, int G, int D, int d_model, size_t* bytes);
+int bf_student_inputs(const void* x, int64_t x_st, const void* q, int64_t q_st, int64_t q_sh, const void* k, int64_t k_st,
+                      int64_t k_sh, int64_t n_tok, int64_t T, int H, int G, int D, int d_model, const float* fq,
+                      const float* fk, const float* w_ab, const float* b_ab, const float* w_mix, const float* b_mix,
+                      const float* A_log, const float* dt_bias, const float* decay_mask, int64_t start, int sinks,
+                      void* qm, void* km, int out_dtype, float* g, float* beta, float* z, void* workspace,
+                      size_t workspace_bytes, void* stream);
 
 /*
  * One prefill chunk of the converted layer: HybridAttention._student with t > 1 (Heimdall/heimdall/hibrit.py:363-424)
