@@ -44,6 +44,8 @@ SIGNATURES = {
                           + [_c_i64, _c_int, _vp, _vp, _c_int] + [_vp] * 4 + [_c_sz, _vp]),
     "bf_gdn_conv_inputs": (_c_int, [_vp, _c_i64, _vp, _c_int, _vp, _c_int] + [_vp] * 5 + [_c_int, _c_i64]
                            + [_c_int] * 3 + [_fp, _fp] + [_vp] * 5 + [_c_int, _vp]),
+    "bf_gdn_layer_step": (_c_int, [_vp, _c_i64, _vp, _vp, _c_int, _vp, _c_int, _c_int, _vp, _vp, _vp, _c_int, _vp, _c_int,
+                                   _vp, _vp, _c_int, _fp, _fp, _fp, _vp, _vp, _vp] + [_c_int] * 4 + [_vp]),
     "bf_gated_norm": (_c_int, [_vp, _c_int, _vp, _vp, _c_i64, _c_int, _fp, _vp, _c_int, _vp]),
     "bf_gdn_fwd_gated": (_c_int, [_vp] * 6 + [_c_int, _c_i64, _c_int, _c_int, _c_int, _fp, _vp, _vp, _vp, _fp, _vp, _vp,
                                        _c_int, _vp, _c_sz, _c_int, _vp]),

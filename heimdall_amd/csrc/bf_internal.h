@@ -463,6 +463,25 @@ struct GatedNormArgs {
     float eps;
 };
 int gated_norm_dispatch(const GatedNormArgs& a, hipStream_t stream);
-   // bf16 operands
+
+struct GdnStepLayerArgs {
+    int B, HK, HV, D, K;
+    int io_dtype;             // of z, prefix, conv_out, a, b, zg, out
+    int w_dtype, al_dtype, dt_dtype, nw_dtype;
+    const void* z;            // [B] rows of (2 HK + HV) D channels, z_st elements apart
+    long z_st;
+    const void* prefix;       // [B][K - 1][C] or null (zeros)
+    void* conv_out;           // [B][K - 1][C]: the last K - 1 rows of [prefix; z]
+    const void* w;            // [C][K]
+    const void *a, *b;        // [B][HV]
+    const void *A_log, *dt_bias;   // [HV]
+    const void* zg;           // [B][HV][D]
+    const void* norm_w;       // [D]
+    float l2_eps, q_scale, eps;
+    const float* s_in;        // [B][HV][D][D]
+    float* s_out;
+    void* out;                // [B][HV][D]
+};
+int gdn_layer_step_dispatch(const GdnStepLayerArgs& a, hipStream_t stream);
 
 }  // namespace bf

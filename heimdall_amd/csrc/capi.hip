@@ -611,6 +611,30 @@ int bf_gdn_conv_inputs(const void* z, int64_t z_st, const void* prefix, int in_d
     return bf::gdn_conv_inputs_dispatch(x, static_cast<hipStream_t>(stream));
 }
 
+int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+                      int w_dtype, int K, const void* a, const void* b, const void* A_log, int A_log_dtype,
+                      const void* dt_bias, int dt_bias_dtype, const void* zg, const void* norm_w, int norm_w_dtype,
+                      float norm_eps, float l2_eps, float q_scale, const float* state_in, float* state_out, void* out,
+                      int B, int HK, int HV, int D, void* stream) {
+    if (B <= 0 || B > 65535 || HK <= 0 || HV <= 0 || HV % HK || K < 2 || K > 16) return BF_STATUS_INVALID;
+    if (!supported_dim(D)) return BF_STATUS_UNSUPPORTED;
+    for (int dt : {io_dtype, w_dtype, A_log_dtype, dt_bias_dtype, norm_w_dtype})
+        if (!supported_dtype(dt)) return BF_STATUS_UNSUPPORTED;
+    if (!z || !conv_out || !conv_w || !a || !b || !A_log || !dt_bias || !zg || !norm_w || !state_in || !state_out || !out)
+        return BF_STATUS_INVALID;
+    if (z_st < (int64_t)(2 * HK + HV) * D || conv_out == prefix) return BF_STATUS_INVALID;
+    // 16-byte vector accesses
+    for (const void* p : {zg, (const void*)state_in, (const void*)state_out, (const void*)out})
+        if ((uintptr_t)p & 15) return BF_STATUS_INVALID;
+    bf::GdnStepLayerArgs x{};
+    x.B = B; x.HK = HK; x.HV = HV; x.D = D; x.K = K; x.io_dtype = io_dtype;
+    x.w_dtype = w_dtype; x.al_dtype = A_log_dtype; x.dt_dtype = dt_bias_dtype; x.nw_dtype = norm_w_dtype;
+    x.z = z; x.z_st = z_st; x.prefix = prefix; x.conv_out = conv_out; x.w = conv_w; x.a = a; x.b = b;
+    x.A_log = A_log; x.dt_bias = dt_bias; x.zg = zg; x.norm_w = norm_w;
+    x.l2_eps = l2_eps; x.q_scale = q_scale; x.eps = norm_eps; x.s_in = state_in; x.s_out = state_out; x.out = out;
+    return bf::gdn_layer_step_dispatch(x, static_cast<hipStream_t>(stream));
+}
+
 int bf_gated_norm(const void* o, int o_dtype, const void* z, const float* w, int64_t rows, int D, float eps,
                   void* out, int io_dtype, void* stream) {
     if (rows < 0) return BF_STATUS_INVALID;

@@ -14,6 +14,8 @@
 //
 // gated_norm_kernel: out = w * RMSNorm(o) * SiLU(zg) per row of D; a bf16 layer keeps the reference's bf16 rounding
 // points (o rounded to bf16, the normalised row rounded, the weight product rounded, then the SiLU product).
+#include <type_traits>
+
 #include "bf_common.h"
 #include "bf_internal.h"
 
@@ -171,11 +173,17 @@ __global__ __launch_bounds__(256) void gdn_conv_inputs_kernel(GdnInArgs a) {
 // round trip into every token's chain). Measured on 4 packed sequences {8192, 16384, 24576, 16384}, H = 32, D = 128,
 // bf16: 915-999 us before, 770-880 us with the gates first, 740-820 us with 4-row groups and 64-token blocks (2-row
 // groups 870 us; 8-row groups 820-850 us at 155 VGPRs; streaming z loads or output stores within noise).
-constexpr int CT = 64;
+// A block takes 64 tokens when that gives the chip enough blocks, else fewer (conv_block): a decode step of 32
+// sequences is 6 blocks of 64 tokens, 49 us of serial rows, and 48 blocks of 4 tokens (H = 32, D = 128).
 constexpr int CP = 4;
+static int conv_block(long n_tok, int ugroups) {
+    int ct = 64;
+    while (ct > CP && (n_tok + ct - 1) / ct * ugroups < 512) ct /= 2;
+    return ct;
+}
 
 template <int D, bool BF>
-__global__ __launch_bounds__(256) void gdn_conv_inputs_k4_kernel(GdnInArgs a) {
+__global__ __launch_bounds__(256) void gdn_conv_inputs_k4_kernel(GdnInArgs a, int CT) {
     constexpr int LPU = D / 8, UPB = 256 / LPU;
     const int U = 2 * a.HK + a.HV;
     const int ugroups = (U + UPB - 1) / UPB;
@@ -306,22 +314,171 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(GatedNormArgs a) {
     store8(a.out, e0, BF ? DT_BF16 : DT_F32, r);
 }
 
+// One token per sequence with a carried state, the whole layer between its projections in one launch: the conv over
+// [prefix; z] with SiLU and l2norm, the gates, the delta-rule step, GatedNorm, and the new conv rows. Workgroup (h, b)
+// holds value head h's whole state (D x D fp32, 16 rows of 4 columns per thread: D * D / 64 threads), so the row of o
+// that the norm needs stays in the workgroup. Its loads go out before the small sums, which then cost no time of their
+// own: the pass is bound by reading and writing the state once (134 MB at B = 32, HV = 32, D = 128). As separate
+// kernels (conv pass, step, rounding, norm, the conv rows' concatenation and the parameters' casts to fp32, 15 launches
+// of 2 .. 49 us) the same step took 140 us of GPU time and 260 us of the host's.
+__device__ __forceinline__ float ldp(const void* p, long i, int dt) {
+    return dt == DT_BF16 ? bf2f(reinterpret_cast<const uint16_t*>(p)[i]) : reinterpret_cast<const float*>(p)[i];
+}
+
+template <int D, bool BF>
+__global__ __launch_bounds__(D * D / 64) void gdn_layer_step_kernel(GdnStepLayerArgs a) {
+    constexpr int NT = D * D / 64, NW = NT / 64, CG = D / 4, RSTEP = NT / CG, RPT = D / RSTEP;
+    static_assert(RPT == 16 && (CG == 16 || CG == 32 || CG == 64), "state split");
+    __shared__ float qs[D], ks[D], vs[D], os[D];
+    __shared__ __align__(16) float red[NW][D];
+    __shared__ float sq[2][NW];
+    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int HK = a.HK, HV = a.HV, r = HV / HK, hk = h / r, K = a.K;
+    const int cg = tid % CG, r0 = tid / CG;
+    const long C = (long)(2 * HK + HV) * D, bh = (long)b * HV + h;
+    using T = typename std::conditional<BF, uint16_t, float>::type;
+    auto ld = [](const T* p) { if constexpr (BF) return bf2f(*p); else return *p; };
+    float4 s[RPT];
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) s[i] = nt_ldf4(a.s_in + (bh * D + r0 + RSTEP * i) * D + 4 * cg);
+
+    // conv + SiLU of this head's q, k and v channels; the new conv rows (q and k by the first head that reads them)
+    const T* z = reinterpret_cast<const T*>(a.z) + b * a.z_st;
+    const T* pre = reinterpret_cast<const T*>(a.prefix) + (long)b * (K - 1) * C;
+    T* nxt = reinterpret_cast<T*>(a.conv_out) + (long)b * (K - 1) * C;
+    float ssq = 0.f, ssk = 0.f;
+    for (int i = tid; i < 3 * D; i += NT) {
+        const int kind = i / D, d = i % D;
+        const long c = (kind == 0 ? hk : (kind == 1 ? HK + hk : 2 * HK + h)) * (long)D + d;
+        const bool wr = kind == 2 || h % r == 0;
+        const T z0 = z[c];
+        float y = ld(&z0) * ldp(a.w, c * K + K - 1, a.w_dtype);
+        if (wr) nxt[(K - 2) * C + c] = z0;
+        for (int j = 1; j < K; ++j) {                    // the row j tokens back, weight column K - 1 - j
+            const T x = a.prefix ? pre[(K - 1 - j) * C + c] : T(0);
+            y = fmaf(ld(&x), ldp(a.w, c * K + K - 1 - j, a.w_dtype), y);
+            if (wr && j < K - 1) nxt[(K - 2 - j) * C + c] = x;
+        }
+        y = silu(y);
+        (kind == 0 ? qs : (kind == 1 ? ks : vs))[d] = y;
+        if (kind == 0) ssq += y * y;
+        else if (kind == 1) ssk += y * y;
+    }
+    ssq = unit_sum<64>(ssq);
+    ssk = unit_sum<64>(ssk);
+    if (lane == 0) { sq[0][wv] = ssq; sq[1][wv] = ssk; }
+    // gates, the same in every thread
+    const float ga = ldp(a.a, bh, a.io_dtype) + ldp(a.dt_bias, h, a.dt_dtype);
+    const float gg = -__expf(ldp(a.A_log, h, a.al_dtype)) * (ga > 20.f ? ga : log1pf(__expf(ga)));
+    const float al = __expf(gg), be = 1.f / (1.f + __expf(-ldp(a.b, bh, a.io_dtype)));
+    lds_barrier();
+    float tq = 0.f, tk = 0.f;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) { tq += sq[0][w]; tk += sq[1][w]; }
+    const float fq = rsqrtf(tq + a.l2_eps) * a.q_scale, fk = rsqrtf(tk + a.l2_eps);
+
+    // sum over the rows: lanes of one column group in the wave, then the waves
+    auto col_sum = [&](const float* x, float f, float (&out)[4]) {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < RPT; ++i) {
+            const float xr = x[r0 + RSTEP * i] * f;
+            v[0] += xr * s[i].x; v[1] += xr * s[i].y; v[2] += xr * s[i].z; v[3] += xr * s[i].w;
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+#pragma unroll
+            for (int off = CG; off < 64; off <<= 1) v[e] += __shfl_xor(v[e], off);
+        }
+        if constexpr (NW > 1) {
+            if (lane < CG) *reinterpret_cast<float4*>(&red[wv][4 * cg]) = make_float4(v[0], v[1], v[2], v[3]);
+            lds_barrier();
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) {
+                const float4 p = *reinterpret_cast<const float4*>(&red[w][4 * cg]);
+                out[0] += p.x; out[1] += p.y; out[2] += p.z; out[3] += p.w;
+            }
+            lds_barrier();
+        } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) out[e] = v[e];
+        }
+    };
+    float rc[4], dl[4], o4[4];
+    col_sum(ks, fk, rc);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) dl[e] = be * (vs[4 * cg + e] - al * rc[e]);
+#pragma unroll
+    for (int i = 0; i < RPT; ++i) {
+        const float k = ks[r0 + RSTEP * i] * fk;
+        s[i].x = al * s[i].x + k * dl[0];
+        s[i].y = al * s[i].y + k * dl[1];
+        s[i].z = al * s[i].z + k * dl[2];
+        s[i].w = al * s[i].w + k * dl[3];
+        nt_stf4(a.s_out + (bh * D + r0 + RSTEP * i) * D + 4 * cg, s[i]);
+    }
+    col_sum(qs, fq, o4);
+    if (r0 == 0) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) os[4 * cg + e] = BF ? bf_round(o4[e]) : o4[e];    // o.to(x.dtype)
+    }
+    lds_barrier();
+    // GatedNorm of the head's row by the first D / 8 lanes, as gated_norm_kernel
+    constexpr int LPR = D / 8;
+    if (tid < LPR) {
+        float o[8], zg[8], out[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) o[e] = os[8 * tid + e];
+        load8<BF>(a.zg, bh * D + 8 * tid, true, zg);
+        float ss = 0.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ss += o[e] * o[e];
+        ss = unit_sum<LPR>(ss);
+        const float inv = rsqrtf(ss / (float)D + a.eps);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const float w = ldp(a.norm_w, 8 * tid + e, a.nw_dtype);
+            if constexpr (BF) out[e] = bf_round(w * bf_round(o[e] * inv)) * silu(zg[e]);
+            else out[e] = w * (o[e] * inv) * silu(zg[e]);
+        }
+        store8(a.out, bh * D + 8 * tid, BF ? DT_BF16 : DT_F32, out);
+    }
+}
+
+int gdn_layer_step_dispatch(const GdnStepLayerArgs& a, hipStream_t stream) {
+    const dim3 grid((unsigned)a.HV, (unsigned)a.B), block((unsigned)(a.D * a.D / 64));
+    const bool bf = a.io_dtype == DT_BF16;
+    switch (a.D) {
+        case 64: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<64, true>), grid, block, 0, stream, a);
+                 else hipLaunchKernelGGL((gdn_layer_step_kernel<64, false>), grid, block, 0, stream, a); break;
+        case 128: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<128, true>), grid, block, 0, stream, a);
+                  else hipLaunchKernelGGL((gdn_layer_step_kernel<128, false>), grid, block, 0, stream, a); break;
+        case 256: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<256, true>), grid, block, 0, stream, a);
+                  else hipLaunchKernelGGL((gdn_layer_step_kernel<256, false>), grid, block, 0, stream, a); break;
+        default: return BF_ERR_UNSUPPORTED;
+    }
+    return (int)hipGetLastError();
+}
+
 int gdn_conv_inputs_dispatch(const GdnInArgs& a, hipStream_t stream) {
     const long threads = a.n_tok * (2 * a.HK + a.HV) * (a.D / 8);
     if (threads == 0) return 0;
     if (a.K == 4) {
         const int upb = 256 / (a.D / 8), U = 2 * a.HK + a.HV;
-        const long blocks = ((a.n_tok + CT - 1) / CT) * ((U + upb - 1) / upb);
+        const int ug = (U + upb - 1) / upb, ct = conv_block(a.n_tok, ug);
+        const long blocks = ((a.n_tok + ct - 1) / ct) * ug;
         if (blocks > 0x7fffffffL) return BF_STATUS_INVALID;
         const dim3 grid((unsigned)blocks), block(256);
         const bool bf = a.in_dtype == DT_BF16;
         switch (a.D) {
-            case 64: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<64, true>), grid, block, 0, stream, a);
-                     else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<64, false>), grid, block, 0, stream, a); break;
-            case 128: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<128, true>), grid, block, 0, stream, a);
-                      else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<128, false>), grid, block, 0, stream, a); break;
-            case 256: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<256, true>), grid, block, 0, stream, a);
-                      else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<256, false>), grid, block, 0, stream, a); break;
+            case 64: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<64, true>), grid, block, 0, stream, a, ct);
+                     else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<64, false>), grid, block, 0, stream, a, ct); break;
+            case 128: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<128, true>), grid, block, 0, stream, a, ct);
+                      else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<128, false>), grid, block, 0, stream, a, ct); break;
+            case 256: if (bf) hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<256, true>), grid, block, 0, stream, a, ct);
+                      else hipLaunchKernelGGL((gdn_conv_inputs_k4_kernel<256, false>), grid, block, 0, stream, a, ct); break;
             default: return BF_ERR_UNSUPPORTED;
         }
         return (int)hipGetLastError();

@@ -8,7 +8,9 @@ them three library calls do the work:
 
 - ``conv_inputs`` (``bf_gdn_conv_inputs``): causal conv + SiLU + l2norm + q scale + head repeat + beta / g gates;
 - the delta rule (``bf_gdn_fwd`` for a chunk, ``bf_gdn_step`` for one token with a carried state);
-- ``gated_norm`` (``bf_gated_norm``): weight * RMSNorm(o) * SiLU(z).
+- ``gated_norm`` (``bf_gated_norm``): weight * RMSNorm(o) * SiLU(z);
+
+or, for one token with a carried state, one call for all of it (``bf_gdn_layer_step``).
 
 ``gdn_layer_packed`` runs the same core on packed variable-length sequences (``cu_seqlens``), each sequence
 independent with its own conv prefix and state.
@@ -147,6 +149,12 @@ class GatedDeltaNet(nn.Module):
         s0 = None if cache is None else cache.get("S")
         step = s0 is not None and t == 1
         a, bb = self.in_proj_a(x), self.in_proj_b(x)
+        if step:
+            r = _layer_step(self, z.reshape(b, -1), a.reshape(b, -1), bb.reshape(b, -1), self.in_proj_z(x).reshape(b, -1),
+                            prefix, s0)
+            if r is not None:
+                o, cache["conv"], cache["S"] = r
+                return self.out_proj(o.view(b, t, self.vd))
         q, k, v, g, beta = conv_inputs(z.reshape(b * t, -1), self.conv1d.weight[:, 0], prefix, a, bb, self.A_log,
                                        self.dt_bias, c.lin_hk, c.lin_hv, c.lin_dk,
                                        cu_seqlens=_seqlens(b, t, x.device),
@@ -169,6 +177,38 @@ class GatedDeltaNet(nn.Module):
         if not fused:
             o = self.norm(o.view(b, t, c.lin_hv, c.lin_dv), zg)
         return self.out_proj(o.reshape(b, t, self.vd))
+
+
+def _layer_step(m, z, a, b, zg, prefix, state):
+    """One token per sequence on ``bf_gdn_layer_step``: z [B, C], a, b [B, hv], zg [B, hv * d] from the projections.
+    Returns (out [B, hv * d], new conv cache, new state), or None where the call does not apply (other dtypes or
+    layouts, a width-1 conv)."""
+    c = m.c
+    B, C = z.shape
+    K = c.conv_k
+    ok = (torch.float32, torch.bfloat16)
+    prm = (m.conv1d.weight, m.A_log, m.dt_bias, m.norm.weight)
+    if (K < 2 or z.dtype not in ok or not (z.dtype == a.dtype == b.dtype == zg.dtype) or B > 65535
+            or any(p.dtype not in ok or not p.is_contiguous() for p in prm) or z.stride(1) != 1 or z.stride(0) < C
+            or state.shape != (B, c.lin_hv, c.lin_dk, c.lin_dv) or c.lin_dk not in (64, 128, 256)
+            or (prefix is not None and prefix.shape != (B, K - 1, C)) or type(m.norm) is not GatedNorm):
+        return None
+    require_device(z, a, b, zg, prefix, state, *prm)
+    if prefix is not None:
+        prefix = prefix.to(z.dtype).contiguous()
+    a, b, zg, s_in = a.contiguous(), b.contiguous(), zg.contiguous(), state.float().contiguous()
+    conv = torch.empty(B, K - 1, C, dtype=z.dtype, device=z.device)
+    out, s = torch.empty_like(zg), torch.empty_like(s_in)
+    if any(t.data_ptr() % 16 for t in (zg, s_in)):
+        return None
+    w, al, dt, nw = prm
+    check(_lib.load().bf_gdn_layer_step(
+        z.data_ptr(), z.stride(0), None if prefix is None else prefix.data_ptr(), conv.data_ptr(), dtype_code(z.dtype),
+        w.data_ptr(), dtype_code(w.dtype), K, a.data_ptr(), b.data_ptr(), al.data_ptr(), dtype_code(al.dtype),
+        dt.data_ptr(), dtype_code(dt.dtype), zg.data_ptr(), nw.data_ptr(), dtype_code(nw.dtype), float(m.norm.eps), 1e-6,
+        float(c.lin_dk ** -0.5), s_in.data_ptr(), s.data_ptr(), out.data_ptr(), B, c.lin_hk, c.lin_hv, c.lin_dk,
+        stream_ptr(z.device)), "bf_gdn_layer_step")
+    return out, conv, s
 
 
 @torch.no_grad()

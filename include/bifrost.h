@@ -300,6 +300,21 @@ int bf_gated_norm(const void* o, int o_dtype, const void* z, const float* w, int
                   void* out, int io_dtype, void* stream);
 
 /*
+ * One token per sequence through the native layer between its projections, with a carried state
+ * (Heimdall/heimdall/hibrit.py:159-184 with t == 1): the values of bf_gdn_conv_inputs (fp32 q, k, v), bf_gdn_step and
+ * bf_gated_norm, and the new conv cache, in one launch.
+ *   z [B] rows of (2 HK + HV) D channels, z_st elements apart; prefix [B][K - 1][C] or null (zeros) and conv_out
+ *   [B][K - 1][C] (the last K - 1 rows of [prefix; z]; not the same memory); a, b [B][HV]; zg, out [B][HV][D]: all in
+ *   io_dtype; conv_w [C][K], A_log, dt_bias [HV], norm_w [D], each in its own dtype; state_in, state_out
+ *   [B][HV][D][D] f32 (may be the same). zg, the states and out 16-byte aligned; K in 2 .. 16.
+ */
+int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+                      int w_dtype, int K, const void* a, const void* b, const void* A_log, int A_log_dtype,
+                      const void* dt_bias, int dt_bias_dtype, const void* zg, const void* norm_w, int norm_w_dtype,
+                      float norm_eps, float l2_eps, float q_scale, const float* state_in, float* state_out, void* out,
+                      int B, int HK, int HV, int D, void* stream);
+
+/*
  * The native layer's delta rule and GatedNorm in one call (Heimdall/heimdall/hibrit.py:180-183: delta_rule, then
  * self.norm(o, z)), for a bf16 layer with D <= 128: bf_gdn_fwd with in_dtype = o_dtype = bf16, whose output row of
  * each (token, head) goes through bf_gated_norm's bf16 arithmetic before it is stored, so out holds the same bits as

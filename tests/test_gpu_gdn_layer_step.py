@@ -1,0 +1,72 @@
+"""bf_gdn_layer_step (one token per sequence through the native layer in one launch) against the separate calls it
+stands for, and the conv pass at the token counts where its block length changes."""
+import pytest
+import torch
+
+from test_gpu_gdn_layer import rel
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,hk,hv,d,K,prefixed", [(1, 1, 1, 64, 4, True), (3, 2, 6, 128, 4, True), (2, 2, 2, 256, 2, True),
+                                                  (2, 1, 2, 128, 4, False), (5, 3, 3, 64, 7, True)])
+def test_layer_step_equals_separate_calls(dev, dtype, b, hk, hv, d, K, prefixed):
+    """out, the state and the conv cache. fp32: sums of D terms in another order, ~1e-6; bf16: q, k, v stay fp32 in both,
+    so only values on a rounding edge of o or the norm differ by one bf16 step (2^-8) here and there."""
+    from heimdall_amd import gdn_layer as gl
+    from heimdall_amd.kernels import gdn_step
+    print(f"gdn layer step B={b} HK={hk} HV={hv} D={d} K={K} {dtype}", flush=True)
+    torch.manual_seed(1)
+    m = gl.GatedDeltaNet(gl.GdnLayerConfig(d=32, lin_hk=hk, lin_hv=hv, lin_dk=d, lin_dv=d, conv_k=K))
+    with torch.no_grad():
+        m.conv1d.weight.normal_(0, 0.5)
+        m.A_log.normal_(-2, 0.5)
+        m.dt_bias.normal_()
+        m.norm.weight.normal_(1, 0.2)
+    m = m.to(device=dev, dtype=dtype)
+    m.A_log.data = m.A_log.data.float()                    # each parameter in its own dtype
+    C = (2 * hk + hv) * d
+    wide = torch.randn(b, C + 8, device=dev).to(dtype)
+    z, a, bb = wide[:, :C], torch.randn(b, hv, device=dev).to(dtype), torch.randn(b, hv, device=dev).to(dtype)
+    zg = torch.randn(b, hv * d, device=dev).to(dtype)
+    prefix = torch.randn(b, K - 1, C, device=dev).to(dtype) if prefixed else None
+    s0 = torch.randn(b, hv, d, d, device=dev) * 0.3
+    with torch.no_grad():
+        out, conv, s = gl._layer_step(m, z, a, bb, zg, prefix, s0)
+        q, k, v, g, beta = gl.conv_inputs(z, m.conv1d.weight[:, 0], prefix, a, bb, m.A_log, m.dt_bias, hk, hv, d,
+                                          cu_seqlens=gl._seqlens(b, 1, dev), out_dtype=torch.float32)
+        o, s_ref = gdn_step(q, k, v, g, beta, s0)
+        ref = gl.gated_norm(o.to(dtype), zg.view(b, hv, d), m.norm.weight, m.norm.eps).reshape(b, -1)
+    full = torch.cat((prefix if prefixed else torch.zeros(b, K - 1, C, device=dev, dtype=dtype), z[:, None]), 1)
+    assert torch.equal(conv, full[:, 1:])
+    assert rel(s, s_ref) < 1e-5, rel(s, s_ref)
+    assert rel(out, ref) < (1e-5 if dtype == torch.float32 else 2e-3), rel(out, ref)
+
+
+@pytest.mark.parametrize("n", [1, 5, 64, 700, 5000])
+def test_conv_blocks(dev, n):
+    """Token blocks of 4 .. 64 (H = 32, D = 128: 5000 tokens are the first with 64-token blocks) over packed sequences
+    give the same bits as one token at a time with the rows before it as its prefix."""
+    from heimdall_amd import gdn_layer as gl
+    hk = hv = 32
+    d, K = 128, 4
+    print(f"conv blocks n={n}", flush=True)
+    C = 3 * hk * d
+    gen = torch.Generator(device=dev).manual_seed(n)
+    z = torch.randn(n, C, device=dev, generator=gen).bfloat16()
+    w = torch.randn(C, K, device=dev, generator=gen)
+    a, b = (torch.randn(n, hv, device=dev, generator=gen) for _ in range(2))
+    al, dt = torch.randn(hv, device=dev, generator=gen), torch.randn(hv, device=dev, generator=gen)
+    cut = sorted({0, n, n // 3, n // 2})
+    cu = torch.tensor(cut, dtype=torch.int32, device=dev)
+    run = lambda z_, pre, a_, b_, cu_: gl.conv_inputs(z_, w, pre, a_, b_, al, dt, hk, hv, d, cu_seqlens=cu_)
+    with torch.no_grad():
+        got = run(z, None, a, b, cu)
+        for i in sorted({0, n // 3, n // 2, n - 1}):
+            lo = max(c for c in cut if c <= i)
+            rows = z[max(lo, i - 3):i]
+            pre = torch.cat((torch.zeros(K - 1 - rows.shape[0], C, device=dev, dtype=z.dtype), rows))[None]
+            one = run(z[i:i + 1], pre, a[i:i + 1], b[i:i + 1], torch.tensor([0, 1], dtype=torch.int32, device=dev))
+            for x, y in zip(got, one):
+                assert torch.equal(x[i:i + 1], y), i
