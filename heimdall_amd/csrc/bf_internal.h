@@ -223,6 +223,27 @@ inline size_t window_split_bytes(const WinMap& m, int D) {
     return (size_t)8 * window_split_x(m) * window_split_p(m) * 128 * (D + 4) * sizeof(float);
 }
 
+// Key parts for queries over a long history (start >= 64 keys per part: each item's key range is about start + T / 2), of
+// the slots past the last full round of an XCD. Unsplit they cost one more round of whole items however few they are;
+// as P parts each, ceil(rem P / 32) rounds of 1/P item plus the partial rows' write and merge. A 64-key block of an
+// item takes ~2.1 us and a part's rows (133 KB at D = 256) ~14 us written and merged. 2048 queries over 14336 earlier
+// keys, H = 24, G = 4, D = 256 (48 slots per XCD, 16 of them as halves): 1047 -> 855 us a call.
+inline int window_long_parts(const WinMap& m, int T, long start) {
+    const long rem = m.per % 32;
+    const double nblk = (double)(start + T / 2) / 64.0;
+    double best = 0.95 * 2.1 * nblk;
+    int parts = 1;
+    for (int p = 2; rem && p <= 8 && nblk >= 8.0 * p; ++p) {
+        const double cost = (double)((rem * p + 31) / 32) * (2.1 * nblk / p + 14.0);
+        if (cost < best) { best = cost; parts = p; }
+    }
+    return parts;
+}
+inline size_t window_long_bytes(const WinMap& m, int T, long start, int D) {
+    const int p = window_long_parts(m, T, start);
+    return p > 1 ? (size_t)8 * (m.per % 32) * p * 128 * (D + 4) * sizeof(float) : 0;
+}
+
 int window_dispatch(const WinArgs& a, hipStream_t stream);
 
 // 4 consecutive elements of the memory read (fp32 or bf16) at element index i (a multiple of 4) as fp32.

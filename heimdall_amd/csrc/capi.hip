@@ -501,7 +501,7 @@ static int window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64
                       const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st, const void* ring_k, const void* ring_v,
                       const int64_t* ring_pos, const void* sink_k, const void* sink_v, int n_sinks, int mix,
                       const void* o_mem, int o_mem_dtype, const float* z, const float* mix_lse, const float* mem_scale,
-                      void* o, int o_dtype, float* lse, float* part, void* stream) {
+                      void* o, int o_dtype, float* lse, float* part, void* stream, bool long_parts = false) {
     if (B <= 0 || G <= 0 || R <= 0 || T <= 0 || W <= 0 || sinks < 0 || start < 0) return BF_STATUS_INVALID;
     if (!supported_dim(D) || !supported_dtype(in_dtype) || !supported_dtype(o_dtype)) return BF_STATUS_UNSUPPORTED;
     if (!q || !k || !v || !o) return BF_STATUS_INVALID;
@@ -521,8 +521,8 @@ static int window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64
     a.o = o; a.lse = lse;
     if (part && in_dtype == BF_DTYPE_BF16) {
         const bf::WinMap wm = bf::window_map(B, G, R, T, W, start);
-        a.split_x = bf::window_split_x(wm);
-        a.split_p = bf::window_split_p(wm);
+        a.split_p = long_parts ? bf::window_long_parts(wm, T, start) : bf::window_split_p(wm);
+        a.split_x = !long_parts ? bf::window_split_x(wm) : a.split_p > 1 ? (int)(wm.per % 32) : 0;
         a.part = part;
     }
     return bf::window_dispatch(a, static_cast<hipStream_t>(stream));
@@ -537,6 +537,28 @@ int bf_window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t s
     return window_fwd(B, G, R, D, T, W, sinks, start, in_dtype, q, q_sb, q_sh, q_st, k, k_sb, k_sh, k_st, v, v_sb,
                       v_sh, v_st, ring_k, ring_v, ring_pos, sink_k, sink_v, n_sinks, mix, o_mem, o_mem_dtype, z,
                       mix_lse, mem_scale, o, o_dtype, lse, nullptr, stream);
+}
+
+int bf_prefix_attention_workspace_size(int B, int G, int R, int D, int T, int cap, int64_t start, int dtype, size_t* bytes) {
+    if (!bytes || B <= 0 || G <= 0 || R <= 0 || T <= 0 || start < 0 || cap < start + T) return BF_STATUS_INVALID;
+    if (!supported_dim(D) || !supported_dtype(dtype)) return BF_STATUS_UNSUPPORTED;
+    *bytes = dtype == BF_DTYPE_BF16 ? bf::window_long_bytes(bf::window_map(B, G, R, T, cap, start), T, start, D) : 0;
+    return BF_STATUS_OK;
+}
+
+int bf_prefix_attention(int B, int G, int R, int D, int T, int cap, int64_t start, int dtype, const void* q, int64_t q_sb,
+                        int64_t q_sh, int64_t q_st, const void* k, const void* v, const int64_t* pos, void* o, int o_dtype,
+                        void* workspace, size_t workspace_bytes, void* stream) {
+    size_t need = 0;
+    const int st = bf_prefix_attention_workspace_size(B, G, R, D, T, cap, start, dtype, &need);
+    if (st) return st;
+    if (!k || !v || !pos) return BF_STATUS_INVALID;
+    if (need && (!workspace || workspace_bytes < need)) return BF_STATUS_WORKSPACE;
+    const size_t off = (size_t)start * D * (dtype == BF_DTYPE_BF16 ? 2 : 4);
+    const int64_t sg = (int64_t)cap * D, sb = G * sg;
+    return window_fwd(B, G, R, D, T, cap, 0, start, dtype, q, q_sb, q_sh, q_st, static_cast<const char*>(k) + off, sb, sg, D,
+                      static_cast<const char*>(v) + off, sb, sg, D, k, v, pos, nullptr, nullptr, 0, 0, nullptr, 0, nullptr,
+                      nullptr, nullptr, o, o_dtype, nullptr, need ? static_cast<float*>(workspace) : nullptr, stream, true);
 }
 
 int bf_mem_project(const void* x, int64_t n_tok, int nh, int D, int64_t x_st, int64_t x_sh, const float* f,

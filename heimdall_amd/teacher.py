@@ -12,7 +12,7 @@ The attended keys are the reference's on every path:
       ``bf_kv_attention`` over the sinks, the selected blocks and the window;
   t <= 16 without retrieval: ``bf_kv_attention`` (split-K over the cache, each query up to its own position);
   t == n: ``bf_window_fwd`` with a window as long as the sequence (causal, MFMA);
-  t < n:  ``bf_window_fwd`` with the cache buffer as its ring, so every earlier position is visible.
+  t < n:  ``bf_prefix_attention``, the window kernel with the cache buffer as its ring, so every earlier position is visible.
 """
 from typing import Optional
 
@@ -226,13 +226,14 @@ def _prefix_attention(qr, kb, vb, n, cache, out_dtype):
         rp = torch.arange(cap, dtype=torch.int64, device=dev)
         cache["ring_pos"] = rp
     q = qr if qr.stride(-1) == 1 else qr.contiguous()
-    kc, vc = kb[:, :, n - t:n], vb[:, :, n - t:n]
     o = torch.empty(B, t, H, D, dtype=out_dtype, device=dev)
-    st = lambda x: (int(x.stride(0)), int(x.stride(1)), int(x.stride(2)))
-    check(_lib.load().bf_window_fwd(B, G, H // G, D, t, cap, 0, n - t, dtype_code(kb.dtype), q.data_ptr(), *st(q),
-                                    kc.data_ptr(), *st(kc), vc.data_ptr(), *st(vc), kb.data_ptr(), vb.data_ptr(),
-                                    rp.data_ptr(), None, None, 0, 0, None, 0, None, None, None, o.data_ptr(),
-                                    dtype_code(out_dtype), None, stream_ptr(dev)), "bf_window_fwd")
+    lib, dt, nbytes = _lib.load(), dtype_code(kb.dtype), ctypes.c_size_t(0)
+    check(lib.bf_prefix_attention_workspace_size(B, G, H // G, D, t, cap, n - t, dt, ctypes.byref(nbytes)),
+          "bf_prefix_attention_workspace_size")
+    ws = workspace(nbytes.value, dev)
+    check(lib.bf_prefix_attention(B, G, H // G, D, t, cap, n - t, dt, q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
+                                  kb.data_ptr(), vb.data_ptr(), rp.data_ptr(), o.data_ptr(), dtype_code(out_dtype),
+                                  ws.data_ptr(), nbytes.value, stream_ptr(dev)), "bf_prefix_attention")
     return o
 
 

@@ -221,6 +221,18 @@ int bf_window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t s
                   int o_dtype, float* lse, void* stream);
 
 /*
+ * T queries at positions start .. start + T - 1 over every key up to their own position, in a cache whose last T rows
+ * are theirs: HybridAttention._teacher with 1 < t < n (Heimdall/heimdall/hibrit.py:275-290). k, v [B][G][cap][D] with
+ * rows 0 .. start + T - 1 filled (row = position, start + T <= cap), pos [cap] int64 = 0 .. cap - 1, q by element strides
+ * (batch, head, token), all in dtype; o [B][T][H][D] in o_dtype. The arithmetic of bf_window_fwd.
+ * Workspace: bf_prefix_attention_workspace_size bytes (0: none needed), 16-byte aligned.
+ */
+int bf_prefix_attention_workspace_size(int B, int G, int R, int D, int T, int cap, int64_t start, int dtype, size_t* bytes);
+int bf_prefix_attention(int B, int G, int R, int D, int T, int cap, int64_t start, int dtype, const void* q, int64_t q_sb,
+                        int64_t q_sh, int64_t q_st, const void* k, const void* v, const int64_t* pos, void* o, int o_dtype,
+                        void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Memory-branch keys of the converted layer, bf16 activations:
  *     out[t][h] = scale * normalize(x[t][h] F_h),   normalize(u) = u / max(||u||_2, 1e-12)
  * Replaces the two projections of HybridAttention._mem_inputs (Heimdall/heimdall/hibrit.py:327-334):

@@ -1,0 +1,53 @@
+"""A chunk of a kept layer whose queries' keys are taken in parts (``bf_prefix_attention``), against the oracle.
+
+The part counts follow the launch's slots per XCD and the key blocks of an item; the cases cover a few slots in many parts,
+one query row past a 128-query item, the shortest history that is split, and a last round more than half full. Tolerance: q, k, v
+and the probabilities are bf16 (2^-9 each) with fp32 sums, as in the unsplit kernel.
+"""
+import ctypes
+
+import pytest
+import torch
+
+from oracle import teacher as ot
+
+TOL16 = 8e-3
+
+
+def _parts(B, G, R, D, T, cap, start):
+    from heimdall_amd import _lib
+    n = ctypes.c_size_t(0)
+    assert _lib.load().bf_prefix_attention_workspace_size(B, G, R, D, T, cap, start, 1, ctypes.byref(n)) == 0
+    return n.value
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("B,H,G,D,n,t", [
+    (1, 4, 2, 256, 4200, 17),          # one item row, the most parts
+    (2, 8, 2, 128, 3000, 129),         # a second item of one query
+    (1, 24, 4, 64, 1600, 100),         # few key blocks: fewer parts
+    (1, 8, 1, 64, 9000, 2100),         # 17 query blocks of 8 heads: 24 slots per XCD, some past an XCD's items
+])
+def test_prefix_parts(dev, B, H, G, D, n, t):
+    from heimdall_amd.teacher import teacher
+    assert _parts(B, G, H // G, D, t, n + 256, n - t) > 0
+    gen = torch.Generator().manual_seed(n)
+    qr, kr, v = (torch.randn(B, h, n, D, generator=gen).to(torch.bfloat16) for h in (H, G, G))
+    cache = {"k": kr[:, :, :n - t].to(dev), "v": v[:, :, :n - t].to(dev)}
+    m = type("M", (), {"retrieval": None})()
+    o = teacher(m, qr[:, :, n - t:].to(dev), kr[:, :, n - t:].to(dev), v[:, :, n - t:].transpose(1, 2).to(dev), cache)
+    ocache = {"k": kr[:, :, :n - t].float(), "v": v[:, :, :n - t].float()}
+    ref = ot.teacher(qr[:, :, n - t:].float(), kr[:, :, n - t:].float(), v[:, :, n - t:].transpose(1, 2).float(), ocache, None)
+    err = ((o.double().cpu() - ref.double()).norm() / ref.double().norm()).item()
+    assert err < TOL16, err
+
+
+def test_prefix_workspace_arguments():
+    from heimdall_amd import _lib
+    n, lib = ctypes.c_size_t(0), _lib.load()
+    size = lib.bf_prefix_attention_workspace_size
+    assert size(1, 4, 6, 256, 2048, 24576, 14336, 0, ctypes.byref(n)) == 0 and n.value == 0       # fp32: never in parts
+    assert size(1, 4, 6, 256, 2048, 24576, 64, 1, ctypes.byref(n)) == 0                           # a short history
+    assert size(1, 4, 6, 96, 2048, 24576, 64, 1, ctypes.byref(n)) == -2
+    assert size(1, 4, 6, 256, 2048, 2048, 1, 1, ctypes.byref(n)) == -1                            # start + T > cap
+    assert lib.bf_prefix_attention(1, 4, 6, 256, 2048, 24576, 14336, 1, 256, 0, 0, 0, 256, 256, 256, 256, 1, None, 0, None) == -3
