@@ -101,6 +101,47 @@ __device__ __forceinline__ uint4 scale16<BF16>(const uint4& v, float s) {
     return make_uint4(scale_pair(v.x, s), scale_pair(v.y, s), scale_pair(v.z, s), scale_pair(v.w, s));
 }
 
+// ds_read_b64_tr_b16: in each 16-lane group, output lane 4q + r receives element r of the 8-byte chunks that lanes
+// 4e + q (e = 0..3) address, in order of e.
+typedef short v4s __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 lds_tr16(const char* p) {
+    const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p));
+    return make_uint2((uint16_t)v[0] | ((uint32_t)(uint16_t)v[1] << 16),
+                      (uint16_t)v[2] | ((uint32_t)(uint16_t)v[3] << 16));
+}
+
+// fp32 operands of a bf16 MFMA: x = p[0] + p[1] + p[2] exactly, three bf16 planes (8 + 8 + 8 of the 24 significand bits:
+// the first truncated, so it never overflows, the second rounded to nearest, the third what is left). Of the nine plane
+// products the six down to 2^-16 of the first are summed (mma3); the three left out are below 2^-23 |a b| and 2^-26 on
+// average, of either sign, less than the rounding of an fp32 product. Six v_mfma_f32_16x16x32_bf16 take 96 cycles, the
+// eight v_mfma_f32_16x16x4_f32 of the same contraction 256. An infinite operand gives NaN.
+struct Planes {
+    uint4 p[3];
+};
+__device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
+    const uint32_t ux = __float_as_uint(x), uy = __float_as_uint(y);
+    h = __builtin_amdgcn_perm(uy, ux, 0x07060302u);                  // the high halves, x's in the low half
+    const float rx = x - __uint_as_float(ux & 0xffff0000u), ry = y - __uint_as_float(uy & 0xffff0000u);
+    m = pack_bf16x2(rx, ry);
+    l = pack_bf16x2(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u));
+}
+__device__ __forceinline__ Planes split8(const float4& a, const float4& b) {
+    Planes s;
+    split_pair(a.x, a.y, s.p[0].x, s.p[1].x, s.p[2].x);
+    split_pair(a.z, a.w, s.p[0].y, s.p[1].y, s.p[2].y);
+    split_pair(b.x, b.y, s.p[0].z, s.p[1].z, s.p[2].z);
+    split_pair(b.z, b.w, s.p[0].w, s.p[1].w, s.p[2].w);
+    return s;
+}
+__device__ __forceinline__ void mma3(f32x4& acc, const Planes& a, const Planes& b) {
+    mma<BF16>(acc, a.p[2], b.p[0]);
+    mma<BF16>(acc, a.p[0], b.p[2]);
+    mma<BF16>(acc, a.p[1], b.p[1]);
+    mma<BF16>(acc, a.p[1], b.p[0]);
+    mma<BF16>(acc, a.p[0], b.p[1]);
+    mma<BF16>(acc, a.p[0], b.p[0]);
+}
+
 // Store 4 consecutive fp32 values (an accumulator column segment) as element type E.
 template <class E>
 __device__ __forceinline__ void store4(typename E::T* p, float a, float b, float c, float d);

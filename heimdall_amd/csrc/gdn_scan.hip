@@ -251,15 +251,6 @@ __device__ __forceinline__ constexpr int tpart(int tile) {
     return E::KF * (tile / (E::VEC / 4)) + 4 * (tile % (E::VEC / 4));
 }
 
-typedef short v4s __attribute__((ext_vector_type(4)));
-// ds_read_b64_tr_b16: in each 16-lane group, output lane 4q + r receives element r of the 8-byte chunks that lanes
-// 4e + q (e = 0..3) address.
-__device__ __forceinline__ uint2 lds_tr16(const char* p) {
-    const v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) v4s*)(p));
-    return make_uint2((uint16_t)v[0] | ((uint32_t)(uint16_t)v[1] << 16),
-                      (uint16_t)v[2] | ((uint32_t)(uint16_t)v[3] << 16));
-}
-
 // GN (output scan, bf16, whole rows per workgroup): each o row goes through the GatedNorm of the native layer before
 // it is stored, with the arithmetic of gated_norm_kernel (gdn_layer.hip), so the bits equal the two separate passes.
 template <class E, int D, bool OUT, bool BO, bool GN = false>

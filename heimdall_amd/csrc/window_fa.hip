@@ -62,15 +62,6 @@ __device__ __forceinline__ int fa_swk(int row) { return NBLK >= 16 ? (row & 15) 
 template <int NBLK>
 __device__ __forceinline__ int fa_swv(int row) { return NBLK >= 16 ? 2 * (row & 7) : 2 * ((row >> 1) & 3); }
 
-typedef short fa_v4s __attribute__((ext_vector_type(4)));
-// ds_read_b64_tr_b16: in each 16-lane group, lane 4q + r receives element r of the 8-byte chunks that lanes 4e + q
-// (e = 0..3) address, in order of e.
-__device__ __forceinline__ uint2 fa_tr16(const char* p) {
-    const fa_v4s v = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) fa_v4s*)(p));
-    return make_uint2((uint16_t)v[0] | ((uint32_t)(uint16_t)v[1] << 16), (uint16_t)v[2] | ((uint32_t)(uint16_t)v[3] << 16));
-}
-
-
 // max / sum of a value over lanes l, l ^ 16, l ^ 32, l ^ 48 by lane swaps (v_permlane16_swap, v_permlane32_swap)
 __device__ __forceinline__ float fa_max4(float v) {
     const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -411,7 +402,7 @@ __global__ __launch_bounds__(FaShape<D>::NT, 1) void window_fa_kernel(WinArgs a)
             constexpr int VPF = 4;
             auto read_v = [&](int dt) {
                 const char* p = Vb + vbase[dt % NVB] + 32 * f * ROWB + 256 * (dt / NVB);
-                const uint2 lo = fa_tr16(p), hi = fa_tr16(p + 16 * ROWB);
+                const uint2 lo = lds_tr16(p), hi = lds_tr16(p + 16 * ROWB);
                 return make_uint4(lo.x, lo.y, hi.x, hi.y);
             };
             uint4 vr[VPF];
