@@ -125,12 +125,12 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32
     m = pack_bf16x2(rx, ry);
     l = pack_bf16x2(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u));
 }
-__device__ __forceinline__ Planes split8(const float4& a, const float4& b) {
+__device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b) {
     Planes s;
-    split_pair(a.x, a.y, s.p[0].x, s.p[1].x, s.p[2].x);
-    split_pair(a.z, a.w, s.p[0].y, s.p[1].y, s.p[2].y);
-    split_pair(b.x, b.y, s.p[0].z, s.p[1].z, s.p[2].z);
-    split_pair(b.z, b.w, s.p[0].w, s.p[1].w, s.p[2].w);
+    split_pair(a[0], a[1], s.p[0].x, s.p[1].x, s.p[2].x);
+    split_pair(a[2], a[3], s.p[0].y, s.p[1].y, s.p[2].y);
+    split_pair(b[0], b[1], s.p[0].z, s.p[1].z, s.p[2].z);
+    split_pair(b[2], b[3], s.p[0].w, s.p[1].w, s.p[2].w);
     return s;
 }
 __device__ __forceinline__ void mma3(f32x4& acc, const Planes& a, const Planes& b) {
@@ -140,6 +140,20 @@ __device__ __forceinline__ void mma3(f32x4& acc, const Planes& a, const Planes& 
     mma<BF16>(acc, a.p[1], b.p[0]);
     mma<BF16>(acc, a.p[0], b.p[1]);
     mma<BF16>(acc, a.p[0], b.p[0]);
+}
+
+// max / sum of a value over lanes l, l ^ 16, l ^ 32, l ^ 48 by lane swaps (v_permlane16_swap, v_permlane32_swap)
+__device__ __forceinline__ float lane_max4(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float lane_sum4(float v) {
+    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
 // Store 4 consecutive fp32 values (an accumulator column segment) as element type E.

@@ -62,20 +62,6 @@ __device__ __forceinline__ int fa_swk(int row) { return NBLK >= 16 ? (row & 15) 
 template <int NBLK>
 __device__ __forceinline__ int fa_swv(int row) { return NBLK >= 16 ? 2 * (row & 7) : 2 * ((row >> 1) & 3); }
 
-// max / sum of a value over lanes l, l ^ 16, l ^ 32, l ^ 48 by lane swaps (v_permlane16_swap, v_permlane32_swap)
-__device__ __forceinline__ float fa_max4(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
-}
-__device__ __forceinline__ float fa_sum4(float v) {
-    const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
-    const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return __uint_as_float(b[0]) + __uint_as_float(b[1]);
-}
-
 // Streaming (non-temporal) accesses of the epilogue: the memory rows are read once and the output rows written once,
 // so they should not displace the K / V tiles other workgroups re-read from L2 (the sliding window over 32768
 // queries ran 1909-1927 us against 1938-1963 us with ordinary accesses).
@@ -362,7 +348,7 @@ __global__ __launch_bounds__(FaShape<D>::NT, 1) void window_fa_kernel(WinArgs a)
             for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) bm = fmaxf(bm, s[kt][qt][e]);
-            bm = fa_max4(bm) * cs;
+            bm = lane_max4(bm) * cs;
             const bool up = bm > m[qt] + FA_SLACK;
             if (__builtin_amdgcn_ballot_w64(up)) {
                 const float mn = up ? bm : m[qt];
@@ -471,7 +457,7 @@ __global__ __launch_bounds__(FaShape<D>::NT, 1) void window_fa_kernel(WinArgs a)
         float* pp = a.part + (((long)xcd * sx + (idx - (per - sx))) * P + half) * FA_BQ * (D + 4);
 #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
-            const float lt = fa_sum4(l[qt]);
+            const float lt = lane_sum4(l[qt]);
             const int qi = QW * wv + 16 * qt + l16;
             if (qi >= nq) continue;
             float* row = pp + (long)qi * (D + 4);
@@ -516,7 +502,7 @@ __global__ __launch_bounds__(FaShape<D>::NT, 1) void window_fa_kernel(WinArgs a)
     float gam[QT];
 #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-        const float lt = fa_sum4(l[qt]);
+        const float lt = lane_sum4(l[qt]);
         const int qi = QW * wv + 16 * qt + l16;
         const float inv = 1.f / lt;
         const float lse = (m[qt] + __log2f(lt)) * FA_LN2;

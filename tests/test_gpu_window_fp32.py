@@ -1,0 +1,54 @@
+"""fp32 window attention at the edges of its tiles, against the same attention in 64 bits: 64- and 128-query workgroups (few
+and many items), a last item of one query, windows shorter than a block, rings with missing rows, sinks past and before them.
+
+Tolerance: every product carries its 24 bits and the sums are fp32, D + W of them in order, so the error stays within a
+few 2^-24 per row: 2e-6 of the norm, and 1e-5 in the log-sum-exp.
+"""
+import math
+
+import pytest
+import torch
+
+from test_gpu_window import make_case, run
+
+pytestmark = pytest.mark.gpu
+
+
+def reference(c):
+    """(o, lse) in 64 bits from the definition: a loop over sequences and heads."""
+    B, H, G, T, W, start = (c[k] for k in ("B", "H", "G", "T", "W", "start"))
+    old = torch.arange(max(0, start - W), start)
+    old = old[c["ring_pos"][old % W] == old]
+    ns = c["sink_k"].shape[2]
+    pos = torch.cat((torch.arange(ns), old, torch.arange(start, start + T)))
+    sink = torch.arange(len(pos)) < ns
+    p = torch.arange(start, start + T)[:, None]
+    see = torch.where(sink, pos <= p, (pos >= c["S"]) & (pos <= p) & (p - pos < W))
+    o, lse = torch.empty(B, T, H, c["D"], dtype=torch.float64), torch.empty(B, H, T, dtype=torch.float64)
+    for b in range(B):
+        for h in range(H):
+            g = h // (H // G)
+            k = torch.cat((c["sink_k"][b, g], c["ring_k"][b, g, old % W], c["kr"][b, g])).double()
+            v = torch.cat((c["sink_v"][b, g], c["ring_v"][b, g, old % W], c["v"][b, :, g])).double()
+            s = (c["qr"][b, h].double() @ k.t() / math.sqrt(c["D"])).masked_fill(~see, -math.inf)
+            lse[b, h] = s.logsumexp(-1)
+            o[b, :, h] = s.softmax(-1) @ v
+    return o, lse
+
+
+@pytest.mark.parametrize("B,H,G,D,T,W,S,start,miss", [
+    (1, 2, 1, 256, 65, 40, 3, 0, 0.0),          # 64-query items, the second of one query
+    (1, 4, 2, 256, 33, 64, 2, 777, 0.2),        # a wrapped ring with missing rows
+    (1, 66, 22, 256, 257, 96, 4, 500, 0.1),     # 128-query items, the third of one query
+    (3, 24, 4, 128, 300, 33, 1, 0, 0.0),
+    (1, 96, 8, 64, 191, 200, 4, 150, 0.0),      # a ring that is not full
+    (1, 8, 8, 64, 1, 16, 0, 40, 0.0),           # one query, no sinks
+])
+def test_window_fp32_tiles(dev, B, H, G, D, T, W, S, start, miss):
+    c = make_case(B, H, G, D, T, W, S, start, seed=T + W, invalid_frac=miss, dtype=torch.float32)
+    print(f"window fp32 B={B} H={H} G={G} D={D} T={T} W={W} S={S} start={start}", flush=True)
+    o, lse = run(c, dev)[:2]
+    ref, ref_lse = reference(c)
+    err = ((o.cpu().double() - ref).norm() / ref.norm()).item()
+    assert err < 2e-6, err
+    assert (lse.cpu().double() - ref_lse).abs().max().item() < 1e-5
