@@ -13,7 +13,7 @@
 //   d(v b) = M^T dvn, d(k b e^gc) = M^T dw, dM = dvn (v b)^T + dw (k b e^gc)^T, dA = -strict_lower(M^T dM M^T)
 // followed by the decay, gate and cumulative-sum chains (chunk_final_kernel).
 //
-// Kernels: bgemm_kernel (batched strided fp32 GEMM on v_mfma_f32_16x16x4f32, optional triangular mask, addend and
+// Kernels: bgemm_kernel (batched strided fp32 GEMM on bf16 MFMAs over exact planes, optional triangular mask, addend and
 // accumulate, in-chunk decay, row scale and row / column dots in the epilogue), chunk_prep_kernel,
 // unit_lower_inverse_kernel, walk_fwd_kernel / walk_bwd_kernel (the two state walks), state_dot_kernel,
 // chunk_final_kernel, dg_scan_kernel. The host side runs the forward walk, the products that need only its states and
@@ -67,19 +67,20 @@ struct BgArgs {
     int acc, mask, cfrag;               // cfrag: C (per z at its batch offset) in fragment order, cm / cn unused
 };
 
-// Tiles of 64 x BN (BN = 64 or 128; 4 waves of 32 x BN/2) over K steps of 32. Each step's 64 x 32 tile of A and
-// 32 x BN tile of B are read with 16-byte loads along whichever dimension is contiguous (AK: A's k, else its m; BK:
-// B's k, else its n) and stored in LDS in the same orientation with 16-byte writes: a k-contiguous operand as
-// [row][k] (pitch 36 floats: the 16 rows of a fragment hit distinct banks; a fragment is one 16-byte read), the other
-// as [k][row] (pitch 4 mod 16 floats: the four k rows a fragment read spans fall 16 banks apart; a fragment is four
-// 4-byte reads). Fragment value j of lane (i, q) is k = 16 kh + 4 q + j for both operands. The LDS tiles are double
-// buffered: step s computes from one buffer, then writes step s + 1's operands (loaded from global during step s - 1)
-// into the other and issues step s + 2's loads, with one barrier per step.
+// Tiles of 64 x BN (BN = 64 or 128; 4 waves of 32 x BN/2) over K steps of 32, on bf16 MFMAs over three exact planes per
+// operand (Planes, bf_common.h): the fp32 MFMA bound the larger products, at half of its peak. Each step's 64 x 32 tile of
+// A and 32 x BN tile of B are read with 16-byte loads along whichever dimension is contiguous (AK: A's k, else its m; BK:
+// B's k, else its n), split, and stored in LDS in the same orientation with 8-byte writes. Position 8 q + j of a 32-wide
+// step is k = 4 q + j (j < 4) or 12 + 4 q + j, for both operands: a k-contiguous operand is stored [row][position] (pitch
+// 80 bytes: the 16 rows of a fragment hit distinct banks; a fragment is one 16-byte read), the other [k][row] (pitch an odd
+// multiple of 32 bytes; a fragment is two transposing reads). One LDS tile (46 KB at most, three workgroups per CU, which
+// fill each other's waits): the next step's loads are in flight while this one multiplies.
+// 8192 tokens, G = 4, R = 6, D = 256, forward and backward: 3102 -> 2958 us.
 // EX: the epilogue extras compiled in: 0 none, 1 msc and rdo, 2 also dgc and cdo. The plain products measurably need
 // the small epilogue, and the row-scaled ones one without the per-element decay.
 template <bool AK, bool BK, int BN, int EX>
 __global__ __launch_bounds__(BW_NT) void bgemm_kernel(BgArgs a) {
-    constexpr int KS = 32, LDK = KS + 4;        // k per step, LDS row pitch (floats)
+    constexpr int KS = 32, LDK = KS + 8;        // k per step, pitch of a k-contiguous operand's rows (elements)
     constexpr int WN = BN / 2, TU = WN / 16;    // wave tile 32 x WN: 2 x TU MFMA tiles
     constexpr int KQ = KS / 4, KG = KS / 16;    // 16-byte slots along k per row; 16-k groups per step
     constexpr int NA = 64 * KS / 1024, NB = BN * KS / 1024;   // 16-byte global loads per thread per step
@@ -97,12 +98,12 @@ __global__ __launch_bounds__(BW_NT) void bgemm_kernel(BgArgs a) {
     const int tm = blockIdx.y * 64, tn = blockIdx.z * BN;
     const int m0 = (wv >> 1) * 32, n0 = (wv & 1) * WN;      // the wave's 32 x WN block inside the tile
     const int i = lane & 15, q = lane >> 4;
-    constexpr int AR = AK ? 64 : KS, AP = AK ? LDK : 64 + 4;     // LDS rows and pitch of A
-    constexpr int BR = BK ? BN : KS, BP = BK ? LDK : BN + 4;     // and of B
-    constexpr int ASZ = 2 * AR * AP, BSZ = 2 * BR * BP, CSZ = 64 * (BN + 4);
-    __shared__ __align__(16) float lds[ASZ + BSZ > CSZ ? ASZ + BSZ : CSZ];   // operand tiles, then the output tile
-    float (*As)[AR][AP] = reinterpret_cast<float (*)[AR][AP]>(lds);
-    float (*Bs)[BR][BP] = reinterpret_cast<float (*)[BR][BP]>(lds + ASZ);
+    constexpr int AP = AK ? LDK : 64 + 16, ASZ = (AK ? 64 : KS) * AP;     // LDS pitch and plane of A (elements)
+    constexpr int BP = BK ? LDK : BN + 16, BSZ = (BK ? BN : KS) * BP;     // and of B
+    constexpr int LSZ = 3 * (ASZ + BSZ) * 2, CSZ = 64 * (BN + 4) * 4;
+    __shared__ __align__(16) char lds[LSZ > CSZ ? LSZ : CSZ];            // operand planes, then the output tile
+    uint16_t* As = reinterpret_cast<uint16_t*>(lds);
+    uint16_t* Bs = As + 3 * ASZ;
     f32x4 acc[2][TU];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -133,42 +134,51 @@ __global__ __launch_bounds__(BW_NT) void bgemm_kernel(BgArgs a) {
         const int k = k0 + tid / 16 + 16 * (h % KG);
         return *reinterpret_cast<const float4*>(B + koff(k, a.sbk, a.bk) + tn + (tid % 16) * 4 + 64 * (h / KG));
     };
-    auto store = [&](int buf, const float4 (&xa)[NA], const float4 (&sa)[NA], const float4 (&xb)[NB]) {
+    // four values into the planes of T (plane size sz): along k from slot k4 of a row, or along rows at one k
+    auto put = [&](uint16_t* T, int sz, int at, const float4& x) {
+        uint2 p[3];
+        split_pair(x.x, x.y, p[0].x, p[1].x, p[2].x);
+        split_pair(x.z, x.w, p[0].y, p[1].y, p[2].y);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(T + i * sz + at) = p[i];
+    };
+    const int kpos = 8 * (tid % KQ % 4) + 4 * (tid % KQ / 4);             // position of this thread's slot of a row
+    auto store = [&](const float4 (&xa)[NA], const float4 (&sa)[NA], const float4 (&xb)[NB]) {
 #pragma unroll
         for (int h = 0; h < NA; ++h) {
             const float4 x = make_float4(xa[h].x * sa[h].x, xa[h].y * sa[h].y, xa[h].z * sa[h].z, xa[h].w * sa[h].w);
-            if (AK) *reinterpret_cast<float4*>(&As[buf][tid / KQ + (256 / KQ) * h][(tid % KQ) * 4]) = x;
-            else *reinterpret_cast<float4*>(&As[buf][tid / 16 + 16 * (h % KG)][(tid % 16) * 4 + 64 * (h / KG)]) = x;
+            put(As, ASZ, AK ? (tid / KQ + (256 / KQ) * h) * AP + kpos
+                            : (tid / 16 + 16 * (h % KG)) * AP + (tid % 16) * 4 + 64 * (h / KG), x);
         }
 #pragma unroll
-        for (int h = 0; h < NB; ++h) {
-            if (BK) *reinterpret_cast<float4*>(&Bs[buf][tid / KQ + (256 / KQ) * h][(tid % KQ) * 4]) = xb[h];
-            else *reinterpret_cast<float4*>(&Bs[buf][tid / 16 + 16 * (h % KG)][(tid % 16) * 4 + 64 * (h / KG)]) = xb[h];
-        }
+        for (int h = 0; h < NB; ++h)
+            put(Bs, BSZ, BK ? (tid / KQ + (256 / KQ) * h) * BP + kpos
+                            : (tid / 16 + 16 * (h % KG)) * BP + (tid % 16) * 4 + 64 * (h / KG), xb[h]);
     };
-    auto compute = [&](int buf) {
+    // planes of the fragment of rows r0 .. r0 + 15
+    auto frag = [&](const uint16_t* T, int sz, int pitch, bool kc, int r0) {
+        Planes f;
 #pragma unroll
-        for (int kh = 0; kh < KG; ++kh) {
-            uint4 af[2], bf[TU];
-            const int kr = 16 * kh + 4 * q;
-#pragma unroll
-            for (int t = 0; t < 2; ++t) {
-                const int r = m0 + 16 * t + i;
-                af[t] = AK ? *reinterpret_cast<const uint4*>(&As[buf][r][kr])
-                           : make_uint4(__float_as_uint(As[buf][kr][r]), __float_as_uint(As[buf][kr + 1][r]),
-                                        __float_as_uint(As[buf][kr + 2][r]), __float_as_uint(As[buf][kr + 3][r]));
+        for (int j = 0; j < 3; ++j) {
+            if (kc) {
+                f.p[j] = ld16(T + j * sz + (r0 + i) * pitch + 8 * q);
+            } else {
+                const char* p = reinterpret_cast<const char*>(T + j * sz + (4 * q + (i >> 2)) * pitch + r0 + 4 * (i & 3));
+                const uint2 lo = lds_tr16(p), hi = lds_tr16(p + 32 * pitch);
+                f.p[j] = make_uint4(lo.x, lo.y, hi.x, hi.y);
             }
+        }
+        return f;
+    };
+    auto compute = [&]() {
+        Planes af[2];
 #pragma unroll
-            for (int u = 0; u < TU; ++u) {
-                const int r = n0 + 16 * u + i;
-                bf[u] = BK ? *reinterpret_cast<const uint4*>(&Bs[buf][r][kr])
-                           : make_uint4(__float_as_uint(Bs[buf][kr][r]), __float_as_uint(Bs[buf][kr + 1][r]),
-                                        __float_as_uint(Bs[buf][kr + 2][r]), __float_as_uint(Bs[buf][kr + 3][r]));
-            }
+        for (int t = 0; t < 2; ++t) af[t] = frag(As, ASZ, AP, AK, m0 + 16 * t);
 #pragma unroll
-            for (int t = 0; t < 2; ++t)
+        for (int u = 0; u < TU; ++u) {
+            const Planes bf = frag(Bs, BSZ, BP, BK, n0 + 16 * u);
 #pragma unroll
-                for (int u = 0; u < TU; ++u) mma<F32>(acc[t][u], af[t], bf[u]);
+            for (int t = 0; t < 2; ++t) mma3(acc[t][u], af[t], bf);
         }
     };
     if (!skip) {
@@ -181,16 +191,12 @@ __global__ __launch_bounds__(BW_NT) void bgemm_kernel(BgArgs a) {
             for (int h = 0; h < NB; ++h) xb[h] = load_b(s * KS, h);
         };
         fetch(0);
-        store(0, xa, sa, xb);
-        if (ns > 1) fetch(1);
-        __syncthreads();
         for (int s = 0; s < ns; ++s) {
-            compute(s & 1);
-            if (s + 1 < ns) {
-                store((s + 1) & 1, xa, sa, xb);
-                if (s + 2 < ns) fetch(s + 2);
-            }
-            __syncthreads();
+            store(xa, sa, xb);
+            lds_barrier();
+            fetch(min(s + 1, ns - 1));                      // (the last step's again: no condition for the loads to join)
+            compute();
+            lds_barrier();
         }
     }
     const float* msc = EX >= 1 && a.msc ? a.msc + z0 * a.ms0 + z1 * a.ms1 : nullptr;
@@ -984,13 +990,13 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
     ok((int)hipEventRecord(ev[0], s));
     ok((int)hipStreamWaitEvent(s2, ev[0], 0));
     const dim3 wgrid(a.num_seqs, G, D / 16);               // walk_sw<D>() == 1: one workgroup per 16-column strip
-    // The walks are the call's critical path on few workgroups: each asks for LDS up to 128 KB of the CU's 160 KB,
-    // so no product workgroup (34-55 KB) shares its CU and slows it (2.11 -> 2.06 ms with the attn product after the
+    // The walks are the call's critical path on few workgroups: each asks for LDS up to 136 KB of the CU's 160 KB,
+    // so no product workgroup (31-46 KB) shares its CU and slows it (2.11 -> 2.06 ms with the attn product after the
     // fork, T = 8192, G = 4, R = 6, D = 256)
     auto walk = [&](bool fwd, hipStream_t st) {
         const dim3 blk(64 * (D >= 128 ? 8 : 4));
         const int kh = D >= 128 ? 2 : 1;
-        const size_t res = 128 * 1024 - (size_t)(16 * (D + 4) + kh * 16 * (BC + 4)) * sizeof(float);
+        const size_t res = 136 * 1024 - (size_t)(16 * (D + 4) + kh * 16 * (BC + 4)) * sizeof(float);
         if (D == 64) hipLaunchKernelGGL(fwd ? walk_fwd_kernel<64> : walk_bwd_kernel<64>, wgrid, blk, res, st, a);
         else if (D == 128) hipLaunchKernelGGL(fwd ? walk_fwd_kernel<128> : walk_bwd_kernel<128>, wgrid, blk, res, st, a);
         else hipLaunchKernelGGL(fwd ? walk_fwd_kernel<256> : walk_bwd_kernel<256>, wgrid, blk, res, st, a);
