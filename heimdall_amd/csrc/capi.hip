@@ -43,7 +43,7 @@ bool supported_dtype(int dt) { return dt == BF_DTYPE_F32 || dt == BF_DTYPE_BF16;
 size_t esize(int dt) { return dt == BF_DTYPE_BF16 ? 2 : 4; }
 
 struct GdnLayout {
-    size_t gcum, T, phi, c, n, sin, total;
+    size_t gcum, T, phi, c, n, sin, spl, need, total;     // need: without the planes at spl (0: none)
     int max_chunks, seg_chunks, max_segs;
 };
 
@@ -97,6 +97,10 @@ GdnLayout gdn_layout(int64_t total_tokens, int num_seqs, int G, int R, int D, in
     L.c = off;    off = align256(off + ns * G * sizeof(float));
     L.n = off;    off = align256(off + ns * G * D * D * sizeof(float));
     L.sin = off;  off = align256(off + ns * G * D * D * sizeof(float));
+    L.need = off;
+    const bool split = bf::gdn_out_split(L.max_chunks, G, R, D, in_dtype);
+    L.spl = split ? off : 0;
+    if (split) off = align256(off + 2 * bf::gdn_plane_elems(L.max_chunks, G, D));
     L.total = off;
     return L;
 }
@@ -150,7 +154,7 @@ int gdn_fwd(const void* q, const void* k, const void* v, const float* g, const f
     if (!cu_seqlens && total_tokens % num_seqs) return BF_STATUS_INVALID;
     if (total_tokens > 0 && (!q || !k || !v || !g || !beta || !o)) return BF_STATUS_INVALID;
     const GdnLayout L = gdn_layout(total_tokens, num_seqs, G, R, D, in_dtype, segment_chunks);
-    if (!workspace || workspace_bytes < L.total) return BF_STATUS_WORKSPACE;
+    if (!workspace || workspace_bytes < L.need) return BF_STATUS_WORKSPACE;
     bf::GdnArgs a{};
     a.q = q; a.k = k; a.v = v; a.g = g; a.beta = beta;
     a.cu_seqlens = cu_seqlens;
@@ -174,6 +178,10 @@ int gdn_fwd(const void* q, const void* k, const void* v, const float* g, const f
     a.ws_c = reinterpret_cast<float*>(ws + L.c);
     a.ws_n = reinterpret_cast<float*>(ws + L.n);
     a.ws_sin = reinterpret_cast<float*>(ws + L.sin);
+    if (L.spl && workspace_bytes >= L.total) {               // a smaller workspace leaves the outputs in the scan
+        a.ws_spl = reinterpret_cast<uint16_t*>(ws + L.spl);
+        a.ws_vpl = a.ws_spl + (size_t)L.max_chunks * G * (D / 16) * (D / 32) * 1536;
+    }
     a.gn_z = gn_z; a.gn_w = gn_w; a.gn_eps = gn_eps;
     if (total_tokens == 0 && !final_state) return BF_STATUS_OK;
     const hipStream_t st = static_cast<hipStream_t>(stream);

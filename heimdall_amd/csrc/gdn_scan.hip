@@ -123,6 +123,19 @@ __device__ __forceinline__ long psi_frag_index(int d, int j) {
     return ((long)((d >> 4) * NKD + j / KF) * 64 + lane) * VEC + j % VEC;
 }
 
+// Planes of a 16-column strip as B operands of bf16 MFMAs (gdn_out_kernel): K step s covers rows 32 s .. 32 s + 31, plane p
+// of the step is 64 lanes x 8 elements, and position 8 lg + j of a step is row 4 lg + j (j < 4) or 12 + 4 lg + j: the
+// accumulators of the step's two 16-row tiles, as they lie in a lane. NT tiles, times f.
+template <int NT>
+__device__ __forceinline__ void put_planes(uint16_t* dst, const f32x4 (&x)[NT][NJ], float f, int lane) {
+#pragma unroll
+    for (int s = 0; s < NT / 2; ++s) {
+        const Planes pl = split8(x[2 * s][0] * f, x[2 * s + 1][0] * f);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) st16(dst + ((s * 3 + p) * 64 + lane) * 8, pl.p[p]);
+    }
+}
+
 // N and the segment entry states (fp32 D x D) are stored in accumulator-fragment order: element (d, j) sits in the
 // 16 x 16 tile (d / 16, j / 16) at lane 16 * ((d % 16) / 4) + j % 16, element d % 4, so the combine kernel reads and
 // writes each tile of a 16-column strip as one contiguous float4 per lane.
@@ -253,7 +266,9 @@ __device__ __forceinline__ constexpr int tpart(int tile) {
 
 // GN (output scan, bf16, whole rows per workgroup): each o row goes through the GatedNorm of the native layer before
 // it is stored, with the arithmetic of gated_norm_kernel (gdn_layer.hip), so the bits equal the two separate passes.
-template <class E, int D, bool OUT, bool BO, bool GN = false>
+// ST (fp32 output scan): instead of the query heads' outputs, every chunk's entry state and v_new go to ws_spl / ws_vpl as
+// planes. A lane's accumulators of two consecutive tiles are eight consecutive positions of a plane_frag fragment.
+template <class E, int D, bool OUT, bool BO, bool GN = false, bool ST = false>
 __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(GdnArgs a) {
     using T = typename E::T;
     using Cfg = SegCfg<E, D, OUT>;
@@ -264,7 +279,8 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
     constexpr bool DBUF = Cfg::DBUF, TPS = Cfg::TPS;
     constexpr bool QL = OUT && DBUF;                     // q staged in LDS, two buffers (bf16); fp32 reads it from global
     constexpr int VW = NW * WCOLS, VROWB = VW * ES;      // V tile: the workgroup's columns
-    constexpr int NFR = OUT ? attn_frags<E>() : 0;       // nonzero attn fragments of one query head
+    static_assert(!ST || (OUT && ES == 4 && NJ == 1), "the state pass is an fp32 output scan");
+    constexpr int NFR = OUT && !ST ? attn_frags<E>() : 0;       // nonzero attn fragments of one query head
     using CL = ChunkLds<E, D, TPS>;
     using OL = OnceLds<E, D, QL ? 2 : 0, VW, NFR * 64 * VEC, !TPS>;
     __shared__ CL cl0;
@@ -678,7 +694,11 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
         // writes are ordered by the barrier that starts head 0, which saves that head its own barrier)
         f32x4 Y[NTC][NJ];
         times_s([&](int ks, int tt) { return lds16(Kb, kq_off(ks, tpart<E>(tt))); }, Y);
-        if constexpr (OUT) {
+        if constexpr (ST) {
+            const long pb = ((long)(sg.cid0 + c) * G + g) * (D / 16) + jc / 16;
+            put_planes<NTD>(a.ws_spl + pb * (D / 32) * 1536, S, sc, lane);
+        }
+        if constexpr (OUT && !ST) {
             const char* Q0b = reinterpret_cast<const char*>(ol.Q[QL ? qb : 0]);
             const rsrc_t rq0 = make_rsrc(reinterpret_cast<const char*>(a.q) + (chunk_tok0(c) * H + (long)g * R) * D * ES,
                                          (uint32_t)(QL ? 0 : (long)chunk_len(c) * H * D * ES));
@@ -723,8 +743,13 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
             }
         }
 
+        if constexpr (ST) {
+            const long pb = ((long)(sg.cid0 + c) * G + g) * (D / 16) + jc / 16;
+            put_planes<NTC>(a.ws_vpl + pb * 2 * 1536, Vn, 1.f, lane);
+        }
+
         // phase 3, per query head r: o_r = scale e^{gc} (q_r S) + attn_r v_new
-        if constexpr (OUT) {
+        if constexpr (OUT && !ST) {
             const long t0 = chunk_tok0(c);
             const int len = chunk_len(c);
             char* Atb = reinterpret_cast<char*>(ol.At);
@@ -1158,6 +1183,169 @@ __attribute__((amdgpu_waves_per_eu(combine_waves<D>() / 4, combine_waves<D>() / 
     if (a.num_seqs < 0) a.ws_c[0] = __uint_as_float(tsink);      // keeps the touches; never taken
 }
 
+// ------------------------------------------------------------------------------------------------ fp32 outputs
+// o_r = scale e^{gc} (q_r S) + attn_r v_new, attn_r = scale (q_r K^T e^{gc_i - gc_j})[i >= j], for the R query heads of one
+// (chunk, KV head, group of 16 NW columns), from the chunk's entry state S and v_new (gdn_seg_kernel, ST). In the scan the
+// heads' products sat in the segment's chain of chunks and ran on the fp32 MFMA, each wave reading all of q from L2; here
+// every chunk is independent and the products are bf16 MFMAs over exact planes (Planes, bf_common.h). A wave holds the
+// planes of its 16 columns of S and v_new in registers for all heads. K's planes stay in LDS; q's go through a double-
+// buffered 64 x 32 slice, stored a slice ahead of the MFMAs and loaded two ahead, one barrier per slice. The ten causal
+// 16 x 16 tiles of attn^T = K q_r^T are shared out over the waves beside their q_r S products, masked, decayed and written
+// to LDS as planes. Positions 8 q + j of every 32-wide step are those of put_planes.
+template <int D>
+constexpr int out_waves() { return D < 128 ? D / 16 : 8; }
+
+template <int D, bool BO>
+__global__ __launch_bounds__(64 * out_waves<D>()) void gdn_out_kernel(GdnArgs a) {
+    constexpr int NW = out_waves<D>(), NT = 64 * NW, NCG = D / (16 * NW), NKS = D / 32, NTA = (10 + NW - 1) / NW;
+    constexpr int NQ = SC * 8 / NT;                      // 16-byte pieces of a q slice per thread
+    __shared__ __align__(16) uint16_t kp[3][SC][D + 8];
+    __shared__ __align__(16) uint16_t qs[2][3][SC][32 + 8];
+    __shared__ __align__(16) uint16_t at[3][SC][SC + 8];
+    __shared__ __align__(16) float gc[SC], eg[SC];
+    const int G = a.G, R = a.R, H = G * R;
+    const int xcd = blockIdx.x % NXCD, local = blockIdx.x / NXCD;
+    const long item = xcd + (long)NXCD * (local / NCG);
+    const int cg = local % NCG;
+    if (item >= (long)a.max_chunks * G) return;
+    const int g = (int)(item % G), cid = (int)(item / G);
+    SeqInfo si;
+    if (!locate_chunk(cid, a.cu_seqlens, a.num_seqs, a.seq_len, SC, si)) return;
+    const int tid = threadIdx.x, lane = lane_id(), wv = wave_id(), l16 = lane & 15, lg = lane >> 4;
+    const int jt = cg * NW + wv;                         // column tile of this wave
+
+    // q slice it = (head, 32-wide step), rows past the chunk's end read as zero
+    const float* qg = reinterpret_cast<const float*>(a.q) + (si.tok0 * H + (long)g * R) * D;
+    const rsrc_t rq = make_rsrc(qg, (uint32_t)((((long)si.len - 1) * H + R) * D * 4));
+    const int slices = R * NKS;
+    f32x4 x[NQ];
+    auto load_q = [&](int it) {
+        const uint32_t so = (uint32_t)(min(it, slices - 1) * 128);       // (r, ks): r D + 32 ks elements
+#pragma unroll
+        for (int h = 0; h < NQ; ++h) {
+            const int row = tid / 8 + NT / 8 * h;
+            x[h] = __builtin_bit_cast(f32x4, buf_ld16(rq, row < si.len ? (uint32_t)(row * H * D + 4 * (tid % 8)) * 4u + so
+                                                                       : 0xFFFFFFF0u));
+        }
+    };
+    const int pos = 8 * (tid % 4) + 4 * (tid % 8 / 4);                   // position of this thread's piece of a step
+    auto put = [](uint16_t* dst, long plane, const f32x4& v) {
+        uint2 s[3];
+        split_pair(v[0], v[1], s[0].x, s[1].x, s[2].x);
+        split_pair(v[2], v[3], s[0].y, s[1].y, s[2].y);
+#pragma unroll
+        for (int p = 0; p < 3; ++p) *reinterpret_cast<uint2*>(dst + p * plane) = s[p];
+    };
+    auto store_q = [&](int buf) {
+#pragma unroll
+        for (int h = 0; h < NQ; ++h) put(&qs[buf][0][tid / 8 + NT / 8 * h][pos], SC * 40, x[h]);
+    };
+
+    load_q(0);
+    // this wave's planes of S and v_new
+    Planes fs[NKS], fv[2];
+    {
+        const long pb = ((long)cid * G + g) * (D / 16) + jt;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) fs[ks].p[p] = ld16(a.ws_spl + (pb * NKS * 3 + ks * 3 + p) * 512 + lane * 8);
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+            for (int p = 0; p < 3; ++p) fv[ks].p[p] = ld16(a.ws_vpl + (pb * 6 + ks * 3 + p) * 512 + lane * 8);
+    }
+    {
+        const rsrc_t rk = make_rsrc(reinterpret_cast<const float*>(a.k) + (si.tok0 * G + g) * D,
+                                    (uint32_t)((((long)si.len - 1) * G + 1) * D * 4));
+        constexpr int PC = D / 4;                        // pieces per row
+#pragma unroll 4
+        for (int c = tid; c < SC * PC; c += NT) {
+            const int row = c / PC, s = c % PC;
+            const f32x4 v = __builtin_bit_cast(f32x4, buf_ld16(rk, row < si.len ? (uint32_t)(row * G * D + 4 * s) * 4u
+                                                                               : 0xFFFFFFF0u));
+            put(&kp[0][row][32 * (s / 8) + 8 * (s % 4) + 4 * (s % 8 / 4)], SC * (D + 8), v);
+        }
+    }
+    for (int i = tid; i < 3 * SC * (SC + 8) / 8; i += NT) st16(&at[0][0][0] + 8 * i, zero16());   // tiles above the diagonal
+    if (tid < SC) {
+        gc[tid] = a.ws_gcum[((long)cid * G + g) * SC + tid];
+        eg[tid] = a.scale * __expf(gc[tid]);
+    }
+    store_q(0);
+    load_q(1);
+    __syncthreads();
+
+    auto frag = [&](const uint16_t* t, long plane, int pitch, int row, int col) {
+        Planes f;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) f.p[p] = ld16(t + p * plane + row * pitch + col);
+        return f;
+    };
+    for (int r = 0; r < R; ++r) {
+        f32x4 acc[4], aacc[NTA];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) acc[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int n = 0; n < NTA; ++n) aacc[n] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // tile n of this wave: f = wv + NW n in the order (0,0), (1,0), (1,1), (2,0), .. of (query tile, key tile)
+        auto tile = [&](int n, int& qi, int& ki) {
+            const int f = wv + NW * n;
+            qi = f < 1 ? 0 : f < 3 ? 1 : f < 6 ? 2 : 3;
+            ki = f - qi * (qi + 1) / 2;
+            return f < 10;
+        };
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const uint16_t* qb = &qs[ks & 1][0][0][0];
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) mma3(acc[tt], frag(qb, SC * 40, 40, 16 * tt + l16, 8 * lg), fs[ks]);
+#pragma unroll
+            for (int n = 0; n < NTA; ++n) {
+                int qi, ki;
+                if (tile(n, qi, ki))
+                    mma3(aacc[n], frag(&kp[0][0][0], SC * (D + 8), D + 8, 16 * ki + l16, 32 * ks + 8 * lg),
+                         frag(qb, SC * 40, 40, 16 * qi + l16, 8 * lg));
+            }
+            store_q((ks & 1) ^ 1);                       // the next slice; past the last one, that one again
+            load_q(r * NKS + ks + 2);
+            lds_barrier();
+        }
+#pragma unroll
+        for (int n = 0; n < NTA; ++n) {
+            int qi, ki;
+            if (tile(n, qi, ki)) {                       // lane: query 16 qi + l16, keys 16 ki + 4 lg + e
+                const int i = 16 * qi + l16, j0 = 16 * ki + 4 * lg;
+                const float gi = gc[i];
+                f32x4 m;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) m[e] = j0 + e <= i ? a.scale * __expf(gi - gc[j0 + e]) * aacc[n][e] : 0.f;
+                put(&at[0][i][32 * (ki / 2) + 8 * lg + 4 * (ki & 1)], SC * (SC + 8), m);
+            }
+        }
+        lds_barrier();
+        // (the next head writes attn after further barriers, past every wave's reads here)
+        const rsrc_t ro = make_rsrc(reinterpret_cast<char*>(a.o) + (si.tok0 * H + (long)g * R + r) * D * (BO ? 2 : 4),
+                                    (uint32_t)((((long)si.len - 1) * H + 1) * D * (BO ? 2 : 4)));
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            const float4 e4 = *reinterpret_cast<const float4*>(&eg[16 * tt + 4 * lg]);
+            acc[tt][0] *= e4.x; acc[tt][1] *= e4.y; acc[tt][2] *= e4.z; acc[tt][3] *= e4.w;
+#pragma unroll
+            for (int ks = 0; ks < (tt < 2 ? 1 : 2); ++ks)
+                mma3(acc[tt], frag(&at[0][0][0], SC * (SC + 8), SC + 8, 16 * tt + l16, 32 * ks + 8 * lg), fv[ks]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int row = 16 * tt + 4 * lg + e;
+                // rows past the chunk's end get an offset past the descriptor's range and are dropped
+                const uint32_t el = (uint32_t)(row * H * D + 16 * jt + l16);
+                if constexpr (BO) buf_sth(ro, row < si.len ? 2u * el : 0xFFFFFFF0u, f2bf(acc[tt][e]));
+                else buf_stf(ro, row < si.len ? 4u * el : 0xFFFFFFF0u, acc[tt][e]);
+            }
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ host launchers
 namespace {
 
@@ -1195,6 +1383,19 @@ int launch_output(const GdnArgs& a, hipStream_t stream) {
             return (int)hipGetLastError();
         } else {
             return BF_ERR_UNSUPPORTED;
+        }
+    }
+    if constexpr (std::is_same<E, F32>::value) {
+        if (a.ws_spl) {
+            hipLaunchKernelGGL((gdn_seg_kernel<E, D, true, false, false, true>), grid, block, 0, stream, a);
+            const hipError_t e = hipGetLastError();
+            if (e != hipSuccess) return (int)e;
+            constexpr int NW = out_waves<D>(), NCG = D / (16 * NW);
+            const long items = (long)a.max_chunks * a.G;
+            const dim3 og((unsigned)(NXCD * ((items + NXCD - 1) / NXCD) * NCG));
+            if (a.o_dtype == DT_BF16) hipLaunchKernelGGL((gdn_out_kernel<D, true>), og, dim3(64 * NW), 0, stream, a);
+            else hipLaunchKernelGGL((gdn_out_kernel<D, false>), og, dim3(64 * NW), 0, stream, a);
+            return (int)hipGetLastError();
         }
     }
     if (a.o_dtype == DT_BF16)

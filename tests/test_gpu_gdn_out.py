@@ -1,0 +1,56 @@
+"""fp32 outputs of several query heads per KV head (the pass over all chunks after the scan), against the recurrence in 64 bits.
+
+Chunk tails of 1 and 63 tokens, one chunk, several segments, packed sequences (one of them empty), every head dim, head counts
+that are not a power of two, an initial state, and bf16 outputs. Tolerance: operands carry their 24 bits and sums are fp32 over
+at most 2 D + 64 terms per chunk and a state carried in fp32, as in the scan: 2e-6 (bf16 outputs: their rounding, 2^-9, and a
+margin of two).
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+def recurrence(q, k, v, g, beta, s):
+    """One sequence in 64 bits: q [T, G, R, D], k, v [T, G, D], g, beta [T, G], s [G, D, D]."""
+    o = torch.empty(q.shape, dtype=torch.float64)
+    for t in range(q.shape[0]):
+        s = s * g[t].exp()[:, None, None]
+        new = (v[t] - (k[t][:, None] @ s)[:, 0]) * beta[t][:, None]
+        s = s + k[t][:, :, None] * new[:, None]
+        o[t] = q[t] @ s
+    return o, s
+
+
+@pytest.mark.parametrize("lens,G,R,D,s0,out_dtype", [
+    ([1], 1, 2, 64, False, torch.float32),
+    ([64], 2, 3, 128, True, torch.float32),
+    ([129], 2, 6, 256, False, torch.float32),
+    ([63, 0, 200, 65], 3, 2, 64, True, torch.float32),
+    ([300, 31], 1, 5, 256, True, torch.float32),
+    ([100], 5, 4, 128, False, torch.bfloat16),
+])
+def test_fp32_outputs(dev, lens, G, R, D, s0, out_dtype):
+    from heimdall_amd._device import gdn_forward
+    gen = torch.Generator().manual_seed(sum(lens) + D)
+    N, B = sum(lens), len(lens)
+    print(f"fp32 outputs lens={lens} G={G} R={R} D={D}", flush=True)
+    q, k = torch.randn(N, G, R, D, generator=gen), F.normalize(torch.randn(N, G, D, generator=gen), dim=-1)
+    v, g = torch.randn(N, G, D, generator=gen), -0.05 * torch.rand(N, G, generator=gen)
+    beta, s = torch.sigmoid(torch.randn(N, G, generator=gen)), torch.randn(B, G, D, D, generator=gen) if s0 else None
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    to = lambda x: x.to(dev)
+    for seg in (0, 1):                                    # 1: a segment per chunk, through the summary and combine passes
+        o, sf = gdn_forward(to(q.reshape(N, G * R, D)), to(k), to(v), to(g), to(beta), num_seqs=B, cu_seqlens=to(cu),
+                            initial_state=None if s is None else to(s), out_dtype=out_dtype, segment_chunks=seg)
+        tol = 2e-6 if out_dtype == torch.float32 else 2 ** -8
+        for i in range(B):
+            a, e = int(cu[i]), int(cu[i + 1])
+            zero = torch.zeros(G, D, D, dtype=torch.float64)
+            ro, rs = recurrence(*(x[a:e].double() for x in (q, k, v, g, beta)), zero if s is None else s[i].double())
+            if e > a:
+                err = (o[a:e].cpu().double().reshape(ro.shape) - ro).norm() / ro.norm()
+                assert err < tol, (seg, i, err)
+            if rs.norm() > 0:
+                assert (sf[i].cpu().double() - rs).norm() / rs.norm() < 2e-6, (seg, i)
