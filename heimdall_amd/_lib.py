@@ -37,6 +37,8 @@ SIGNATURES = {
     "bf_prefix_attention": (_c_int, [_c_int] * 6 + [_c_i64, _c_int, _vp] + [_c_i64] * 3 + [_vp] * 4
                             + [_c_int, _vp, _c_sz, _vp]),
     "bf_mem_project": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_i64, _c_i64, _vp, _fp, _vp, _c_int, _c_int, _vp]),
+    "bf_mem_project_f32_workspace_size": (_c_int, [_c_int, _c_int, ctypes.POINTER(_c_sz)]),
+    "bf_mem_project_f32": (_c_int, [_vp, _c_i64, _c_int, _c_int, _c_i64, _c_i64, _vp, _fp, _vp, _vp, _c_sz, _vp]),
     "bf_mem_gates": (_c_int, [_vp, _c_i64, _c_i64, _c_int, _c_i64, _vp, _vp, _vp, _c_i64, _c_int, _vp, _vp, _vp]),
     "bf_gate_project_workspace_size": (_c_int, [_c_i64, _c_int, _c_int, ctypes.POINTER(_c_sz)]),
     "bf_gate_project": (_c_int, [_vp, _c_i64, _c_int, _c_i64, _vp, _vp, _c_int, _vp, _vp, _vp, _c_int, _vp, _vp,

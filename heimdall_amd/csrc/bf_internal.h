@@ -338,6 +338,9 @@ inline size_t gate_project_workspace(long n_tok, int d, int nout) {
 }
 int gate_project_dispatch(const GateProjArgs& a, hipStream_t stream);
 int mem_project_dispatch(const MemProjArgs& a, hipStream_t stream);
+// fp32 rows: f's planes go to `planes` (mem_project32_bytes) first
+inline size_t mem_project32_bytes(int nh, int D) { return (size_t)nh * D * D * 6; }
+int mem_project32_dispatch(const MemProjArgs& a, uint16_t* planes, hipStream_t stream);
 
 // The memory inputs of a few tokens (student_front). Above FRONT_MAX_TOK the tiled kernels are the faster ones.
 constexpr long FRONT_MAX_TOK = 256;

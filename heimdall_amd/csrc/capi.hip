@@ -582,6 +582,28 @@ int bf_mem_project(const void* x, int64_t n_tok, int nh, int D, int64_t x_st, in
     return bf::mem_project_dispatch(a, static_cast<hipStream_t>(stream));
 }
 
+int bf_mem_project_f32_workspace_size(int nh, int D, size_t* bytes) {
+    if (!bytes || nh <= 0 || nh > 65535) return BF_STATUS_INVALID;
+    if (!supported_dim(D)) return BF_STATUS_UNSUPPORTED;
+    *bytes = bf::mem_project32_bytes(nh, D);
+    return BF_STATUS_OK;
+}
+
+int bf_mem_project_f32(const float* x, int64_t n_tok, int nh, int D, int64_t x_st, int64_t x_sh, const float* f, float scale,
+                       float* out, void* workspace, size_t workspace_bytes, void* stream) {
+    size_t need = 0;
+    const int st = bf_mem_project_f32_workspace_size(nh, D, &need);
+    if (st) return st;
+    if (n_tok < 0 || x_st <= 0 || x_sh < 0 || x_st % 4 || x_sh % 4) return BF_STATUS_INVALID;
+    if (n_tok == 0) return BF_STATUS_OK;
+    if (!x || !f || !out || ((uintptr_t)x & 15) || ((uintptr_t)out & 15) || ((uintptr_t)workspace & 15)) return BF_STATUS_INVALID;
+    if (!workspace || workspace_bytes < need) return BF_STATUS_WORKSPACE;
+    bf::MemProjArgs a{};
+    a.x = x; a.n_tok = n_tok; a.nh = nh; a.D = D; a.x_st = x_st; a.x_sh = x_sh;
+    a.f = f; a.scale = scale; a.out = out; a.out_dtype = BF_DTYPE_F32;
+    return bf::mem_project32_dispatch(a, static_cast<uint16_t*>(workspace), static_cast<hipStream_t>(stream));
+}
+
 int bf_mem_gates(const float* ab, int64_t n_tok, int64_t T, int G, int64_t ab_st, const float* A_log,
                  const float* dt_bias, const float* decay_mask, int64_t start, int sinks, float* g, float* beta,
                  void* stream) {

@@ -594,4 +594,145 @@ int student_front(FrontArgs& a, bool finish, hipStream_t stream) {
     }
 }
 
+// ------------------------------------------------------------------------------------------------ fp32 projection
+// out[t][h] = normalize(x[t][h] F_h) * scale for fp32 rows on bf16 MFMAs over exact planes (Planes, bf_common.h), in two
+// launches. The first writes F's planes as B operands: fragment (head, 16 columns, 32 rows, plane) is 64 lanes x 8
+// elements, position 8 lg + j being row 4 lg + j (j < 4) or 12 + 4 lg + j. The second takes 64 tokens of one head: their
+// planes in LDS, a wave's columns over all of D with F's fragments read one step ahead from L2 (a head's 393 KB at D = 256
+// are read by all its tiles, which neighbour each other on an XCD), the norm over the waves through LDS, and whole rows
+// out. As a transposing copy, an fp32 library product per head, a copy back, a norm and three elementwise passes the
+// q and k projections of 4096 tokens, H = 16, G = 4, D = 256 took 270 us; in these launches 117.
+template <int D>
+__global__ __launch_bounds__(2 * D) void mem_planes_kernel(const float* f, uint16_t* planes) {
+    constexpr int NKS = D / 32;
+    const int ct = blockIdx.x, h = blockIdx.y, lane = lane_id(), ks = wave_id(), l16 = lane & 15, lg = lane >> 4;
+    const float* p = f + ((long)h * D + 32 * ks + 4 * lg) * D + 16 * ct + l16;
+    f32x4 a, b;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        a[j] = p[j * D];
+        b[j] = p[(16 + j) * D];
+    }
+    const Planes s = split8(a, b);
+    uint16_t* dst = planes + ((((long)h * (D / 16) + ct) * NKS + ks) * 3 * 64 + lane) * 8;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) st16(dst + i * 512, s.p[i]);
+}
+
+template <int D>
+constexpr int proj32_waves() { return D < 128 ? D / 16 : 8; }
+
+template <int D>
+__global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(MemProjArgs a, const uint16_t* planes) {
+    constexpr int NW = proj32_waves<D>(), NT = 64 * NW, CT = D / (16 * NW), NKS = D / 32, TOK = 64;
+    constexpr int XP = TOK * (D + 8), PC = D / 4;        // elements of a plane, 16-byte pieces of a row
+    __shared__ __align__(16) char lds[3 * XP * 2];       // the rows' planes, then the output rows [TOK][D + 4] fp32
+    __shared__ float part[NW][TOK];
+    static_assert(TOK * (D + 4) * 4 <= 3 * XP * 2, "output rows");
+    uint16_t* xs = reinterpret_cast<uint16_t*>(lds);
+    const long tiles = (a.n_tok + TOK - 1) / TOK, items = tiles * a.nh, per = (items + 7) / 8;
+    const long item = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per || item >= items) return;
+    const int h = (int)(item / tiles);
+    const long t0 = item % tiles * TOK;
+    const int n = (int)min((long)TOK, a.n_tok - t0);
+    const int tid = threadIdx.x, lane = lane_id(), wv = wave_id(), l16 = lane & 15, lg = lane >> 4;
+
+    const float* x = reinterpret_cast<const float*>(a.x) + t0 * a.x_st + h * a.x_sh;
+#pragma unroll 4
+    for (int c = tid; c < TOK * PC; c += NT) {
+        const int row = c / PC, s = c % PC;              // rows past the last token: the last one again (not stored)
+        const f32x4 v = *reinterpret_cast<const f32x4*>(x + min(row, n - 1) * a.x_st + 4 * s);
+        uint2 p[3];
+        split_pair(v[0], v[1], p[0].x, p[1].x, p[2].x);
+        split_pair(v[2], v[3], p[0].y, p[1].y, p[2].y);
+        uint16_t* dst = xs + row * (D + 8) + 32 * (s / 8) + 8 * (s % 4) + 4 * (s % 8 / 4);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(dst + i * XP) = p[i];
+    }
+    const uint16_t* fp = planes + ((long)h * (D / 16) + wv * CT) * NKS * 1536 + lane * 8;
+    auto read_f = [&](int ks, Planes (&f)[CT]) {
+#pragma unroll
+        for (int c = 0; c < CT; ++c)
+#pragma unroll
+            for (int i = 0; i < 3; ++i) f[c].p[i] = ld16(fp + ((long)(c * NKS + ks) * 3 + i) * 512);
+    };
+    f32x4 acc[4][CT];
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[tt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    Planes f[2][CT];
+    read_f(0, f[0]);
+    __syncthreads();
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) {
+        read_f(min(ks + 1, NKS - 1), f[(ks + 1) & 1]);
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            Planes ax;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) ax.p[i] = ld16(xs + i * XP + (16 * tt + l16) * (D + 8) + 32 * ks + 8 * lg);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) mma3(acc[tt][c], ax, f[ks & 1][c]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // row norms: this wave's columns (lanes of equal lg), then the waves
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            float ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < CT; ++c) ss += acc[tt][c][e] * acc[tt][c][e];
+#pragma unroll
+            for (int m = 1; m < 16; m <<= 1) ss += __shfl_xor(ss, m);
+            if (l16 == 0) part[wv][16 * tt + 4 * lg + e] = ss;
+        }
+    __syncthreads();                                     // also: every wave is done with the planes
+    float* os = reinterpret_cast<float*>(lds);
+#pragma unroll
+    for (int tt = 0; tt < 4; ++tt)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int row = 16 * tt + 4 * lg + e;
+            float ss = 0.f;
+#pragma unroll
+            for (int w = 0; w < NW; ++w) ss += part[w][row];
+            const float nrm = fmaxf(sqrtf(ss), 1e-12f);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) os[row * (D + 4) + 16 * (wv * CT + c) + l16] = acc[tt][c][e] / nrm * a.scale;
+        }
+    __syncthreads();
+    float* out = reinterpret_cast<float*>(a.out) + (t0 * a.nh + h) * D;
+#pragma unroll 4
+    for (int c = tid; c < n * PC; c += NT) {
+        const int row = c / PC, s = c % PC;
+        st16(out + (long)row * a.nh * D + 4 * s, ld16(os + row * (D + 4) + 4 * s));
+    }
+}
+
+namespace {
+template <int D>
+int launch_project32(const MemProjArgs& a, uint16_t* planes, hipStream_t stream) {
+    hipLaunchKernelGGL((mem_planes_kernel<D>), dim3(D / 16, a.nh), dim3(2 * D), 0, stream, static_cast<const float*>(a.f), planes);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return (int)e;
+    const long per = ((a.n_tok + 63) / 64 * a.nh + 7) / 8;
+    if (8 * per > 0x7fffffffL || a.nh > 65535) return BF_STATUS_INVALID;
+    hipLaunchKernelGGL((mem_project32_kernel<D>), dim3((unsigned)(8 * per)), dim3(64 * proj32_waves<D>()), 0, stream, a, planes);
+    return (int)hipGetLastError();
+}
+}  // namespace
+
+int mem_project32_dispatch(const MemProjArgs& a, uint16_t* planes, hipStream_t stream) {
+    switch (a.D) {
+        case 64: return launch_project32<64>(a, planes, stream);
+        case 128: return launch_project32<128>(a, planes, stream);
+        case 256: return launch_project32<256>(a, planes, stream);
+        default: return BF_ERR_UNSUPPORTED;
+    }
+}
+
 }  // namespace bf

@@ -9,7 +9,7 @@ the same shapes and meaning, mutated in place), so a cache can move between the 
 The window + sink attention, the delta-rule memory and the gamma mix run in ``libbifrost_hip.so``:
   t == 1  -> ``bf_decode_fwd`` (one bandwidth-bound pass: state update, window read, mix, ring write)
   t > 1   -> ``bf_gdn_fwd`` (memory branch) then ``bf_window_fwd`` (window + sinks + LSE, fused gamma mix)
-The frozen projections and the small per-token gate GEMMs (fq/fk, ab, mix) stay in PyTorch.
+The gate GEMMs (ab, mix) of fp32 activations, and everything that autograd records, stay in PyTorch.
 
 ``student`` can be bound onto the reference class as a drop-in: ``HybridAttention._student = student``; likewise the
 teacher path of the kept full-attention layers, ``HybridAttention._teacher = teacher`` and ``set_retrieval``
@@ -52,12 +52,41 @@ def _heads_matmul(x: torch.Tensor, f: torch.Tensor) -> torch.Tensor:
     return y.reshape(h, b, t, d).permute(1, 2, 0, 3)
 
 
+def _project_f32(x: torch.Tensor, f: torch.Tensor, scale: float) -> torch.Tensor:
+    """fp32 x [b, t, h, D] -> normalize(x_h f_h) * scale per head: bf_mem_project_f32 on the GPU where nothing is recorded or
+    transformed, PyTorch operators otherwise. Below 64 tokens a tile of the kernel would be mostly empty and its first
+    pass over f is most of the work."""
+    b, t, h, d = x.shape
+    if (not x.is_cuda or b * t < 64 or d not in (64, 128, 256) or f.shape != (h, d, d) or f.device != x.device
+            or (torch.is_grad_enabled() and (x.requires_grad or f.requires_grad)) or _transformed(x, f)):
+        return F.normalize(_heads_matmul(x, f), dim=-1) * scale
+    if (x.stride(-1) != 1 or (b > 1 and x.stride(0) != t * x.stride(1)) or x.stride(1) % 4 or x.stride(2) % 4
+            or min(x.stride(1), x.stride(2)) < 1 or x.data_ptr() % 16):
+        x = x.clone(memory_format=torch.contiguous_format)       # (a dense but misaligned x too)
+    f = _f32(f)
+    out = torch.empty(b, t, h, d, dtype=torch.float32, device=x.device)
+    lib, nb = _lib.load(), _lib.ctypes.c_size_t(0)
+    check(lib.bf_mem_project_f32_workspace_size(h, d, _lib.ctypes.byref(nb)), "bf_mem_project_f32_workspace_size")
+    ws = workspace(nb.value, x.device)
+    check(lib.bf_mem_project_f32(x.data_ptr(), b * t, h, d, x.stride(1), x.stride(2), f.data_ptr(), float(scale),
+                                 out.data_ptr(), ws.data_ptr(), nb.value, stream_ptr(x.device)), "bf_mem_project_f32")
+    return out
+
+
+def _transformed(*tensors) -> bool:
+    """Tensors that a kernel cannot read as they are: traced, subclasses (fake tensors), under vmap or another function
+    transform, or dual in forward mode."""
+    fwd = torch.autograd.forward_ad
+    return (torch.jit.is_tracing() or any(type(t) not in (torch.Tensor, nn.Parameter) for t in tensors)
+            or any(torch._C._functorch.is_functorch_wrapped_tensor(t) for t in tensors)
+            or (fwd._current_level >= 0 and any(fwd.unpack_dual(t).tangent is not None for t in tensors)))
+
+
 def mem_inputs(self, x, q, k, pos):
     """qm = normalize(q_h F_q,h) / sqrt(D); km = normalize(k_g F_k,g); g = -exp(A_log) softplus(a + dt_bias) mask;
     beta = sigmoid(b) [pos >= sinks]  (``hibrit.py:327-334``), all fp32."""
     dh = self.c.dh
-    qm = F.normalize(_heads_matmul(q.float(), self.fq), dim=-1) * dh ** -0.5
-    km = F.normalize(_heads_matmul(k.float(), self.fk), dim=-1)
+    qm, km = _project_f32(q.float(), self.fq, dh ** -0.5), _project_f32(k.float(), self.fk, 1.0)
     a, bb = F.linear(x.float(), self.ab.weight.float(), self.ab.bias.float()).chunk(2, dim=-1)
     g = -self.A_log.float().exp() * F.softplus(a + self.dt_bias.float()) * self.decay_mask.float()
     beta = torch.sigmoid(bb) * (pos >= self.sinks).float()[None, :, None]

@@ -248,6 +248,14 @@ int bf_mem_project(const void* x, int64_t n_tok, int nh, int D, int64_t x_st, in
                    float scale, void* out, int in_dtype, int out_dtype, void* stream);
 
 /*
+ * The same for fp32 rows, with no operand rounded: x, f, out fp32 (x and out 16-byte aligned, x_st and x_sh multiples of 4).
+ * Workspace: bf_mem_project_f32_workspace_size bytes, 16-byte aligned.
+ */
+int bf_mem_project_f32_workspace_size(int nh, int D, size_t* bytes);
+int bf_mem_project_f32(const float* x, int64_t n_tok, int nh, int D, int64_t x_st, int64_t x_sh, const float* f, float scale,
+                       float* out, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * Memory-branch gates of the converted layer, replacing the gate lines of HybridAttention._mem_inputs
  * (Heimdall/heimdall/hibrit.py:331-333):
  *     g[i][j]    = -exp(A_log[j]) * softplus(ab[i][j] + dt_bias[j]) * decay_mask[j]     (softplus threshold 20)
