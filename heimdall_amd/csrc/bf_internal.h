@@ -398,7 +398,7 @@ struct GdnBwdArgs {
     // outputs (same layouts); ds0 may be null
     float *dq, *dk, *dv, *dg, *dbeta, *ds0;
     // workspace, chunk-major [chunk][g][...] (cg = chunk * G + g)
-    float *gam, *eg, *dgz, *Am, *Mi, *dA, *kb, *vb, *kbe, *ktl, *ktlF, *ktlTF, *u, *w, *wF, *wTF, *attn, *dattn, *qdot, *zr, *zc, *zrA, *zcA;
+    float *gam, *eg, *dgz, *Am, *Mi, *dA, *kb, *vb, *kbe, *ktl, *ktlF, *ktlTF, *u, *wF, *wTF, *attn, *dattn, *qdot, *zr, *zc, *zrA, *zcA;
     float *Sc, *E2, *dSx, *part, *psd;
     float *E1, *dvn, *vn, *dkt, *dw, *dvb, *dkbe, *dkb, *dkacc;
 };
@@ -509,7 +509,10 @@ struct GdnStepLayerArgs {
     const void* prefix;       // [B][K - 1][C] or null (zeros)
     void* conv_out;           // [B][K - 1][C]: the last K - 1 rows of [prefix; z]
     const void* w;            // [C][K]
-    const void *a, *b;        // [B][HV]
+    const void *a, *b;        // [B][HV], or (x set) the projections' weights [HV][d]: then a = round(x w_a^T), b likewise
+    const void* x;            // [B] rows of d elements, x_st apart, io_dtype; or null
+    long x_st;
+    int d;
     const void *A_log, *dt_bias;   // [HV]
     const void* zg;           // [B][HV][D]
     const void* norm_w;       // [D]

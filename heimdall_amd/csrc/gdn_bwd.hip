@@ -493,7 +493,18 @@ __device__ __forceinline__ void walk_fwd(const GdnBwdArgs& a, int strip) {
             for (int v = 0; v < 4; ++v) VT[kh][16 * c2 + i16][16 * tq + 4 * q + v] = acc[v];
         }
         lds_barrier();
-        // S = e^(gc_C') S + kt^T v_new (v_new = the sum of the parts); the next chunk's kt^T rides along
+        // v_new (the sum of the parts) out; S = e^(gc_C') S + kt^T v_new; the next chunk's kt^T rides along
+        if (kh == 0) {
+#pragma unroll
+            for (int c2 = 0; c2 < SW; ++c2)
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    float x = VT[0][16 * c2 + i16][16 * tq + 4 * q + v];
+#pragma unroll
+                    for (int p = 1; p < KH; ++p) x += VT[p][16 * c2 + i16][16 * tq + 4 * q + v];
+                    a.vn[(cg * BC + 16 * tq + 4 * q + v) * D + col0 + 16 * c2 + i16] = x;
+                }
+        }
         const float ec = expf(cur.gl);
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
@@ -889,12 +900,12 @@ Op tr(Op o) { std::swap(o.rs, o.cs); return o; }
 constexpr int kBwdMaxDevices = 64;
 struct BwdSide {
     hipStream_t s = nullptr;
-    hipEvent_t ev[7] = {};
+    hipEvent_t ev[6] = {};
 };
 std::mutex g_bwd_mu;
 BwdSide g_bwd_side[kBwdMaxDevices];
 
-int side_stream(hipStream_t& s2, hipEvent_t (&ev)[7]) {
+int side_stream(hipStream_t& s2, hipEvent_t (&ev)[6]) {
     int dev = -1;
     hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
@@ -904,7 +915,7 @@ int side_stream(hipStream_t& s2, hipEvent_t (&ev)[7]) {
         if (!x && (e = hipEventCreateWithFlags(&x, hipEventDisableTiming)) != hipSuccess) return (int)e;
     if (!sd.s && (e = hipStreamCreateWithFlags(&sd.s, hipStreamNonBlocking)) != hipSuccess) return (int)e;
     s2 = sd.s;
-    for (int i = 0; i < 7; ++i) ev[i] = sd.ev[i];
+    for (int i = 0; i < 6; ++i) ev[i] = sd.ev[i];
     return 0;
 }
 
@@ -915,12 +926,12 @@ size_t gdn_bwd_workspace(int num_seqs, long T, int G, int R, int D) {
     const long cc = BC * BC, cd = (long)BC * D, dd = (long)D * D;
     const long floats = NC * (BC * 5 + 8                             // gam, eg, dgz, zrA, zcA, part, psd
                               + cc * 3                               // Am, M, dA
-                              + cd * 10                              // kb, vb, kbe, ktl, u, w; ktl, kt^T, w, w^T in fragment order
+                              + cd * 9                               // kb, vb, kbe, ktl, u; ktl, kt^T, w, w^T in fragment order
                               + (long)R * (cc * 2 + (D / 64 + 2) * BC)   // attn, dattn; qdot, zr, zc
                               + dd * 3                               // Sc, E2, dSx
                               + cd * 9                               // E1, dvn, vn, dkt, dw, dvb, dkbe, dkb, dkacc
                               + cc * 2);                             // dM, T1
-    return (size_t)floats * sizeof(float) + 256 * 49;                // each buffer rounded up to 256 bytes
+    return (size_t)floats * sizeof(float) + 256 * 48;                // each buffer rounded up to 256 bytes
 }
 
 int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
@@ -938,7 +949,7 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
     a.Am = take(NC * cc); a.Mi = take(NC * cc); a.dA = take(NC * cc);
     a.zrA = take(NC * BC); a.zcA = take(NC * BC); a.zr = take(NC * R * BC); a.zc = take(NC * R * BC);
     a.kb = take(NC * cd); a.vb = take(NC * cd); a.kbe = take(NC * cd); a.ktl = take(NC * cd);
-    a.u = take(NC * cd); a.w = take(NC * cd);
+    a.u = take(NC * cd);
     a.ktlF = take(NC * cd); a.ktlTF = take(NC * cd); a.wF = take(NC * cd); a.wTF = take(NC * cd);
     a.attn = take(NC * R * cc); a.dattn = take(NC * R * cc);
     a.qdot = take(NC * R * (D / 64) * BC);
@@ -963,7 +974,7 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
     const int nzg = (int)NC, nzr = (int)(NC * R);
 
     hipStream_t s2 = nullptr;
-    hipEvent_t ev[7] = {};
+    hipEvent_t ev[6] = {};
     ok(side_stream(s2, ev));
     if (e) return e;
     // prep
@@ -976,16 +987,15 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
             KSplit{}, dec));
     hipLaunchKernelGGL(unit_lower_inverse_kernel, dim3((unsigned)NC), dim3(64), 0, s, a.Am, a.Mi);
     ok((int)hipGetLastError());
-    // u = M (v b), w = M (k b e^gc)
+    // u = M (v b), w = M (k b e^gc); only the walks read w, in fragment order
     ok(gemm(BC, D, BC, nzg, G, 1, W(a.Mi, BC, BC), W(a.vb, BC, D), a.u, (long)G * cd, cd, 0, D, 1, 1.f, 0, 0, nullptr, s));
-    ok(gemm(BC, D, BC, nzg, G, 1, W(a.Mi, BC, BC), W(a.kbe, BC, D), a.w, (long)G * cd, cd, 0, D, 1, 1.f, 0, 0, nullptr, s));
     Epi fr;
     fr.frag = 1;                                          // w and w^T in fragment order for the state walks
     ok(gemm(BC, D, BC, nzg, G, 1, W(a.Mi, BC, BC), W(a.kbe, BC, D), a.wF, (long)G * cd, cd, 0, D, 1, 1.f, 0, 0, nullptr,
             s, KSplit{}, fr));
     ok(gemm(D, BC, BC, nzg, G, 1, tr(W(a.kbe, BC, D)), tr(W(a.Mi, BC, BC)), a.wTF, (long)G * cd, cd, 0, BC, 1, 1.f, 0, 0,
             nullptr, s, KSplit{}, fr));                   // w^T = (k b e^gc)^T M^T
-    // Side stream: the forward walk, then what needs only the entry states (v_new, dattn, dq). Main stream: attn, E1,
+    // Side stream: the forward walk, then what needs only its entry states and v_new (dattn, dq). Main stream: attn, E1,
     // E2, the reverse walk, then what needs dS' and dvn, joining the side stream where its results are read.
     ok((int)hipEventRecord(ev[0], s));
     ok((int)hipStreamWaitEvent(s2, ev[0], 0));
@@ -1007,10 +1017,7 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
             (long)R * cc, cc, BC, 1, a.scale, 0, 1, nullptr, s, KSplit{}, dec));
     ok((int)hipEventRecord(ev[4], s));                     // attn
     walk(true, s2);
-    ok((int)hipEventRecord(ev[1], s2));                    // entry states Sc
-    // v_new = u - w S
-    ok(gemm(BC, D, D, nzg, G, 1, W(a.w, BC, D), W(a.Sc, D, D), a.vn, (long)G * cd, cd, 0, D, 1, -1.f, 0, 0, a.u, s2));
-    ok((int)hipEventRecord(ev[2], s2));                    // v_new
+    ok((int)hipEventRecord(ev[1], s2));                    // entry states Sc and v_new
     // dattn_r = tril(dO_r v_new^T); dqd_r = dO_r S^T goes straight into dq_r = s e^gc dqd_r (token-major; the attn
     // share is added below), with each row's dot with q_r (the query path's d gc share) as partials in qdot
     // (the decayed dattn_r; the decay's d gc share from dQK_r . QK_r = dattn_r(undecayed) . attn_r as row and column
@@ -1047,8 +1054,8 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
     walk(false, s);
     // Side stream, after its products: the state path's d gc share, e^(gc_C') <S, dS'>, once the reverse walk has
     // written dS' (enqueued here, after that walk's record, so the wait binds to this call's walk)
-    ok((int)hipEventRecord(ev[6], s));                     // dS'
-    ok((int)hipStreamWaitEvent(s2, ev[6], 0));
+    ok((int)hipEventRecord(ev[2], s));                     // dS'
+    ok((int)hipStreamWaitEvent(s2, ev[2], 0));
     hipLaunchKernelGGL(state_dot_kernel, dim3((unsigned)NB, G, 4), dim3(BW_NT), 0, s2, a);
     ok((int)hipGetLastError());
     ok((int)hipEventRecord(ev[3], s2));                    // dattn, dq, qdot, zr, zc, psd
@@ -1079,7 +1086,6 @@ int gdn_bwd(GdnBwdArgs a, void* ws, hipStream_t s) {
     ok(gemm(BC, D, BC, nzg, G, 1, tr(W(a.dA, BC, BC)), W(a.kb, BC, D), a.dkacc, (long)G * cd, cd, 0, D, 1, 1.f, 1, 0,
             nullptr, s));
     // dkt = v_new dS'^T
-    ok((int)hipStreamWaitEvent(s, ev[2], 0));
     ok(gemm(BC, D, D, nzg, G, 1, W(a.vn, BC, D), tr(W(a.dSx, D, D)), a.dkt, (long)G * cd, cd, 0, D, 1, 1.f, 0, 0,
             nullptr, s));
     ok((int)hipStreamWaitEvent(s, ev[3], 0));             // the side stream's dq, qdot, zr, zc
