@@ -51,6 +51,9 @@ SIGNATURES = {
                            + [_c_int] * 3 + [_fp, _fp] + [_vp] * 5 + [_c_int, _vp]),
     "bf_gdn_layer_step": (_c_int, [_vp, _c_i64, _vp, _vp, _c_int, _vp, _c_int, _c_int, _vp, _vp, _vp, _c_int, _vp, _c_int,
                                    _vp, _vp, _c_int, _fp, _fp, _fp, _vp, _vp, _vp] + [_c_int] * 4 + [_vp]),
+    "bf_gdn_layer_step_x": (_c_int, [_vp, _c_i64, _vp, _vp, _c_int, _vp, _c_int, _c_int, _vp, _c_i64, _c_int, _vp, _vp, _vp,
+                                     _c_int, _vp, _c_int, _vp, _vp, _c_int, _fp, _fp, _fp, _vp, _vp, _vp] + [_c_int] * 4
+                            + [_vp]),
     "bf_gated_norm": (_c_int, [_vp, _c_int, _vp, _vp, _c_i64, _c_int, _fp, _vp, _c_int, _vp]),
     "bf_gdn_fwd_gated": (_c_int, [_vp] * 6 + [_c_int, _c_i64, _c_int, _c_int, _c_int, _fp, _vp, _vp, _vp, _fp, _vp, _vp,
                                        _c_int, _vp, _c_sz, _c_int, _vp]),

@@ -663,11 +663,12 @@ int bf_gdn_conv_inputs(const void* z, int64_t z_st, const void* prefix, int in_d
     return bf::gdn_conv_inputs_dispatch(x, static_cast<hipStream_t>(stream));
 }
 
-int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+// bf_gdn_layer_step, with the gate projections inside where x is given (bf_gdn_layer_step_x)
+static int layer_step(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
                       int w_dtype, int K, const void* a, const void* b, const void* A_log, int A_log_dtype,
                       const void* dt_bias, int dt_bias_dtype, const void* zg, const void* norm_w, int norm_w_dtype,
                       float norm_eps, float l2_eps, float q_scale, const float* state_in, float* state_out, void* out,
-                      int B, int HK, int HV, int D, void* stream) {
+                      int B, int HK, int HV, int D, const void* x_rows, int64_t x_st, int d, void* stream) {
     if (B <= 0 || B > 65535 || HK <= 0 || HV <= 0 || HV % HK || K < 2 || K > 16) return BF_STATUS_INVALID;
     if (!supported_dim(D)) return BF_STATUS_UNSUPPORTED;
     for (int dt : {io_dtype, w_dtype, A_log_dtype, dt_bias_dtype, norm_w_dtype})
@@ -683,8 +684,32 @@ int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* con
     x.w_dtype = w_dtype; x.al_dtype = A_log_dtype; x.dt_dtype = dt_bias_dtype; x.nw_dtype = norm_w_dtype;
     x.z = z; x.z_st = z_st; x.prefix = prefix; x.conv_out = conv_out; x.w = conv_w; x.a = a; x.b = b;
     x.A_log = A_log; x.dt_bias = dt_bias; x.zg = zg; x.norm_w = norm_w;
+    x.x = x_rows; x.x_st = x_st; x.d = d;
     x.l2_eps = l2_eps; x.q_scale = q_scale; x.eps = norm_eps; x.s_in = state_in; x.s_out = state_out; x.out = out;
     return bf::gdn_layer_step_dispatch(x, static_cast<hipStream_t>(stream));
+}
+
+int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+                      int w_dtype, int K, const void* a, const void* b, const void* A_log, int A_log_dtype,
+                      const void* dt_bias, int dt_bias_dtype, const void* zg, const void* norm_w, int norm_w_dtype,
+                      float norm_eps, float l2_eps, float q_scale, const float* state_in, float* state_out, void* out,
+                      int B, int HK, int HV, int D, void* stream) {
+    return layer_step(z, z_st, prefix, conv_out, io_dtype, conv_w, w_dtype, K, a, b, A_log, A_log_dtype, dt_bias,
+                      dt_bias_dtype, zg, norm_w, norm_w_dtype, norm_eps, l2_eps, q_scale, state_in, state_out, out, B, HK,
+                      HV, D, nullptr, 0, 0, stream);
+}
+
+int bf_gdn_layer_step_x(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+                        int w_dtype, int K, const void* x, int64_t x_st, int d, const void* w_a, const void* w_b,
+                        const void* A_log, int A_log_dtype, const void* dt_bias, int dt_bias_dtype, const void* zg,
+                        const void* norm_w, int norm_w_dtype, float norm_eps, float l2_eps, float q_scale,
+                        const float* state_in, float* state_out, void* out, int B, int HK, int HV, int D, void* stream) {
+    if (!x || d <= 0 || d % 8 || x_st < d || x_st % 8) return BF_STATUS_INVALID;
+    for (const void* p : {x, w_a, w_b})
+        if ((uintptr_t)p & 15) return BF_STATUS_INVALID;
+    return layer_step(z, z_st, prefix, conv_out, io_dtype, conv_w, w_dtype, K, w_a, w_b, A_log, A_log_dtype, dt_bias,
+                      dt_bias_dtype, zg, norm_w, norm_w_dtype, norm_eps, l2_eps, q_scale, state_in, state_out, out, B, HK,
+                      HV, D, x, x_st, d, stream);
 }
 
 int bf_gated_norm(const void* o, int o_dtype, const void* z, const float* w, int64_t rows, int D, float eps,

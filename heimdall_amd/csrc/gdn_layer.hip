@@ -320,18 +320,21 @@ __global__ __launch_bounds__(256) void gated_norm_kernel(GatedNormArgs a) {
 // that the norm needs stays in the workgroup. Its loads go out before the small sums, which then cost no time of their
 // own: the pass is bound by reading and writing the state once (134 MB at B = 32, HV = 32, D = 128). As separate
 // kernels (conv pass, step, rounding, norm, the conv rows' concatenation and the parameters' casts to fp32, 15 launches
-// of 2 .. 49 us) the same step took 140 us of GPU time and 260 us of the host's.
+// of 2 .. 49 us) the same step took 140 us of GPU time and 260 us of the host's. With x, the gate logits (two products of
+// 5120 x 32 by one row each, 11 us apiece as library calls) are formed here too, under the state's loads: the layer's step,
+// its other projections included, went from 145 to
+// 105 us at 32 sequences (d = 5120; D = 128. At D = 256 they would cost registers that the state needs).
 __device__ __forceinline__ float ldp(const void* p, long i, int dt) {
     return dt == DT_BF16 ? bf2f(reinterpret_cast<const uint16_t*>(p)[i]) : reinterpret_cast<const float*>(p)[i];
 }
 
-template <int D, bool BF>
+template <int D, bool BF, bool XG>
 __global__ __launch_bounds__(D * D / 64) void gdn_layer_step_kernel(GdnStepLayerArgs a) {
     constexpr int NT = D * D / 64, NW = NT / 64, CG = D / 4, RSTEP = NT / CG, RPT = D / RSTEP;
     static_assert(RPT == 16 && (CG == 16 || CG == 32 || CG == 64), "state split");
     __shared__ float qs[D], ks[D], vs[D], os[D];
     __shared__ __align__(16) float red[NW][D];
-    __shared__ float sq[2][NW];
+    __shared__ float sq[XG ? 4 : 2][NW];
     const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int HK = a.HK, HV = a.HV, r = HV / HK, hk = h / r, K = a.K;
     const int cg = tid % CG, r0 = tid / CG;
@@ -364,17 +367,48 @@ __global__ __launch_bounds__(D * D / 64) void gdn_layer_step_kernel(GdnStepLayer
         if (kind == 0) ssq += y * y;
         else if (kind == 1) ssk += y * y;
     }
+    // the gate logits of this head from the layer's input, 8 elements of x and of either weight row at a time
+    float sa = 0.f, sb = 0.f;
+    if constexpr (XG) {
+        for (int i = 8 * tid; i < a.d; i += 8 * NT) {
+            float xv[8], wa[8], wb[8];
+            load8<BF>(a.x, b * a.x_st + i, true, xv);
+            load8<BF>(a.a, (long)h * a.d + i, true, wa);
+            load8<BF>(a.b, (long)h * a.d + i, true, wb);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                sa = fmaf(xv[e], wa[e], sa);
+                sb = fmaf(xv[e], wb[e], sb);
+            }
+        }
+    }
     ssq = unit_sum<64>(ssq);
     ssk = unit_sum<64>(ssk);
     if (lane == 0) { sq[0][wv] = ssq; sq[1][wv] = ssk; }
+    if constexpr (XG) {
+        sa = unit_sum<64>(sa);
+        sb = unit_sum<64>(sb);
+        if (lane == 0) { sq[2][wv] = sa; sq[3][wv] = sb; }
+    }
     // gates, the same in every thread
-    const float ga = ldp(a.a, bh, a.io_dtype) + ldp(a.dt_bias, h, a.dt_dtype);
-    const float gg = -__expf(ldp(a.A_log, h, a.al_dtype)) * (ga > 20.f ? ga : log1pf(__expf(ga)));
-    const float al = __expf(gg), be = 1.f / (1.f + __expf(-ldp(a.b, bh, a.io_dtype)));
+    float al = 0.f, be = 0.f;
+    auto gates = [&](float la, float lb) {
+        const float ga = la + ldp(a.dt_bias, h, a.dt_dtype);
+        const float gg = -__expf(ldp(a.A_log, h, a.al_dtype)) * (ga > 20.f ? ga : log1pf(__expf(ga)));
+        al = __expf(gg);
+        be = 1.f / (1.f + __expf(-lb));
+    };
+    if constexpr (!XG) gates(ldp(a.a, bh, a.io_dtype), ldp(a.b, bh, a.io_dtype));
     lds_barrier();
     float tq = 0.f, tk = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) { tq += sq[0][w]; tk += sq[1][w]; }
+    if constexpr (XG) {                                  // (rounded as the projections' outputs are)
+        float la = 0.f, lb = 0.f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) { la += sq[2][w]; lb += sq[3][w]; }
+        gates(BF ? bf_round(la) : la, BF ? bf_round(lb) : lb);
+    }
     const float fq = rsqrtf(tq + a.l2_eps) * a.q_scale, fk = rsqrtf(tk + a.l2_eps);
 
     // sum over the rows: lanes of one column group in the wave, then the waves
@@ -450,13 +484,17 @@ __global__ __launch_bounds__(D * D / 64) void gdn_layer_step_kernel(GdnStepLayer
 int gdn_layer_step_dispatch(const GdnStepLayerArgs& a, hipStream_t stream) {
     const dim3 grid((unsigned)a.HV, (unsigned)a.B), block((unsigned)(a.D * a.D / 64));
     const bool bf = a.io_dtype == DT_BF16;
+    auto go = [&](auto k16, auto k32) {
+        if (bf) hipLaunchKernelGGL(k16, grid, block, 0, stream, a);
+        else hipLaunchKernelGGL(k32, grid, block, 0, stream, a);
+    };
     switch (a.D) {
-        case 64: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<64, true>), grid, block, 0, stream, a);
-                 else hipLaunchKernelGGL((gdn_layer_step_kernel<64, false>), grid, block, 0, stream, a); break;
-        case 128: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<128, true>), grid, block, 0, stream, a);
-                  else hipLaunchKernelGGL((gdn_layer_step_kernel<128, false>), grid, block, 0, stream, a); break;
-        case 256: if (bf) hipLaunchKernelGGL((gdn_layer_step_kernel<256, true>), grid, block, 0, stream, a);
-                  else hipLaunchKernelGGL((gdn_layer_step_kernel<256, false>), grid, block, 0, stream, a); break;
+        case 64: if (a.x) go(gdn_layer_step_kernel<64, true, true>, gdn_layer_step_kernel<64, false, true>);
+                 else go(gdn_layer_step_kernel<64, true, false>, gdn_layer_step_kernel<64, false, false>); break;
+        case 128: if (a.x) go(gdn_layer_step_kernel<128, true, true>, gdn_layer_step_kernel<128, false, true>);
+                  else go(gdn_layer_step_kernel<128, true, false>, gdn_layer_step_kernel<128, false, false>); break;
+        case 256: if (a.x) return BF_ERR_UNSUPPORTED;
+                  go(gdn_layer_step_kernel<256, true, false>, gdn_layer_step_kernel<256, false, false>); break;
         default: return BF_ERR_UNSUPPORTED;
     }
     return (int)hipGetLastError();

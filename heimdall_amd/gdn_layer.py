@@ -148,10 +148,14 @@ class GatedDeltaNet(nn.Module):
         prefix = None if cache is None else cache.get("conv")
         s0 = None if cache is None else cache.get("S")
         step = s0 is not None and t == 1
-        a, bb = self.in_proj_a(x), self.in_proj_b(x)
+        inside = step and _gates_inside(self, x)
+        a, bb = (None, None) if inside else (self.in_proj_a(x), self.in_proj_b(x))
         if step:
-            r = _layer_step(self, z.reshape(b, -1), a.reshape(b, -1), bb.reshape(b, -1), self.in_proj_z(x).reshape(b, -1),
-                            prefix, s0)
+            zg = self.in_proj_z(x).reshape(b, -1)
+            r = _layer_step(self, z.reshape(b, -1), x[:, 0] if inside else a.reshape(b, -1),
+                            None if inside else bb.reshape(b, -1), zg, prefix, s0)
+            if r is None and inside:
+                a, bb = self.in_proj_a(x), self.in_proj_b(x)
             if r is not None:
                 o, cache["conv"], cache["S"] = r
                 return self.out_proj(o.view(b, t, self.vd))
@@ -179,8 +183,27 @@ class GatedDeltaNet(nn.Module):
         return self.out_proj(o.reshape(b, t, self.vd))
 
 
+def _gates_inside(m, x) -> bool:
+    """Whether the step kernel forms the gate logits itself: plain bias-free ``nn.Linear`` projections (no hooks, no
+    parametrizations, no autocast) in x's dtype, rows of whole 16-byte pieces. From 64 sequences on each head's weights would
+    be read more often than the two products cost."""
+    if x.shape[0] > 64 or m.c.lin_dk > 128 or x.shape[-1] % 8 or x.stride(-1) != 1 or x.stride(0) % 8 or x.stride(0) < x.shape[-1]:
+        return False
+    mod = nn.modules.module
+    if torch.is_autocast_enabled(x.device.type) or mod._global_forward_hooks or mod._global_forward_pre_hooks or x.data_ptr() % 16:
+        return False
+    for p in (m.in_proj_a, m.in_proj_b):
+        w = p.weight
+        if (type(p) is not nn.Linear or "forward" in p.__dict__ or p.bias is not None or p._forward_hooks or p._forward_pre_hooks
+                or type(w) is not nn.Parameter or w.dtype != x.dtype or w.device != x.device or not w.is_contiguous()
+                or w.shape != (m.c.lin_hv, x.shape[-1]) or w.data_ptr() % 16):
+            return False
+    return True
+
+
 def _layer_step(m, z, a, b, zg, prefix, state):
-    """One token per sequence on ``bf_gdn_layer_step``: z [B, C], a, b [B, hv], zg [B, hv * d] from the projections.
+    """One token per sequence on ``bf_gdn_layer_step``: z [B, C], a, b [B, hv], zg [B, hv * d] from the projections; or a the
+    layer's input rows [B, d_model] and b None, and the kernel forms the gate logits (``_gates_inside``).
     Returns (out [B, hv * d], new conv cache, new state), or None where the call does not apply (other dtypes or
     layouts, a width-1 conv)."""
     c = m.c
@@ -188,7 +211,7 @@ def _layer_step(m, z, a, b, zg, prefix, state):
     K = c.conv_k
     ok = (torch.float32, torch.bfloat16)
     prm = (m.conv1d.weight, m.A_log, m.dt_bias, m.norm.weight)
-    if (K < 2 or z.dtype not in ok or not (z.dtype == a.dtype == b.dtype == zg.dtype) or B > 65535
+    if (K < 2 or z.dtype not in ok or not (z.dtype == a.dtype == zg.dtype) or (b is not None and b.dtype != z.dtype) or B > 65535
             or any(p.dtype not in ok or not p.is_contiguous() for p in prm) or z.stride(1) != 1 or z.stride(0) < C
             or state.shape != (B, c.lin_hv, c.lin_dk, c.lin_dv) or c.lin_dk not in (64, 128, 256)
             or (prefix is not None and prefix.shape != (B, K - 1, C)) or type(m.norm) is not GatedNorm):
@@ -196,18 +219,23 @@ def _layer_step(m, z, a, b, zg, prefix, state):
     require_device(z, a, b, zg, prefix, state, *prm)
     if prefix is not None:
         prefix = prefix.to(z.dtype).contiguous()
-    a, b, zg, s_in = a.contiguous(), b.contiguous(), zg.contiguous(), state.float().contiguous()
+    zg, s_in = zg.contiguous(), state.float().contiguous()
     conv = torch.empty(B, K - 1, C, dtype=z.dtype, device=z.device)
     out, s = torch.empty_like(zg), torch.empty_like(s_in)
     if any(t.data_ptr() % 16 for t in (zg, s_in)):
         return None
     w, al, dt, nw = prm
-    check(_lib.load().bf_gdn_layer_step(
-        z.data_ptr(), z.stride(0), None if prefix is None else prefix.data_ptr(), conv.data_ptr(), dtype_code(z.dtype),
-        w.data_ptr(), dtype_code(w.dtype), K, a.data_ptr(), b.data_ptr(), al.data_ptr(), dtype_code(al.dtype),
-        dt.data_ptr(), dtype_code(dt.dtype), zg.data_ptr(), nw.data_ptr(), dtype_code(nw.dtype), float(m.norm.eps), 1e-6,
-        float(c.lin_dk ** -0.5), s_in.data_ptr(), s.data_ptr(), out.data_ptr(), B, c.lin_hk, c.lin_hv, c.lin_dk,
-        stream_ptr(z.device)), "bf_gdn_layer_step")
+    head = (z.data_ptr(), z.stride(0), None if prefix is None else prefix.data_ptr(), conv.data_ptr(), dtype_code(z.dtype),
+            w.data_ptr(), dtype_code(w.dtype), K)
+    tail = (al.data_ptr(), dtype_code(al.dtype), dt.data_ptr(), dtype_code(dt.dtype), zg.data_ptr(), nw.data_ptr(),
+            dtype_code(nw.dtype), float(m.norm.eps), 1e-6, float(c.lin_dk ** -0.5), s_in.data_ptr(), s.data_ptr(),
+            out.data_ptr(), B, c.lin_hk, c.lin_hv, c.lin_dk, stream_ptr(z.device))
+    if b is None:
+        check(_lib.load().bf_gdn_layer_step_x(*head, a.data_ptr(), a.stride(0), a.shape[1], m.in_proj_a.weight.data_ptr(),
+                                              m.in_proj_b.weight.data_ptr(), *tail), "bf_gdn_layer_step_x")
+    else:
+        a, b = a.contiguous(), b.contiguous()
+        check(_lib.load().bf_gdn_layer_step(*head, a.data_ptr(), b.data_ptr(), *tail), "bf_gdn_layer_step")
     return out, conv, s
 
 

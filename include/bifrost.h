@@ -335,6 +335,16 @@ int bf_gdn_layer_step(const void* z, int64_t z_st, const void* prefix, void* con
                       int B, int HK, int HV, int D, void* stream);
 
 /*
+ * The same with the gate projections inside: a = x w_a^T and b = x w_b^T, summed in fp32 and rounded to io_dtype, for x [B]
+ * rows of d elements x_st apart and w_a, w_b [HV][d], all in io_dtype, 16-byte aligned, d and x_st multiples of 8; D <= 128.
+ */
+int bf_gdn_layer_step_x(const void* z, int64_t z_st, const void* prefix, void* conv_out, int io_dtype, const void* conv_w,
+                        int w_dtype, int K, const void* x, int64_t x_st, int d, const void* w_a, const void* w_b,
+                        const void* A_log, int A_log_dtype, const void* dt_bias, int dt_bias_dtype, const void* zg,
+                        const void* norm_w, int norm_w_dtype, float norm_eps, float l2_eps, float q_scale,
+                        const float* state_in, float* state_out, void* out, int B, int HK, int HV, int D, void* stream);
+
+/*
  * The native layer's delta rule and GatedNorm in one call (Heimdall/heimdall/hibrit.py:180-183: delta_rule, then
  * self.norm(o, z)), for a bf16 layer with D <= 128: bf_gdn_fwd with in_dtype = o_dtype = bf16, whose output row of
  * each (token, head) goes through bf_gated_norm's bf16 arithmetic before it is stored, so out holds the same bits as

@@ -44,6 +44,29 @@ def test_layer_step_equals_separate_calls(dev, dtype, b, hk, hv, d, K, prefixed)
     assert rel(out, ref) < (1e-5 if dtype == torch.float32 else 2e-3), rel(out, ref)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("b,hk,hv,d,x", [(1, 1, 2, 64, 8), (3, 2, 2, 128, 520), (2, 1, 1, 128, 2056), (5, 1, 3, 64, 1024)])
+def test_step_with_gates_inside(dev, dtype, b, hk, hv, d, x):
+    """The gate logits formed in the step kernel against the projections: rows shorter and longer than one pass of the
+    workgroup. fp32: sums in another order; bf16: a logit on a rounding edge moves by one step (2^-8 of it) here and there."""
+    from heimdall_amd import gdn_layer as gl
+    print(f"gates inside B={b} HV={hv} D={d} d_model={x} {dtype}", flush=True)
+    torch.manual_seed(2)
+    m = gl.GatedDeltaNet(gl.GdnLayerConfig(d=x, lin_hk=hk, lin_hv=hv, lin_dk=d, lin_dv=d)).to(device=dev, dtype=dtype)
+    u = torch.randn(b, 1, x, device=dev).to(dtype)
+    cache = lambda: dict(conv=torch.ones(b, 3, (2 * hk + hv) * d, device=dev, dtype=dtype), S=torch.ones(b, hv, d, d, device=dev) * 0.1)
+    assert gl._gates_inside(m, u)
+    c0, c1 = cache(), cache()
+    o = m(u, c0)
+    handle = m.in_proj_a.register_forward_hook(lambda *a: None)          # a hooked projection is called
+    assert not gl._gates_inside(m, u)
+    ref = m(u, c1)
+    handle.remove()
+    tol = 1e-5 if dtype == torch.float32 else 4e-3
+    assert rel(o, ref) < tol and rel(c0["S"], c1["S"]) < tol and torch.equal(c0["conv"], c1["conv"])
+    assert not gl._gates_inside(m, u[..., :x - 1] if x % 8 == 0 else u)
+
+
 @pytest.mark.parametrize("n", [1, 5, 64, 700, 5000])
 def test_conv_blocks(dev, n):
     """Token blocks of 4 .. 64 (H = 32, D = 128: 5000 tokens are the first with 64-token blocks) over packed sequences
