@@ -125,15 +125,10 @@ __device__ __forceinline__ long psi_frag_index(int d, int j) {
 
 // Planes of a 16-column strip as B operands of bf16 MFMAs (gdn_out_kernel): K step s covers rows 32 s .. 32 s + 31, plane p
 // of the step is 64 lanes x 8 elements, and position 8 lg + j of a step is row 4 lg + j (j < 4) or 12 + 4 lg + j: the
-// accumulators of the step's two 16-row tiles, as they lie in a lane. NT tiles, times f.
-template <int NT>
-__device__ __forceinline__ void put_planes(uint16_t* dst, const f32x4 (&x)[NT][NJ], float f, int lane) {
+// accumulators of the step's two 16-row tiles, as they lie in a lane.
+__device__ __forceinline__ void put_planes(uint16_t* dst, int step, const Planes& pl, int lane) {
 #pragma unroll
-    for (int s = 0; s < NT / 2; ++s) {
-        const Planes pl = split8(x[2 * s][0] * f, x[2 * s + 1][0] * f);
-#pragma unroll
-        for (int p = 0; p < 3; ++p) st16(dst + ((s * 3 + p) * 64 + lane) * 8, pl.p[p]);
-    }
+    for (int p = 0; p < 3; ++p) st16(dst + ((step * 3 + p) * 64 + lane) * 8, pl.p[p]);
 }
 
 // N and the segment entry states (fp32 D x D) are stored in accumulator-fragment order: element (d, j) sits in the
@@ -266,9 +261,7 @@ __device__ __forceinline__ constexpr int tpart(int tile) {
 
 // GN (output scan, bf16, whole rows per workgroup): each o row goes through the GatedNorm of the native layer before
 // it is stored, with the arithmetic of gated_norm_kernel (gdn_layer.hip), so the bits equal the two separate passes.
-// ST (fp32 output scan): instead of the query heads' outputs, every chunk's entry state and v_new go to ws_spl / ws_vpl as
-// planes. A lane's accumulators of two consecutive tiles are eight consecutive positions of a plane_frag fragment.
-template <class E, int D, bool OUT, bool BO, bool GN = false, bool ST = false>
+template <class E, int D, bool OUT, bool BO, bool GN = false>
 __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(GdnArgs a) {
     using T = typename E::T;
     using Cfg = SegCfg<E, D, OUT>;
@@ -279,8 +272,7 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
     constexpr bool DBUF = Cfg::DBUF, TPS = Cfg::TPS;
     constexpr bool QL = OUT && DBUF;                     // q staged in LDS, two buffers (bf16); fp32 reads it from global
     constexpr int VW = NW * WCOLS, VROWB = VW * ES;      // V tile: the workgroup's columns
-    static_assert(!ST || (OUT && ES == 4 && NJ == 1), "the state pass is an fp32 output scan");
-    constexpr int NFR = OUT && !ST ? attn_frags<E>() : 0;       // nonzero attn fragments of one query head
+    constexpr int NFR = OUT ? attn_frags<E>() : 0;       // nonzero attn fragments of one query head
     using CL = ChunkLds<E, D, TPS>;
     using OL = OnceLds<E, D, QL ? 2 : 0, VW, NFR * 64 * VEC, !TPS>;
     __shared__ CL cl0;
@@ -694,11 +686,7 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
         // writes are ordered by the barrier that starts head 0, which saves that head its own barrier)
         f32x4 Y[NTC][NJ];
         times_s([&](int ks, int tt) { return lds16(Kb, kq_off(ks, tpart<E>(tt))); }, Y);
-        if constexpr (ST) {
-            const long pb = ((long)(sg.cid0 + c) * G + g) * (D / 16) + jc / 16;
-            put_planes<NTD>(a.ws_spl + pb * (D / 32) * 1536, S, sc, lane);
-        }
-        if constexpr (OUT && !ST) {
+        if constexpr (OUT) {
             const char* Q0b = reinterpret_cast<const char*>(ol.Q[QL ? qb : 0]);
             const rsrc_t rq0 = make_rsrc(reinterpret_cast<const char*>(a.q) + (chunk_tok0(c) * H + (long)g * R) * D * ES,
                                          (uint32_t)(QL ? 0 : (long)chunk_len(c) * H * D * ES));
@@ -743,13 +731,8 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
             }
         }
 
-        if constexpr (ST) {
-            const long pb = ((long)(sg.cid0 + c) * G + g) * (D / 16) + jc / 16;
-            put_planes<NTC>(a.ws_vpl + pb * 2 * 1536, Vn, 1.f, lane);
-        }
-
         // phase 3, per query head r: o_r = scale e^{gc} (q_r S) + attn_r v_new
-        if constexpr (OUT && !ST) {
+        if constexpr (OUT) {
             const long t0 = chunk_tok0(c);
             const int len = chunk_len(c);
             char* Atb = reinterpret_cast<char*>(ol.At);
@@ -1183,9 +1166,233 @@ __attribute__((amdgpu_waves_per_eu(combine_waves<D>() / 4, combine_waves<D>() / 
     if (a.num_seqs < 0) a.ws_c[0] = __uint_as_float(tsink);      // keeps the touches; never taken
 }
 
+// ------------------------------------------------------------------------------------------------ fp32 segment scan
+// The chunk map of gdn_seg_kernel for fp32 runs, on bf16 MFMAs over exact planes (Planes, bf_common.h): OUT = false the
+// summary of a segment, OUT = true the states of a segment (gdn_out_split), where every chunk's entry state and v_new go to
+// ws_spl / ws_vpl. The fp32 MFMA alone took 18 of the 25 us of a chunk at D = 256. K's planes (98 KB there) and T''s are
+// stored in LDS by all waves, from registers loaded a chunk ahead; the planes of the wave's own S columns, of
+// V - e^{gc} K S and of v' are split from its accumulators, which lie in a lane as a step's operand does (put_planes).
+// K rows stay in their own order, since K^T is read through transposing reads of 16 consecutive dims: an A fragment of
+// K is two 8-byte reads, dims 4 lg .. and 16 + 4 lg .. of the step. The 16-byte blocks of a row are permuted by
+// 2 (row & 7) | (row >> 3 & 1): 16 rows of an 8-byte read, and 8 rows x 32 bytes of a transposing one, fall into distinct
+// banks. 8192 tokens, G = 4, R = 6, D = 256: the summary 188 -> 127 us, the states 118 -> 87.
+template <int D, bool OUT>
+__global__ __launch_bounds__((SegCfg<F32, D, OUT>::NW * 64)) void gdn_seg32_kernel(GdnArgs a) {
+    using Cfg = SegCfg<F32, D, OUT>;
+    constexpr int NW = Cfg::NW, NCG = Cfg::NCG, NT = 64 * NW, NTD = D / 16, NKS = D / 32, NBLK = D / 8;
+    constexpr int PC = D / 4, NPK = SC * PC / NT, NPT = 512 / NT;        // K pieces and T' fragments per thread
+    static_assert(WCOLS == 16, "one column tile per wave");
+    __shared__ __align__(16) uint16_t kp[3][SC * D];
+    __shared__ __align__(16) uint16_t tp[8][3][64][8];                    // T' fragments (token tile, step)
+    __shared__ __align__(16) float gc[SC];
+    const int G = a.G;
+    const int xcd = blockIdx.x % NXCD, local = blockIdx.x / NXCD;
+    const int grp = xcd + NXCD * (local / NCG), cg = local % NCG;
+    if (grp >= a.max_segs * G) return;
+    const int g = grp % G;
+    int sid;
+    SegInfo sg;
+    if (!locate_segment(a, grp / G, sid, sg)) return;
+    if (!OUT && sg.p == sg.nseg - 1) return;
+    const int tid = threadIdx.x, lane = lane_id(), wv = wave_id(), l16 = lane & 15, lg = lane >> 4;
+    const int j0 = (cg * NW + wv) * 16;                   // first of this wave's columns in [0, COLS)
+    const bool phi_part = !OUT && j0 >= D;
+    const int jc = phi_part ? j0 - D : j0, n = sg.n, count = sg.count;
+
+    // state strip: rows 16 td + 4 lg + i, column jc + l16
+    f32x4 S[NTD];
+#pragma unroll
+    for (int td = 0; td < NTD; ++td) {
+        f32x4 v = {0.f, 0.f, 0.f, 0.f};
+        const int d0 = 16 * td + 4 * lg, j = jc + l16;
+        if constexpr (OUT) {
+            if (sg.p > 0) {                               // entry state from the combine (fragment order)
+                v = *reinterpret_cast<const f32x4*>(a.ws_sin + ((long)sid * G + g) * D * D + acc_frag_index<D>(d0, j));
+            } else if (a.s0) {                            // the caller's initial state (row-major)
+                const float* src = a.s0 + ((long)n * G + g) * D * D;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) v[i] = src[(long)(d0 + i) * D + j];
+            }
+        } else if (phi_part) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = d0 + i == j ? 1.f : 0.f;
+        }
+        S[td] = v;
+    }
+
+    // a chunk's operands in registers; rows past its end read as zero through the descriptors' range
+    f32x4 xk[NPK], xt[NPT][2];
+    float xg = 0.f, cum_g = 0.f;
+    auto load = [&](int c) {
+        const long t0 = sg.tok0 + (long)c * SC, rem = sg.tok1 - t0, len = rem < SC ? rem : SC;
+        const long cid = sg.cid0 + c;
+        const uint32_t range = (uint32_t)(((len - 1) * G + 1) * D * 4);
+        const rsrc_t rk = make_rsrc(reinterpret_cast<const float*>(a.k) + (t0 * G + g) * D, range);
+#pragma unroll
+        for (int i = 0; i < NPK; ++i) {
+            const int e = tid + NT * i;
+            xk[i] = __builtin_bit_cast(f32x4, buf_ld16(rk, (uint32_t)((e / PC) * G * D + 4 * (e % PC)) * 4u));
+        }
+        const float* T = reinterpret_cast<const float*>(a.ws_T) + (cid * G + g) * SC * SC;
+#pragma unroll
+        for (int i = 0; i < NPT; ++i) {
+            const int f = (tid + NT * i) / 64, tt = f / 2, st = f % 2;
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+                xt[i][h] = *reinterpret_cast<const f32x4*>(T + ((long)(((2 * st + h) * 4 + tt) * 64 + lane)) * 4);
+        }
+        if (tid < SC) xg = a.ws_gcum[(cid * G + g) * SC + tid];
+    };
+    // V of the wave's columns, zero for the Phi columns (an empty range)
+    auto load_v = [&](int c, float (&xv)[16]) {
+        const long t0 = sg.tok0 + (long)c * SC, rem = sg.tok1 - t0, len = rem < SC ? rem : SC;
+        const rsrc_t rv = make_rsrc(reinterpret_cast<const float*>(a.v) + (t0 * G + g) * D,
+                                    phi_part ? 0u : (uint32_t)(((len - 1) * G + 1) * D * 4));
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            xv[i] = buf_ldf(rv, (uint32_t)((16 * (i / 4) + 4 * lg + i % 4) * G * D + jc + l16) * 4u);
+    };
+    auto sw = [](int row) { return (2 * (row & 7) | ((row >> 3) & 1)) & (NBLK - 1); };
+    auto park = [&]() {
+#pragma unroll
+        for (int i = 0; i < NPK; ++i) {
+            const int e = tid + NT * i, row = e / PC, s = e % PC;
+            uint2 p[3];
+            split_pair(xk[i][0], xk[i][1], p[0].x, p[1].x, p[2].x);
+            split_pair(xk[i][2], xk[i][3], p[0].y, p[1].y, p[2].y);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) *reinterpret_cast<uint2*>(&kp[q][row * D + 8 * ((s >> 1) ^ sw(row)) + 4 * (s & 1)]) = p[q];
+        }
+#pragma unroll
+        for (int i = 0; i < NPT; ++i) {
+            const Planes t = split8(xt[i][0], xt[i][1]);
+#pragma unroll
+            for (int q = 0; q < 3; ++q) st16(tp[(tid + NT * i) / 64][q][lane], t.p[q]);
+        }
+        if (tid < SC) gc[tid] = xg;
+    };
+    // A fragments: K rows 16 tt + l16 at the dims of step ks, K^T rows 16 td + l16 at the tokens of step st
+    const int rt = 4 * lg + (l16 >> 2);
+    int sa = sw(l16), sb = sw(rt);
+    auto frag_k = [&](int tt, int ks) {
+        Planes f;
+        const int row = 16 * tt + l16, b0 = (4 * ks + (lg >> 1)) ^ sa, b1 = (4 * ks + 2 + (lg >> 1)) ^ sa;
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            // (volatile: reads of two planes merged into one instruction would have to be moved into place)
+            typedef volatile __attribute__((address_space(3))) uint64_t lds64;
+            const uint64_t lo = *(lds64*)&kp[q][row * D + 8 * b0 + 4 * (lg & 1)];
+            const uint64_t hi = *(lds64*)&kp[q][row * D + 8 * b1 + 4 * (lg & 1)];
+            f.p[q] = make_uint4((uint32_t)lo, (uint32_t)(lo >> 32), (uint32_t)hi, (uint32_t)(hi >> 32));
+        }
+        return f;
+    };
+    auto frag_kt = [&](int td, int st) {
+        Planes f;
+        const int b = (2 * td + ((l16 & 3) >> 1)) ^ sb, at = (32 * st + rt) * D + 8 * b + 4 * (l16 & 1);
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            const char* p = reinterpret_cast<const char*>(&kp[q][at]);
+            const uint2 lo = lds_tr16(p), hi = lds_tr16(p + 16 * D * 2);
+            f.p[q] = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        }
+        return f;
+    };
+
+    if (count > 0) load(0);
+    for (int c = 0; c < count; ++c) {
+        const long pb = ((long)(sg.cid0 + c) * G + g) * (D / 16) + jc / 16;
+        lds_barrier();                                   // every wave is done with the last chunk's tiles
+        park();
+        float v[16];
+        load_v(c, v);                                    // (arrives under Y = K S)
+        // opaque in each chunk: the fragments' permuted addresses would be kept for all chunks, in registers the state needs
+        asm volatile("" : "+v"(sa), "+v"(sb));
+        lds_barrier();
+        const float gl = gc[SC - 1], decay = __expf(gl);
+        cum_g += gl;
+        f32x4 Y[4], Vn[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) Y[tt] = Vn[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        // Y = K S
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const Planes b = split8(S[2 * ks], S[2 * ks + 1]);
+            if constexpr (OUT) put_planes(a.ws_spl + pb * NKS * 1536, ks, b, lane);
+#pragma unroll
+            for (int tt = 0; tt < 4; ++tt) mma3(Y[tt], frag_k(tt, ks), b);
+            __builtin_amdgcn_sched_barrier(0);           // (or every step's reads, and their registers, move to the front)
+        }
+        // v_new = T' (V - e^{gc} Y)
+        f32x4 ev[4];
+#pragma unroll
+        for (int tt = 0; tt < 4; ++tt) {
+            const float4 g4 = *reinterpret_cast<const float4*>(&gc[16 * tt + 4 * lg]);
+            const float gv[4] = {g4.x, g4.y, g4.z, g4.w};
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                Y[tt][i] = v[4 * tt + i] - __expf(gv[i]) * Y[tt][i];
+                ev[tt][i] = __expf(gl - gv[i]);
+            }
+        }
+        load(c + 1 < count ? c + 1 : c);                 // (past the last chunk that one again: no condition for the loads to join)
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            const Planes b = split8(Y[2 * st], Y[2 * st + 1]);
+#pragma unroll
+            for (int tt = 2 * st; tt < 4; ++tt) {        // T' is lower triangular
+                Planes t;
+#pragma unroll
+                for (int q = 0; q < 3; ++q) t.p[q] = ld16(tp[2 * tt + st][q][lane]);
+                mma3(Vn[tt], t, b);
+            }
+        }
+        // S = e^{gc_last} S + K^T (e^{gc_last - gc} v_new)
+#pragma unroll
+        for (int td = 0; td < NTD; ++td) S[td] *= decay;
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            if constexpr (OUT) put_planes(a.ws_vpl + pb * 2 * 1536, st, split8(Vn[2 * st], Vn[2 * st + 1]), lane);
+            const Planes b = split8(Vn[2 * st] * ev[2 * st], Vn[2 * st + 1] * ev[2 * st + 1]);
+#pragma unroll
+            for (int td = 0; td < NTD; ++td) {
+                mma3(S[td], frag_kt(td, st), b);
+                if (td & 1) __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+    }
+
+    if constexpr (OUT) {
+        if (sg.p == sg.nseg - 1 && a.s_out) {
+            float* dst = a.s_out + ((long)n * G + g) * D * D;
+#pragma unroll
+            for (int td = 0; td < NTD; ++td)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) dst[(long)(16 * td + 4 * lg + i) * D + jc + l16] = S[td][i];
+        }
+    } else {
+        // segment map S_end = Phi S_start + N, stored as N, Psi = Phi - c I and c = e^{sum of g}
+        const float c = __expf(cum_g);
+        const long off = ((long)sid * G + g) * D * D;
+#pragma unroll
+        for (int td = 0; td < NTD; ++td) {
+            const int d0 = 16 * td + 4 * lg, j = jc + l16;
+            if (phi_part) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    reinterpret_cast<float*>(a.ws_phi)[off + psi_frag_index<F32, D>(d0 + i, j)] = S[td][i] - (d0 + i == j ? c : 0.f);
+            } else {
+                *reinterpret_cast<f32x4*>(a.ws_n + off + acc_frag_index<D>(d0, j)) = S[td];
+            }
+        }
+        if (cg == 0 && wv == 0 && lane == 0) a.ws_c[(long)sid * G + g] = c;
+    }
+}
+
 // ------------------------------------------------------------------------------------------------ fp32 outputs
 // o_r = scale e^{gc} (q_r S) + attn_r v_new, attn_r = scale (q_r K^T e^{gc_i - gc_j})[i >= j], for the R query heads of one
-// (chunk, KV head, group of 16 NW columns), from the chunk's entry state S and v_new (gdn_seg_kernel, ST). In the scan the
+// (chunk, KV head, group of 16 NW columns), from the chunk's entry state S and v_new (gdn_seg32_kernel). In the scan the
 // heads' products sat in the segment's chain of chunks and ran on the fp32 MFMA, each wave reading all of q from L2; here
 // every chunk is independent and the products are bf16 MFMAs over exact planes (Planes, bf_common.h). A wave holds the
 // planes of its 16 columns of S and v_new in registers for all heads. K's planes stay in LDS; q's go through a double-
@@ -1361,7 +1568,8 @@ template <class E, int D>
 int launch_states(const GdnArgs& a, hipStream_t stream, bool summary, bool combine) {
     if (summary) {
         const dim3 grid = seg_grid<E, D, false>(a), block(SegCfg<E, D, false>::NW * 64);
-        hipLaunchKernelGGL((gdn_seg_kernel<E, D, false, false>), grid, block, 0, stream, a);
+        if constexpr (std::is_same<E, F32>::value) hipLaunchKernelGGL((gdn_seg32_kernel<D, false>), grid, block, 0, stream, a);
+        else hipLaunchKernelGGL((gdn_seg_kernel<E, D, false, false>), grid, block, 0, stream, a);
         const hipError_t e = hipGetLastError();
         if (e != hipSuccess) return (int)e;
     }
@@ -1387,7 +1595,7 @@ int launch_output(const GdnArgs& a, hipStream_t stream) {
     }
     if constexpr (std::is_same<E, F32>::value) {
         if (a.ws_spl) {
-            hipLaunchKernelGGL((gdn_seg_kernel<E, D, true, false, false, true>), grid, block, 0, stream, a);
+            hipLaunchKernelGGL((gdn_seg32_kernel<D, true>), grid, block, 0, stream, a);
             const hipError_t e = hipGetLastError();
             if (e != hipSuccess) return (int)e;
             constexpr int NW = out_waves<D>(), NCG = D / (16 * NW);
