@@ -56,12 +56,13 @@ struct GdnArgs {
     float gn_eps;
 };
 
-// fp32 scans of several query heads per KV head write every chunk's entry state and v_new, and the heads' outputs are
-// products over all chunks at once (gdn_out_kernel), while those planes stay under 2 GiB. One head is left to the scan.
-// 8192 tokens, G = 4, R = 6, D = 256, forward: the scan with outputs 751 us, now its states 118 and the outputs 296.
+// fp32 scans write every chunk's entry state and v_new, and the query heads' outputs are products over all chunks at once
+// (gdn_out_kernel), while those planes stay under 2 GiB. 8192 tokens, G = 4, R = 6, D = 256, forward: the scan with outputs
+// 751 us, its states 118 (87 on planes) and the outputs 296. One head per KV head gains too from D = 128 on (1 x 8192 tokens,
+// H = 4, D = 256: 552 -> 427 us; 3 x 3000, H = 4, D = 128: 201 -> 151), not at D = 64 (1 x 5000, H = 16: 126 -> 130).
 inline size_t gdn_plane_elems(long max_chunks, int G, int D) { return (size_t)max_chunks * G * (D / 16) * (D / 32 + 2) * 1536; }
 inline bool gdn_out_split(long max_chunks, int G, int R, int D, int in_dtype) {
-    return in_dtype == DT_F32 && R >= 2 && 2 * gdn_plane_elems(max_chunks, G, D) <= (size_t)2 << 30;
+    return in_dtype == DT_F32 && (R >= 2 || D >= 128) && 2 * gdn_plane_elems(max_chunks, G, D) <= (size_t)2 << 30;
 }
 
 int gdn_prep(const GdnArgs& a, hipStream_t stream);

@@ -1,4 +1,4 @@
-"""fp32 outputs of several query heads per KV head (the pass over all chunks after the scan), against the recurrence in 64 bits.
+"""fp32 outputs (the pass over all chunks after the scan), against the recurrence in 64 bits.
 
 Chunk tails of 1 and 63 tokens, one chunk, several segments, packed sequences (one of them empty), every head dim, head counts
 that are not a power of two, an initial state, and bf16 outputs. Tolerance: operands carry their 24 bits and sums are fp32 over
@@ -30,6 +30,8 @@ def recurrence(q, k, v, g, beta, s):
     ([63, 0, 200, 65], 3, 2, 64, True, torch.float32),
     ([300, 31], 1, 5, 256, True, torch.float32),
     ([100], 5, 4, 128, False, torch.bfloat16),
+    ([130, 7], 2, 1, 256, True, torch.float32),
+    ([77], 3, 1, 128, False, torch.float32),
 ])
 def test_fp32_outputs(dev, lens, G, R, D, s0, out_dtype):
     from heimdall_amd._device import gdn_forward
