@@ -169,7 +169,7 @@ def _few_inputs(self, x, q, k, start: int, out_dtype):
     G, H, D = self.c.hkv, self.c.h, self.c.dh
     b, t, d = x.shape
     lib = _lib.load()
-    if (b * t > lib.bf_student_inputs_max_tokens() or x.dtype != torch.bfloat16 or d % 8 or 2 * G + H > 64
+    if (b * t > _lib.STUDENT_INPUTS_MAX or x.dtype != torch.bfloat16 or d % 8 or 2 * G + H > 64
             or D not in (64, 128, 256) or x.stride(-1) != 1 or x.stride(1) % 8 or x.data_ptr() % 16
             or (b > 1 and x.stride(0) != t * x.stride(1)) or (t > 1 and x.stride(1) < d)):
         return None
@@ -471,7 +471,7 @@ def student(self, x, q, k, v, qr, kr, start: int, cache: Optional[dict], memory:
         # fused: the gate projections, qm / km (bf16 for a chunk's scan, fp32 for the decode step and the few-token
         # memory branch), gates
         odt = torch.bfloat16 if t > FEW_MAX_T else torch.float32
-        few = _few_inputs(self, x, q, k, start, odt) if t > 1 else None
+        few = _few_inputs(self, x, q, k, start, odt) if 1 < t and b * t <= _lib.STUDENT_INPUTS_MAX else None
         if few is not None:
             qm, km, g, beta, zmix = few
         else:

@@ -76,6 +76,11 @@ def test_status_codes_without_gpu(cpu_lib):
     assert st == -1                                                                            # no phase
 
 
+def test_limits_match_the_library(cpu_lib):
+    from heimdall_amd import _lib
+    assert cpu_lib.bf_student_inputs_max_tokens() == _lib.STUDENT_INPUTS_MAX
+
+
 def test_workspace_size_grows_with_tokens(cpu_lib):
     a, b = ctypes.c_size_t(0), ctypes.c_size_t(0)
     cpu_lib.bf_gdn_workspace_size(4096, 1, 4, 1, 256, 1, 0, ctypes.byref(a))
