@@ -597,11 +597,12 @@ int student_front(FrontArgs& a, bool finish, hipStream_t stream) {
 // ------------------------------------------------------------------------------------------------ fp32 projection
 // out[t][h] = normalize(x[t][h] F_h) * scale for fp32 rows on bf16 MFMAs over exact planes (Planes, bf_common.h), in two
 // launches. The first writes F's planes as B operands: fragment (head, 16 columns, 32 rows, plane) is 64 lanes x 8
-// elements, position 8 lg + j being row 4 lg + j (j < 4) or 12 + 4 lg + j. The second takes 64 tokens of one head: their
-// planes in LDS, a wave's columns over all of D with F's fragments read one step ahead from L2 (a head's 393 KB at D = 256
+// elements, position 8 lg + j being row 4 lg + j (j < 4) or 12 + 4 lg + j. The second takes 32 tokens of one head: their
+// planes in LDS (three workgroups per CU at D = 256; with 64 tokens one, whose load, products and store followed each other:
+// q's pass 84 us against 68), a wave's columns over all of D with F's fragments read one step ahead from L2 (a head's 393 KB at D = 256
 // are read by all its tiles, which neighbour each other on an XCD), the norm over the waves through LDS, and whole rows
 // out. As a transposing copy, an fp32 library product per head, a copy back, a norm and three elementwise passes the
-// q and k projections of 4096 tokens, H = 16, G = 4, D = 256 took 270 us; in these launches 117.
+// q and k projections of 4096 tokens, H = 16, G = 4, D = 256 took 270 us; in these launches 100.
 template <int D>
 __global__ __launch_bounds__(2 * D) void mem_planes_kernel(const float* f, uint16_t* planes) {
     constexpr int NKS = D / 32;
@@ -619,12 +620,13 @@ __global__ __launch_bounds__(2 * D) void mem_planes_kernel(const float* f, uint1
     for (int i = 0; i < 3; ++i) st16(dst + i * 512, s.p[i]);
 }
 
+constexpr int P32_TOK = 32;      // tokens per workgroup
 template <int D>
 constexpr int proj32_waves() { return D < 128 ? D / 16 : 8; }
 
 template <int D>
 __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(MemProjArgs a, const uint16_t* planes) {
-    constexpr int NW = proj32_waves<D>(), NT = 64 * NW, CT = D / (16 * NW), NKS = D / 32, TOK = 64;
+    constexpr int NW = proj32_waves<D>(), NT = 64 * NW, CT = D / (16 * NW), NKS = D / 32, TOK = P32_TOK, NTT = TOK / 16;
     constexpr int XP = TOK * (D + 8), PC = D / 4;        // elements of a plane, 16-byte pieces of a row
     __shared__ __align__(16) char lds[3 * XP * 2];       // the rows' planes, then the output rows [TOK][D + 4] fp32
     __shared__ float part[NW][TOK];
@@ -657,9 +659,9 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
 #pragma unroll
             for (int i = 0; i < 3; ++i) f[c].p[i] = ld16(fp + ((long)(c * NKS + ks) * 3 + i) * 512);
     };
-    f32x4 acc[4][CT];
+    f32x4 acc[NTT][CT];
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
+    for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[tt][c] = f32x4{0.f, 0.f, 0.f, 0.f};
     Planes f[2][CT];
@@ -669,7 +671,7 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
     for (int ks = 0; ks < NKS; ++ks) {
         read_f(min(ks + 1, NKS - 1), f[(ks + 1) & 1]);
 #pragma unroll
-        for (int tt = 0; tt < 4; ++tt) {
+        for (int tt = 0; tt < NTT; ++tt) {
             Planes ax;
 #pragma unroll
             for (int i = 0; i < 3; ++i) ax.p[i] = ld16(xs + i * XP + (16 * tt + l16) * (D + 8) + 32 * ks + 8 * lg);
@@ -680,7 +682,7 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
     }
     // row norms: this wave's columns (lanes of equal lg), then the waves
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
+    for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             float ss = 0.f;
@@ -693,7 +695,7 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
     __syncthreads();                                     // also: every wave is done with the planes
     float* os = reinterpret_cast<float*>(lds);
 #pragma unroll
-    for (int tt = 0; tt < 4; ++tt)
+    for (int tt = 0; tt < NTT; ++tt)
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int row = 16 * tt + 4 * lg + e;
@@ -719,7 +721,7 @@ int launch_project32(const MemProjArgs& a, uint16_t* planes, hipStream_t stream)
     hipLaunchKernelGGL((mem_planes_kernel<D>), dim3(D / 16, a.nh), dim3(2 * D), 0, stream, static_cast<const float*>(a.f), planes);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return (int)e;
-    const long per = ((a.n_tok + 63) / 64 * a.nh + 7) / 8;
+    const long per = ((a.n_tok + P32_TOK - 1) / P32_TOK * a.nh + 7) / 8;
     if (8 * per > 0x7fffffffL || a.nh > 65535) return BF_STATUS_INVALID;
     hipLaunchKernelGGL((mem_project32_kernel<D>), dim3((unsigned)(8 * per)), dim3(64 * proj32_waves<D>()), 0, stream, a, planes);
     return (int)hipGetLastError();

@@ -54,8 +54,7 @@ def _heads_matmul(x: torch.Tensor, f: torch.Tensor) -> torch.Tensor:
 
 def _project_f32(x: torch.Tensor, f: torch.Tensor, scale: float) -> torch.Tensor:
     """fp32 x [b, t, h, D] -> normalize(x_h f_h) * scale per head: bf_mem_project_f32 on the GPU where nothing is recorded or
-    transformed, PyTorch operators otherwise. Below 64 tokens a tile of the kernel would be mostly empty and its first
-    pass over f is most of the work."""
+    transformed, PyTorch operators otherwise. Below 64 tokens the kernel's first pass over f would be most of its work."""
     b, t, h, d = x.shape
     if (not x.is_cuda or b * t < 64 or d not in (64, 128, 256) or f.shape != (h, d, d) or f.device != x.device
             or (torch.is_grad_enabled() and (x.requires_grad or f.requires_grad)) or _transformed(x, f)):

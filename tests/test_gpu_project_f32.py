@@ -1,4 +1,4 @@
-"""The fp32 memory projection (``bf_mem_project_f32``) at the edges of its 64-token tiles, against 64 bits; and the calls that
+"""The fp32 memory projection (``bf_mem_project_f32``) at the edges of its 32-token tiles, against 64 bits; and the calls that
 keep the PyTorch operators. Tolerance: operands carry their 24 bits, sums of D products in fp32: 1e-6 of the norm.
 """
 import pytest
