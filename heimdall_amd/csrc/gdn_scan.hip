@@ -155,36 +155,28 @@ __device__ __forceinline__ void seq_bounds(const GdnArgs& a, int n, long& s0, lo
     s1 = a.cu_seqlens ? (long)a.cu_seqlens[n + 1] : (long)(n + 1) * a.seq_len;
 }
 
-// Segments enumerate sequence 0's segments, then sequence 1's, ... (sid, their place in the workspace); an empty
-// sequence has one empty segment. Workgroups take them in another order: idx counts the whole segments (L chunks) of
-// all sequences first, then each sequence's last one where it is shorter. Packed sequences leave about half a segment
-// over each; started last, the short ones fill the slots that the long ones leave instead of delaying them (4 packed
-// sequences, 65536 tokens, H = 32, D = 128, L = 129: the layer core 2.62 -> 2.43 ms). The outputs do not depend on the order.
-__device__ __forceinline__ bool locate_segment(const GdnArgs& a, int idx, int& sid, SegInfo& s) {
+// Segments enumerate sequence 0's segments, then sequence 1's, ...; an empty sequence has one empty segment.
+__device__ __forceinline__ bool locate_segment(const GdnArgs& a, int sid, SegInfo& s) {
     const int L = a.seg_chunks;
-    for (int tails = 0; tails < 2; ++tails) {
-        int base_seg = 0, base_cid = 0;
-        for (int n = 0; n < a.num_seqs; ++n) {
-            long s0, s1;
-            seq_bounds(a, n, s0, s1);
-            const int nc = (int)((s1 - s0 + SC - 1) / SC), whole = nc / L;
-            const int ns = nc > 0 ? (nc + L - 1) / L : 1, mine = tails ? ns - whole : whole;
-            if (idx < mine) {
-                const int p = tails ? whole : idx;
-                sid = base_seg + p;
-                s.n = n;
-                s.p = p;
-                s.nseg = ns;
-                s.cid0 = base_cid + p * L;
-                s.count = nc - p * L < L ? nc - p * L : L;
-                s.tok0 = s0 + (long)p * L * SC;
-                s.tok1 = s1;
-                return true;
-            }
-            idx -= mine;
-            base_seg += ns;
-            base_cid += nc;
+    int base_seg = 0, base_cid = 0;
+    for (int n = 0; n < a.num_seqs; ++n) {
+        long s0, s1;
+        seq_bounds(a, n, s0, s1);
+        const int nc = (int)((s1 - s0 + SC - 1) / SC);
+        const int ns = nc > 0 ? (nc + L - 1) / L : 1;
+        if (sid < base_seg + ns) {
+            const int p = sid - base_seg;
+            s.n = n;
+            s.p = p;
+            s.nseg = ns;
+            s.cid0 = base_cid + p * L;
+            s.count = nc - p * L < L ? nc - p * L : L;
+            s.tok0 = s0 + (long)p * L * SC;
+            s.tok1 = s1;
+            return true;
         }
+        base_seg += ns;
+        base_cid += nc;
     }
     return false;
 }
@@ -283,10 +275,9 @@ __global__ __launch_bounds__(SEG_THREADS, SEG_WAVES_PER_EU) void gdn_seg_kernel(
     const int xcd = blockIdx.x % NXCD, local = blockIdx.x / NXCD;
     const int grp = xcd + NXCD * (local / NCG), cg = local % NCG;
     if (grp >= a.max_segs * G) return;
-    const int g = grp % G;
-    int sid;
+    const int g = grp % G, sid = grp / G;
     SegInfo sg;
-    if (!locate_segment(a, grp / G, sid, sg)) return;
+    if (!locate_segment(a, sid, sg)) return;
     if (!OUT && sg.p == sg.nseg - 1) return;
 
     const int lane = lane_id(), wv = wave_id(), l16 = lane & 15, lg = lane >> 4;
@@ -1190,9 +1181,9 @@ __global__ __launch_bounds__((SegCfg<F32, D, OUT>::NW * 64)) void gdn_seg32_kern
     const int grp = xcd + NXCD * (local / NCG), cg = local % NCG;
     if (grp >= a.max_segs * G) return;
     const int g = grp % G;
-    int sid;
+    const int sid = grp / G;
     SegInfo sg;
-    if (!locate_segment(a, grp / G, sid, sg)) return;
+    if (!locate_segment(a, sid, sg)) return;
     if (!OUT && sg.p == sg.nseg - 1) return;
     const int tid = threadIdx.x, lane = lane_id(), wv = wave_id(), l16 = lane & 15, lg = lane >> 4;
     const int j0 = (cg * NW + wv) * 16;                   // first of this wave's columns in [0, COLS)
