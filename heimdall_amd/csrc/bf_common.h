@@ -110,27 +110,34 @@ __device__ __forceinline__ uint2 lds_tr16(const char* p) {
                       (uint16_t)v[2] | ((uint32_t)(uint16_t)v[3] << 16));
 }
 
-// fp32 operands of a bf16 MFMA: x = p[0] + p[1] + p[2] exactly, three bf16 planes (8 + 8 + 8 of the 24 significand bits:
-// the first truncated, so it never overflows, the second rounded to nearest, the third what is left). Of the nine plane
-// products the six down to 2^-16 of the first are summed (mma3); the three left out are below 2^-23 |a b| and 2^-26 on
-// average, of either sign, less than the rounding of an fp32 product. Six v_mfma_f32_16x16x32_bf16 take 96 cycles, the
-// eight v_mfma_f32_16x16x4_f32 of the same contraction 256. An infinite operand gives NaN.
+// fp32 operands of a bf16 MFMA: x = p[0] + p[1] + p[2], three bf16 planes (8 + 8 + 8 of the 24 significand bits, each rounded
+// to nearest, so the second is within 2^-8 and the third within 2^-17 of x). The sum is exact from 2^-109 up (the third plane
+// is a bf16 number there) to 2^128 (1 - 2^-9), the largest the first plane rounds to, and off by 2^-24 of x above. Of the nine
+// plane products the six down to 2^-16 of the first are summed (mma3); the three left out are at most 2^-24 |a b|, as much as
+// rounding the product to fp32, and 2^-27.5 rms, of either sign (with the first plane truncated, which needs no clamp,
+// they reach 2^-22). The instruction's own addition to the accumulator errs by up to 2^-23, where an fp32 MFMA rounds to
+// nearest: against 64 bits, in units of the sum of |a b|, one product is off by 2^-24.8 rms (fp32 MFMA 2^-25.2), 16 products
+// of one size by 2^-26.5 (2^-25.5: one addition stands for eight). Six v_mfma_f32_16x16x32_bf16 take 96 cycles, the eight
+// v_mfma_f32_16x16x4_f32 of the same contraction 256. An infinite operand gives NaN.
 struct Planes {
     uint4 p[3];
 };
+// CLAMP = false: x, y below the largest that rounds to a finite plane.
+template <bool CLAMP = true>
 __device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
-    const uint32_t ux = __float_as_uint(x), uy = __float_as_uint(y);
-    h = __builtin_amdgcn_perm(uy, ux, 0x07060302u);                  // the high halves, x's in the low half
-    const float rx = x - __uint_as_float(ux & 0xffff0000u), ry = y - __uint_as_float(uy & 0xffff0000u);
+    constexpr float TOP = 0x1.fefffep127f;                           // that number
+    h = CLAMP ? pack_bf16x2(__builtin_amdgcn_fmed3f(x, -TOP, TOP), __builtin_amdgcn_fmed3f(y, -TOP, TOP)) : pack_bf16x2(x, y);
+    const float rx = x - __uint_as_float(h << 16), ry = y - __uint_as_float(h & 0xffff0000u);
     m = pack_bf16x2(rx, ry);
     l = pack_bf16x2(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u));
 }
+template <bool CLAMP = true>
 __device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b) {
     Planes s;
-    split_pair(a[0], a[1], s.p[0].x, s.p[1].x, s.p[2].x);
-    split_pair(a[2], a[3], s.p[0].y, s.p[1].y, s.p[2].y);
-    split_pair(b[0], b[1], s.p[0].z, s.p[1].z, s.p[2].z);
-    split_pair(b[2], b[3], s.p[0].w, s.p[1].w, s.p[2].w);
+    split_pair<CLAMP>(a[0], a[1], s.p[0].x, s.p[1].x, s.p[2].x);
+    split_pair<CLAMP>(a[2], a[3], s.p[0].y, s.p[1].y, s.p[2].y);
+    split_pair<CLAMP>(b[0], b[1], s.p[0].z, s.p[1].z, s.p[2].z);
+    split_pair<CLAMP>(b[2], b[3], s.p[0].w, s.p[1].w, s.p[2].w);
     return s;
 }
 __device__ __forceinline__ void mma3(f32x4& acc, const Planes& a, const Planes& b) {

@@ -306,7 +306,7 @@ __global__ __launch_bounds__(64 * NW) void window_kernel(WinArgs a) {
                         o[qt][dt][0] *= corr; o[qt][dt][1] *= corr; o[qt][dt][2] *= corr; o[qt][dt][3] *= corr;
                     }
                 }
-                pb[qt] = split8(s[qt][0], s[qt][1]);
+                pb[qt] = split8<false>(s[qt][0], s[qt][1]);      // (probabilities)
             }
             // O^T += V^T P^T: the K index 8 lg + e is key 4 lg + e of the first 16 (e < 4) or of the second
             auto read_v = [&](int dt) {
