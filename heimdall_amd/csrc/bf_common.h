@@ -118,26 +118,34 @@ __device__ __forceinline__ uint2 lds_tr16(const char* p) {
 // they reach 2^-22). The instruction's own addition to the accumulator errs by up to 2^-23, where an fp32 MFMA rounds to
 // nearest: against 64 bits, in units of the sum of |a b|, one product is off by 2^-24.8 rms (fp32 MFMA 2^-25.2), 16 products
 // of one size by 2^-26.5 (2^-25.5: one addition stands for eight). Six v_mfma_f32_16x16x32_bf16 take 96 cycles, the eight
-// v_mfma_f32_16x16x4_f32 of the same contraction 256. An infinite operand gives NaN.
+// v_mfma_f32_16x16x4_f32 of the same contraction 256.
 struct Planes {
     uint4 p[3];
 };
-// CLAMP = false: x, y below the largest that rounds to a finite plane.
-template <bool CLAMP = true>
+// Which operands a split takes: SMALL, below the largest number that rounds to a finite plane; FINITE, where an infinity
+// becomes NaN, as it ends as one in the delta rule and its backward whatever the products give (the zeros of a triangle meet
+// it); ANY. There the first two planes are those of x clamped to that number, and an infinity (or NaN) stands in the third
+// alone, which meets only the other operand's first plane, zero only where that operand is: the sum is infinite, of the right
+// sign, where an fp32 product is. (Other operands up to 2^8 in size: past that the clamped planes' own products overflow, of
+// either sign.) In the scans and the backward too, ANY would cost a training segment of 8192 tokens another 0.6 %, 15 us.
+enum SplitRange { SPLIT_SMALL, SPLIT_FINITE, SPLIT_ANY };
+template <SplitRange RANGE = SPLIT_FINITE>
 __device__ __forceinline__ void split_pair(float x, float y, uint32_t& h, uint32_t& m, uint32_t& l) {
     constexpr float TOP = 0x1.fefffep127f;                           // that number
-    h = CLAMP ? pack_bf16x2(__builtin_amdgcn_fmed3f(x, -TOP, TOP), __builtin_amdgcn_fmed3f(y, -TOP, TOP)) : pack_bf16x2(x, y);
-    const float rx = x - __uint_as_float(h << 16), ry = y - __uint_as_float(h & 0xffff0000u);
-    m = pack_bf16x2(rx, ry);
+    const float cx = RANGE == SPLIT_SMALL ? x : __builtin_amdgcn_fmed3f(x, -TOP, TOP);
+    const float cy = RANGE == SPLIT_SMALL ? y : __builtin_amdgcn_fmed3f(y, -TOP, TOP);
+    h = pack_bf16x2(cx, cy);
+    const float hx = __uint_as_float(h << 16), hy = __uint_as_float(h & 0xffff0000u), rx = x - hx, ry = y - hy;
+    m = RANGE == SPLIT_ANY ? pack_bf16x2(cx - hx, cy - hy) : pack_bf16x2(rx, ry);
     l = pack_bf16x2(rx - __uint_as_float(m << 16), ry - __uint_as_float(m & 0xffff0000u));
 }
-template <bool CLAMP = true>
+template <SplitRange RANGE = SPLIT_FINITE>
 __device__ __forceinline__ Planes split8(const f32x4& a, const f32x4& b) {
     Planes s;
-    split_pair<CLAMP>(a[0], a[1], s.p[0].x, s.p[1].x, s.p[2].x);
-    split_pair<CLAMP>(a[2], a[3], s.p[0].y, s.p[1].y, s.p[2].y);
-    split_pair<CLAMP>(b[0], b[1], s.p[0].z, s.p[1].z, s.p[2].z);
-    split_pair<CLAMP>(b[2], b[3], s.p[0].w, s.p[1].w, s.p[2].w);
+    split_pair<RANGE>(a[0], a[1], s.p[0].x, s.p[1].x, s.p[2].x);
+    split_pair<RANGE>(a[2], a[3], s.p[0].y, s.p[1].y, s.p[2].y);
+    split_pair<RANGE>(b[0], b[1], s.p[0].z, s.p[1].z, s.p[2].z);
+    split_pair<RANGE>(b[2], b[3], s.p[0].w, s.p[1].w, s.p[2].w);
     return s;
 }
 __device__ __forceinline__ void mma3(f32x4& acc, const Planes& a, const Planes& b) {

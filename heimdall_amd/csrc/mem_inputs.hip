@@ -614,7 +614,7 @@ __global__ __launch_bounds__(2 * D) void mem_planes_kernel(const float* f, uint1
         a[j] = p[j * D];
         b[j] = p[(16 + j) * D];
     }
-    const Planes s = split8(a, b);
+    const Planes s = split8<SPLIT_ANY>(a, b);
     uint16_t* dst = planes + ((((long)h * (D / 16) + ct) * NKS + ks) * 3 * 64 + lane) * 8;
 #pragma unroll
     for (int i = 0; i < 3; ++i) st16(dst + i * 512, s.p[i]);
@@ -646,8 +646,8 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
         const int row = c / PC, s = c % PC;              // rows past the last token: the last one again (not stored)
         const f32x4 v = *reinterpret_cast<const f32x4*>(x + min(row, n - 1) * a.x_st + 4 * s);
         uint2 p[3];
-        split_pair(v[0], v[1], p[0].x, p[1].x, p[2].x);
-        split_pair(v[2], v[3], p[0].y, p[1].y, p[2].y);
+        split_pair<SPLIT_ANY>(v[0], v[1], p[0].x, p[1].x, p[2].x);
+        split_pair<SPLIT_ANY>(v[2], v[3], p[0].y, p[1].y, p[2].y);
         uint16_t* dst = xs + row * (D + 8) + 32 * (s / 8) + 8 * (s % 4) + 4 * (s % 8 / 4);
 #pragma unroll
         for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(dst + i * XP) = p[i];

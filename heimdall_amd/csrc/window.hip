@@ -82,8 +82,8 @@ struct W32Rows {
         uint2 s[3];
         // opaque here, or the split moves up out of the two branches that store the piece, into more registers
         asm volatile("" : "+v"(x[j]));
-        split_pair(x[j][0], x[j][1], s[0].x, s[1].x, s[2].x);
-        split_pair(x[j][2], x[j][3], s[0].y, s[1].y, s[2].y);
+        split_pair<SPLIT_ANY>(x[j][0], x[j][1], s[0].x, s[1].x, s[2].x);
+        split_pair<SPLIT_ANY>(x[j][2], x[j][3], s[0].y, s[1].y, s[2].y);
 #pragma unroll
         for (int i = 0; i < 3; ++i) *reinterpret_cast<uint2*>(&t[i][row(wv, lane, j)][4 * (lane % (D / 4))]) = s[i];
     }
@@ -128,8 +128,8 @@ __global__ __launch_bounds__(64 * NW) void window_kernel(WinArgs a) {
         const float* qrow = Qb + (qi0 + min(qrel + 16 * qt, nq - 1)) * a.q_st + dh;
 #pragma unroll
         for (int kf = 0; kf < NKD; ++kf)
-            fq[qt][kf] = split8(*reinterpret_cast<const f32x4*>(qrow + 32 * kf + 8 * lg),
-                                *reinterpret_cast<const f32x4*>(qrow + 32 * kf + 8 * lg + 4));
+            fq[qt][kf] = split8<SPLIT_ANY>(*reinterpret_cast<const f32x4*>(qrow + 32 * kf + 8 * lg),
+                                           *reinterpret_cast<const f32x4*>(qrow + 32 * kf + 8 * lg + 4));
     }
     f32x4 o[QT][NDT];
     float m[QT], l[QT];
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(64 * NW) void window_kernel(WinArgs a) {
                         o[qt][dt][0] *= corr; o[qt][dt][1] *= corr; o[qt][dt][2] *= corr; o[qt][dt][3] *= corr;
                     }
                 }
-                pb[qt] = split8<false>(s[qt][0], s[qt][1]);      // (probabilities)
+                pb[qt] = split8<SPLIT_SMALL>(s[qt][0], s[qt][1]);      // (probabilities)
             }
             // O^T += V^T P^T: the K index 8 lg + e is key 4 lg + e of the first 16 (e < 4) or of the second
             auto read_v = [&](int dt) {

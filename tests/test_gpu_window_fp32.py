@@ -52,3 +52,29 @@ def test_window_fp32_tiles(dev, B, H, G, D, T, W, S, start, miss):
     err = ((o.cpu().double() - ref).norm() / ref.norm()).item()
     assert err < 2e-6, err
     assert (lse.cpu().double() - ref_lse).abs().max().item() < 1e-5
+
+
+def classes(x):
+    """0 finite, 1 +inf, 2 -inf, 3 nan."""
+    return torch.where(x.isnan(), 3, torch.where(x == math.inf, 1, torch.where(x == -math.inf, 2, 0)))
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("T", [40, 200])
+def test_window_fp32_infinities(dev, D, T):
+    """Infinite elements give what they give in 64 bits: in a value row that every query sees, that column; in a key, a score
+    of -inf, which leaves the key out. The finite elements stay within the tolerance above."""
+    c = make_case(1, 4, 2, D, T, 64, 4, 300, seed=T, dtype=torch.float32)
+    print(f"window fp32 infinities D={D} T={T}", flush=True)
+    c["sink_v"][0, 0, 1, 3] = math.inf
+    c["sink_v"][0, 1, 2, D - 1] = -math.inf
+    c["qr"][..., 2] = -1.0
+    c["kr"][0, 0, 20, 2] = math.inf
+    c["ring_k"][0, 1, :, 2] = 0.0
+    c["ring_k"][0, 1, 290 % 64, 2] = math.inf
+    o, lse = run(c, dev)[:2]
+    ref, ref_lse = reference(c)
+    assert torch.equal(classes(o.cpu()), classes(ref))
+    fin = ref.isfinite()
+    assert ((o.cpu().double() - ref)[fin].norm() / ref[fin].norm()).item() < 2e-6
+    assert (lse.cpu().double() - ref_lse).abs().max().item() < 1e-5
