@@ -702,7 +702,7 @@ __global__ __launch_bounds__(64 * proj32_waves<D>()) void mem_project32_kernel(M
             float ss = 0.f;
 #pragma unroll
             for (int w = 0; w < NW; ++w) ss += part[w][row];
-            const float nrm = fmaxf(sqrtf(ss), 1e-12f);
+            const float root = sqrtf(ss), nrm = root < 1e-12f ? 1e-12f : root;      // (NaN stays, which fmaxf would drop)
 #pragma unroll
             for (int c = 0; c < CT; ++c) os[row * (D + 4) + 16 * (wv * CT + c) + l16] = acc[tt][c][e] / nrm * a.scale;
         }

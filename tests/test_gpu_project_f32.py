@@ -36,6 +36,22 @@ def test_projection_tiles(dev, b, t, h, d, layout):
     assert not zero.any()
 
 
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_projection_of_nonfinite_values(dev, d):
+    """What the operators give in 64 bits: a NaN in a projection makes the head's rows NaN, an infinity their other elements
+    zero, a row with an infinity is NaN."""
+    from heimdall_amd.hibrit import _project_f32
+    gen = torch.Generator().manual_seed(d)
+    x, f = torch.randn(1, 70, 3, d, generator=gen), torch.randn(3, d, d, generator=gen)
+    f[0, 3, 5], f[1, 4, 6], x[0, 9, 2, 1] = float("nan"), float("inf"), float("inf")
+    ref = torch.stack([F.normalize(x[:, :, h].double() @ f[h].double(), dim=-1) for h in range(3)], 2)
+    with torch.no_grad():
+        o = _project_f32(x.to(dev), f.to(dev), 1.0).cpu()
+    assert torch.equal(o.isnan(), ref.isnan()) and not o.isinf().any()
+    fin = ref.isfinite()
+    assert (o.double() - ref)[fin].abs().max().item() < 1e-6
+
+
 def test_recorded_and_transformed_calls(dev):
     """Gradients, vmap and forward mode go through PyTorch operators, with the same values."""
     from heimdall_amd.hibrit import _project_f32
