@@ -183,19 +183,25 @@ class GatedDeltaNet(nn.Module):
         return self.out_proj(o.reshape(b, t, self.vd))
 
 
+def _plain(p, cls) -> bool:
+    """A call of module p is cls.forward and nothing else: no subclass, no forward of its own, no hooks."""
+    mod = nn.modules.module
+    return (type(p) is cls and "forward" not in p.__dict__ and not p._forward_hooks and not p._forward_pre_hooks
+            and not mod._global_forward_hooks and not mod._global_forward_pre_hooks)
+
+
 def _gates_inside(m, x) -> bool:
     """Whether the step kernel forms the gate logits itself: plain bias-free ``nn.Linear`` projections (no hooks, no
     parametrizations, no autocast) in x's dtype, rows of whole 16-byte pieces. From 64 sequences on each head's weights would
     be read more often than the two products cost."""
     if x.shape[0] > 64 or m.c.lin_dk > 128 or x.shape[-1] % 8 or x.stride(-1) != 1 or x.stride(0) % 8 or x.stride(0) < x.shape[-1]:
         return False
-    mod = nn.modules.module
-    if torch.is_autocast_enabled(x.device.type) or mod._global_forward_hooks or mod._global_forward_pre_hooks or x.data_ptr() % 16:
+    if torch.is_autocast_enabled(x.device.type) or x.data_ptr() % 16:
         return False
     for p in (m.in_proj_a, m.in_proj_b):
         w = p.weight
-        if (type(p) is not nn.Linear or "forward" in p.__dict__ or p.bias is not None or p._forward_hooks or p._forward_pre_hooks
-                or type(w) is not nn.Parameter or w.dtype != x.dtype or w.device != x.device or not w.is_contiguous()
+        if (not _plain(p, nn.Linear) or p.bias is not None or type(w) is not nn.Parameter or w.dtype != x.dtype
+                or w.device != x.device or not w.is_contiguous()
                 or w.shape != (m.c.lin_hv, x.shape[-1]) or w.data_ptr() % 16):
             return False
     return True
@@ -205,7 +211,7 @@ def _layer_step(m, z, a, b, zg, prefix, state):
     """One token per sequence on ``bf_gdn_layer_step``: z [B, C], a, b [B, hv], zg [B, hv * d] from the projections; or a the
     layer's input rows [B, d_model] and b None, and the kernel forms the gate logits (``_gates_inside``).
     Returns (out [B, hv * d], new conv cache, new state), or None where the call does not apply (other dtypes or
-    layouts, a width-1 conv)."""
+    layouts, a width-1 conv, a norm that is more than its own forward)."""
     c = m.c
     B, C = z.shape
     K = c.conv_k
@@ -214,7 +220,7 @@ def _layer_step(m, z, a, b, zg, prefix, state):
     if (K < 2 or z.dtype not in ok or not (z.dtype == a.dtype == zg.dtype) or (b is not None and b.dtype != z.dtype) or B > 65535
             or any(p.dtype not in ok or not p.is_contiguous() for p in prm) or z.stride(1) != 1 or z.stride(0) < C
             or state.shape != (B, c.lin_hv, c.lin_dk, c.lin_dv) or c.lin_dk not in (64, 128, 256)
-            or (prefix is not None and prefix.shape != (B, K - 1, C)) or type(m.norm) is not GatedNorm):
+            or (prefix is not None and prefix.shape != (B, K - 1, C)) or not _plain(m.norm, GatedNorm)):
         return None
     require_device(z, a, b, zg, prefix, state, *prm)
     if prefix is not None:

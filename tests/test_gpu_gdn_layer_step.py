@@ -67,6 +67,51 @@ def test_step_with_gates_inside(dev, dtype, b, hk, hv, d, x):
     assert not gl._gates_inside(m, u[..., :x - 1] if x % 8 == 0 else u)
 
 
+def make_layer(dev, dtype, hk, hv, d, x, norm=None):
+    from heimdall_amd import gdn_layer as gl
+    torch.manual_seed(4)
+    m = gl.GatedDeltaNet(gl.GdnLayerConfig(d=x, lin_hk=hk, lin_hv=hv, lin_dk=d, lin_dv=d))
+    if norm is not None:
+        m.norm = norm
+    m = m.to(device=dev, dtype=dtype)
+    with torch.no_grad():
+        m.conv1d.weight.normal_(0, 0.5)
+    return m
+
+
+def step_cache(dev, dtype, b, hk, hv, d):
+    gen = torch.Generator(device=dev).manual_seed(b)
+    return dict(conv=torch.randn(b, 3, (2 * hk + hv) * d, device=dev, generator=gen).to(dtype),
+                S=torch.randn(b, hv, d, d, device=dev, generator=gen) * 0.1)
+
+
+@pytest.mark.parametrize("how", ["hook", "pre-hook", "global hook", "instance"])
+def test_step_calls_a_changed_norm(dev, how):
+    """A norm with hooks or a forward of its own is called: its doubled output doubles the layer's (bf16, tolerance as above)."""
+    from heimdall_amd import gdn_layer as gl
+    m = make_layer(dev, torch.bfloat16, 1, 2, 64, 72)
+    u = torch.randn(2, 1, 72, device=dev).bfloat16()
+    handle = m.in_proj_a.register_forward_hook(lambda *a: None)          # the same projections in both calls
+    ref = m(u, step_cache(dev, torch.bfloat16, 2, 1, 2, 64))
+    if how == "hook":
+        m.norm.register_forward_hook(lambda mod, args, out: 2 * out)
+    elif how == "pre-hook":
+        m.norm.register_forward_pre_hook(lambda mod, args: (args[0], args[1] * 0))
+    elif how == "global hook":
+        handle = torch.nn.modules.module.register_module_forward_hook(
+            lambda mod, args, out: 2 * out if mod is m.norm else None)
+    else:
+        m.norm.forward = lambda x, z: 2 * gl.gated_norm(x, z, m.norm.weight, m.norm.eps)
+    try:
+        o = m(u, step_cache(dev, torch.bfloat16, 2, 1, 2, 64))
+    finally:
+        handle.remove()
+    if how == "pre-hook":                                  # a gate of zero: SiLU(0) = 0
+        assert ref.any() and not o.any()
+    else:
+        assert rel(o, 2 * ref) < 4e-3
+
+
 @pytest.mark.parametrize("n", [1, 5, 64, 700, 5000])
 def test_conv_blocks(dev, n):
     """Token blocks of 4 .. 64 (H = 32, D = 128: 5000 tokens are the first with 64-token blocks) over packed sequences
