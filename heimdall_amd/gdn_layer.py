@@ -150,10 +150,10 @@ class GatedDeltaNet(nn.Module):
         step = s0 is not None and t == 1
         inside = step and _gates_inside(self, x)
         a, bb = (None, None) if inside else (self.in_proj_a(x), self.in_proj_b(x))
+        zg = self.in_proj_z(x) if step else None
         if step:
-            zg = self.in_proj_z(x).reshape(b, -1)
             r = _layer_step(self, z.reshape(b, -1), x[:, 0] if inside else a.reshape(b, -1),
-                            None if inside else bb.reshape(b, -1), zg, prefix, s0)
+                            None if inside else bb.reshape(b, -1), zg.reshape(b, -1), prefix, s0)
             if r is None and inside:
                 a, bb = self.in_proj_a(x), self.in_proj_b(x)
             if r is not None:
@@ -166,7 +166,7 @@ class GatedDeltaNet(nn.Module):
         if cache is not None:
             full = z if prefix is None else torch.cat((prefix.to(z.dtype), z), 1)
             cache["conv"] = F.pad(full, (0, 0, max(0, k1 - full.size(1)), 0))[:, -k1:]
-        zg = self.in_proj_z(x).view(b, t, c.lin_hv, c.lin_dv)
+        zg = (zg if step else self.in_proj_z(x)).view(b, t, c.lin_hv, c.lin_dv)
         fused = not step and _fused_norm(q.dtype, c.lin_dv)
         if step:
             o, s = gdn_step(q, k, v, g, beta, s0)

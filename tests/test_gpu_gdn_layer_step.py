@@ -112,6 +112,22 @@ def test_step_calls_a_changed_norm(dev, how):
         assert rel(o, 2 * ref) < 4e-3
 
 
+def test_step_runs_each_projection_once(dev):
+    """Where the step call does not apply (here: another norm), as where it does, every projection runs once."""
+    from heimdall_amd import gdn_layer as gl
+
+    class Norm(gl.GatedNorm):
+        pass
+
+    for norm in (None, Norm(64)):
+        m = make_layer(dev, torch.bfloat16, 1, 2, 64, 72, norm)
+        calls = {}
+        for name in ("in_proj_qkv", "in_proj_z", "in_proj_a", "in_proj_b", "out_proj"):
+            getattr(m, name).register_forward_hook(lambda mod, args, out, name=name: calls.__setitem__(name, calls.get(name, 0) + 1))
+        m(torch.randn(2, 1, 72, device=dev).bfloat16(), step_cache(dev, torch.bfloat16, 2, 1, 2, 64))
+        assert len(calls) == 5 and set(calls.values()) == {1}, calls
+
+
 @pytest.mark.parametrize("n", [1, 5, 64, 700, 5000])
 def test_conv_blocks(dev, n):
     """Token blocks of 4 .. 64 (H = 32, D = 128: 5000 tokens are the first with 64-token blocks) over packed sequences
