@@ -732,10 +732,12 @@ static bool kv_aligned(const void* p, int64_t s1, int64_t s2) {
 
 // workspace of bf_layer_prefill_fwd: the GDN inputs and outputs for up to B T memory queries, o_mem, the new state
 // and the GDN workspace. The GDN part is laid out for B T tokens with the segment length chosen for B T tokens; the
-// inner call runs on at most B T tokens with that same segment length, and every buffer of the GDN layout grows
-// monotonically with the token count at a fixed segment length, so the reservation always suffices.
+// inner call runs on at most B T tokens with that same segment length, and every buffer of the GDN layout but its planes grows
+// monotonically with the token count at a fixed segment length, so the reservation always suffices for those. The planes come
+// last: where there is no room for the inner call's (a workspace of `need` bytes, or an outer count too large for them),
+// bf_gdn_fwd leaves the outputs in the scan. The fp32 o_mem of a few-token chunk lies in om and o_mem, which follow each other.
 struct LayerWs {
-    size_t wq, wk, wv, wg, wb, om, o_mem, few, s_new, part, gdn, total;
+    size_t wq, wk, wv, wg, wb, om, o_mem, s_new, part, gdn, need, total;
     int seg_chunks;
 };
 static LayerWs layer_ws(int B, int G, int R, int D, int T, int in_dtype) {
@@ -750,12 +752,12 @@ static LayerWs layer_ws(int B, int G, int R, int D, int T, int in_dtype) {
     put(w.wb, BT * G * 4);
     put(w.om, BT * H * D * esz);
     put(w.o_mem, BT * H * D * esz);
-    put(w.few, T <= bf::FEW_MAX_T ? BT * H * D * 4 : 0);      // o_mem of the few-token memory branch, fp32
     put(w.s_new, (size_t)B * G * D * D * 4);
     // the item map's slot count does not depend on the window or the position
     put(w.part, in_dtype == BF_DTYPE_BF16 ? bf::window_split_bytes(bf::window_map(B, G, R, T, 1, 0), D) : 0);
     const GdnLayout gl = gdn_layout((int64_t)B * T, B, G, R, D, in_dtype, 0);
     w.seg_chunks = gl.seg_chunks;
+    w.need = at + align256(gl.need);
     put(w.gdn, gl.total);
     w.total = at;
     return w;
@@ -786,7 +788,7 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
     const bool use_mem = memory && start + T > W;
     if (use_mem && (!z || !mix_lse || !mem_scale)) return BF_STATUS_INVALID;
     const LayerWs L = layer_ws(B, G, R, D, T, in_dtype);
-    if (!workspace || workspace_bytes < L.total || (reinterpret_cast<uintptr_t>(workspace) & 255))
+    if (!workspace || workspace_bytes < L.need || (reinterpret_cast<uintptr_t>(workspace) & 255))
         return BF_STATUS_WORKSPACE;
     char* ws = static_cast<char*>(workspace);
     const hipStream_t st = static_cast<hipStream_t>(stream);
@@ -808,7 +810,7 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
     // a few tokens over a cache: token by token on the state, in place (R <= 8 query heads per KV head)
     const bool few = use_mem && T <= bf::FEW_MAX_T && R <= 8;
     if (few) {
-        a.o_mem = ws + L.few;
+        a.o_mem = ws + L.om;
         if ((rc = bf::few_mem_dispatch(a, state_valid ? state : nullptr, st))) return rc;
         o_mem = a.o_mem;
         o_mem_dtype = BF_DTYPE_F32;
@@ -834,7 +836,7 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
         a.om = om;
         rc = bf_gdn_fwd(wq, wk, wv, wg, wb, nullptr, B, (int64_t)B * a.Tq, G, R, D, in_dtype, 1.f,
                         state_valid ? state : nullptr, om, in_dtype, reinterpret_cast<float*>(ws + L.s_new), L.seg_chunks,
-                        ws + L.gdn, L.total - L.gdn,
+                        ws + L.gdn, workspace_bytes - L.gdn,
                         BF_GDN_PHASE_ALL, stream);
         if (rc) return rc;
         if (!rows && (rc = bf::layer_launch(a, 1, st))) return rc;

@@ -29,6 +29,8 @@ def test_student_inputs_equal_separate_calls(dev, b, t, h, g, d, dm, out):
 
 
 # fp32: sums of D products and 16 state updates in fp32, ~1e-6; bf16: operands rounded to bf16 (2^-9 each)
+
+
 @pytest.mark.parametrize("dtype,tol", [(torch.float32, 1e-4), (torch.bfloat16, 2e-2)])
 @pytest.mark.parametrize("h,g,d,w", [(4, 2, 64, 8), (12, 2, 128, 16), (8, 1, 256, 24)])
 def test_short_chunks_match_oracle(dev, dtype, tol, h, g, d, w):
@@ -48,3 +50,38 @@ def test_short_chunks_match_oracle(dev, dtype, tol, h, g, d, w):
             assert rel(o, o_ref) < tol, (a, n, rel(o, o_ref))
             a += n
     compare_caches(c_ref, c_gpu, tol)
+
+
+@pytest.mark.parametrize("dtype,b,g,r,d,t", [(torch.float32, 1, 2, 2, 128, 300), (torch.float32, 2, 2, 3, 64, 5),
+                                             (torch.bfloat16, 2, 2, 3, 64, 3)])
+def test_workspace_of_the_plain_layout(dev, monkeypatch, dtype, b, g, r, d, t):
+    """bf_layer_prefill_fwd with a workspace that has no room for the fp32 scan's planes, nor for anything of its own in a short
+    chunk, against the full one: the same values (the scan's sums in another order, 1e-5; the short chunk's bits)."""
+    from heimdall_amd import _lib, hibrit
+    h, w = g * r, 16
+    al = lambda n: (n + 255) // 256 * 256
+    es = 2 if dtype == torch.bfloat16 else 4
+    n = _lib.ctypes.c_size_t(0)
+    _lib.check(_lib.load().bf_gdn_workspace_size(b * t, b, g, r, d, 1 if es == 2 else 0, 0, _lib.ctypes.byref(n)), "size")
+    planes = 2 * (b * t // 64 + b) * g * (d // 16) * (d // 32 + 2) * 1536 if es == 4 else 0
+    plain = sum(map(al, (b * t * h * d * es, b * t * g * d * es, b * t * g * d * es, b * t * g * 4, b * t * g * 4,
+                         b * t * h * d * es, b * t * h * d * es, b * g * d * d * 4))) + al(n.value - planes)
+    if es == 2:                                            # the window's key parts: 3 slots per XCD in 8 parts
+        plain += 8 * 3 * 8 * 128 * (d + 4) * 4
+    m = make_core(h, g, d, 32, window=w, sinks=2).to(dev)
+    args = to_dev(make_inputs(m, b, 40 + t, seed=6, dtype=dtype), dev)
+    c0, c1 = {}, {}
+    with torch.no_grad():
+        for c in (c0, c1):
+            hibrit.student(m, *split(args, 0, 40), 0, c)
+        ref = hibrit.student(m, *split(args, 40, 40 + t), 40, c0)
+        full, got = hibrit.workspace, []
+
+        def small(nbytes, dev_):
+            got.append(nbytes)
+            return full(min(nbytes, plain) if nbytes >= plain else nbytes, dev_)
+
+        monkeypatch.setattr(hibrit, "workspace", small)
+        o = hibrit.student(m, *split(args, 40, 40 + t), 40, c1)
+    assert any(x >= plain for x in got)
+    assert rel(o, ref) < 1e-5 and rel(c1["S"], c0["S"]) < 1e-5
