@@ -763,6 +763,11 @@ static LayerWs layer_ws(int B, int G, int R, int D, int T, int in_dtype) {
     return w;
 }
 
+int bf_layer_few_tokens(int R, int in_dtype) {
+    if (R <= 0) return BF_STATUS_INVALID;
+    return supported_dtype(in_dtype) ? bf::few_tokens(R, in_dtype) : BF_STATUS_UNSUPPORTED;
+}
+
 int bf_layer_prefill_workspace_size(int B, int G, int R, int D, int T, int in_dtype, size_t* bytes) {
     if (!bytes || B <= 0 || G <= 0 || R <= 0 || T <= 0) return BF_STATUS_INVALID;
     if (!supported_dim(D) || !supported_dtype(in_dtype)) return BF_STATUS_UNSUPPORTED;
@@ -807,8 +812,8 @@ int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, in
     int rc;
     const void* o_mem = nullptr;
     int o_mem_dtype = in_dtype;
-    // a few tokens over a cache: token by token on the state, in place (R <= 8 query heads per KV head)
-    const bool few = use_mem && T <= bf::FEW_MAX_T && R <= 8;
+    // a few tokens over a cache: token by token on the state, in place
+    const bool few = use_mem && T <= bf::few_tokens(R, in_dtype);
     if (few) {
         a.o_mem = ws + L.om;
         if ((rc = bf::few_mem_dispatch(a, state_valid ? state : nullptr, st))) return rc;

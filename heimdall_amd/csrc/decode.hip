@@ -611,12 +611,12 @@ __global__ __launch_bounds__(NT_DEC) void decode_tail_kernel(DecodeArgs a) {
     if (x == 0 && g == 0 && tid == 0 && (a.pos_arr || b == 0)) a.ring_pos[(a.pos_arr ? (long)b * W : 0L) + pos % W] = pos;
 }
 
-// The memory branch of a chunk of a few tokens over a cache (an MTP verification; T <= FEW_MAX_T): workgroup (x, g, b)
+// The memory branch of a chunk of a few tokens over a cache (an MTP verification; T <= few_tokens): workgroup (x, g, b)
 // holds 64 columns of the state in registers and takes the tokens in turn: the row of position p - W leaves the window
 // (a ring row if ring_pos holds that position, or a row of this chunk) and is written into the state, then the R query
 // heads read it. Each token costs two sums over the slab's rows (~2 us), where the chunked scan pays for 64 tokens,
 // five launches and bf16 copies of the stream: at T = 2, H = 24, G = 4, D = 256 this pass replaced stream, prep, scan
-// and state copy. Above 16 tokens the scan is the faster one.
+// and state copy (74 against 84 us a call; few_tokens has the other sizes).
 template <int D, int RM>
 __global__ __launch_bounds__(NT_DEC) void few_mem_kernel(LayerArgs a, const float* s_in) {
     constexpr int RSTEP = 256 / SCG, RPT = D / RSTEP;

@@ -276,7 +276,6 @@ def _decode(self, x, qr, kr, v, qm, km, g, beta, start, st, sink_k, sink_v, memo
 # G = 4, D = 256, W = 2048 + 4, a t = 2 chunk costs 207 us through the chunk kernels and 261 us as two decode steps,
 # whose time is mostly host launch gaps between their six library calls.
 SMALL_CHUNK = 1
-FEW_MAX_T = 16      # chunks of up to this many tokens take bf_layer_prefill_fwd's token-by-token memory branch (fp32)
 BATCH_KEYS = ("sink_k", "sink_v", "ring_k", "ring_v", "ring_km", "ring_g", "ring_beta", "ring_pos", "S")
 
 
@@ -469,7 +468,8 @@ def student(self, x, q, k, v, qr, kr, start: int, cache: Optional[dict], memory:
     if all(z.dtype == torch.bfloat16 for z in (q, k, qr, kr)):
         # fused: the gate projections, qm / km (bf16 for a chunk's scan, fp32 for the decode step and the few-token
         # memory branch), gates
-        odt = torch.bfloat16 if t > FEW_MAX_T else torch.float32
+        few_t = _lib.load().bf_layer_few_tokens(c.h // c.hkv, dtype_code(compute_dtype(qr, kr, v)))
+        odt = torch.float32 if t <= max(1, few_t) else torch.bfloat16
         few = _few_inputs(self, x, q, k, start, odt) if 1 < t and b * t <= _lib.STUDENT_INPUTS_MAX else None
         if few is not None:
             qm, km, g, beta, zmix = few

@@ -395,6 +395,8 @@ int bf_student_inputs(const void* x, int64_t x_st, const void* q, int64_t q_st, 
  * f32, lse [B][H][T] f32 or null. Workspace from bf_layer_prefill_workspace_size, 256-byte aligned; its last part may be left
  * out as bf_gdn_fwd's (N_tok = B T, num_seqs = B).
  */
+/* Chunks of up to this many tokens write and read the memory token by token in fp32, longer ones through bf_gdn_fwd. */
+int bf_layer_few_tokens(int R, int in_dtype);
 int bf_layer_prefill_workspace_size(int B, int G, int R, int D, int T, int in_dtype, size_t* bytes);
 int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t start, int memory, int in_dtype,
                          const void* qr, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* kr, int64_t k_sb,

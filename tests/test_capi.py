@@ -81,6 +81,14 @@ def test_limits_match_the_library(cpu_lib):
     assert cpu_lib.bf_student_inputs_max_tokens() == _lib.STUDENT_INPUTS_MAX
 
 
+def test_few_token_line(cpu_lib):
+    """Tokens up to which a chunk's memory branch runs token by token, by query heads per KV head."""
+    heads = (1, 2, 4, 5, 6, 8, 9)
+    assert [cpu_lib.bf_layer_few_tokens(r, 1) for r in heads] == [8, 8, 8, 4, 4, 4, 0]
+    assert [cpu_lib.bf_layer_few_tokens(r, 0) for r in heads] == [12] * 6 + [0]
+    assert cpu_lib.bf_layer_few_tokens(0, 1) == -1 and cpu_lib.bf_layer_few_tokens(1, 2) == -2
+
+
 def test_workspace_size_grows_with_tokens(cpu_lib):
     a, b = ctypes.c_size_t(0), ctypes.c_size_t(0)
     cpu_lib.bf_gdn_workspace_size(4096, 1, 4, 1, 256, 1, 0, ctypes.byref(a))
