@@ -236,14 +236,27 @@ inline size_t window_split_bytes(const WinMap& m, int D) {
     return (size_t)8 * window_split_x(m) * window_split_p(m) * 128 * (D + 4) * sizeof(float);
 }
 
-// Key parts for queries over a long history (start >= 64 keys per part: each item's key range is about start + T / 2), of
-// the slots past the last full round of an XCD. Unsplit they cost one more round of whole items however few they are;
-// as P parts each, ceil(rem P / 32) rounds of 1/P item plus the partial rows' write and merge. A 64-key block of an
-// item takes ~2.1 us and a part's rows (133 KB at D = 256) ~14 us written and merged. 2048 queries over 14336 earlier
-// keys, H = 24, G = 4, D = 256 (48 slots per XCD, 16 of them as halves): 1047 -> 855 us a call.
-inline int window_long_parts(const WinMap& m, int T, long start) {
+// Key parts for queries over a long history (each item's key range is about start + T / 2), of the slots past the last full
+// round of an XCD. Unsplit they cost one more round of whole items however few they are; as P parts each, ceil(rem P / 32)
+// rounds of 1/P item plus the partial rows' write and merge. A 64-key block of an item takes ~2.1 us and a part's rows (133 KB
+// at D = 256) ~14 us written and merged. 2048 queries over 14336 earlier keys, H = 24, G = 4, D = 256 (48 slots per XCD, 16 of
+// them as halves): 1047 -> 855 us a call.
+// Items of different lengths fill an odd number of full rounds unevenly: the map pairs short items with long ones, so the CUs
+// are free at different times, and the last round's items, the longer the earlier, take up the difference. With lengths from
+// `first` to first + span keys on the XCD of the longest, halves then save first / 2 keys and span (16 - rem) / per, and that
+// has to be 5 blocks at D = 256 and 4 at 128. At D = 256, whole / halves, T = 2048, per = 48: 99 / 107 us over 1 earlier key,
+// 115 / 120 over 300, 161 / 157 over 1000; T = 2816, per = 44: 114 / 117 over 1, 131 / 130 over 300; T = 7000, per = 112:
+// 447 / 465 over 1; T = 2304, per = 36: 99 / 84 over 1; G = 2 (an XCD has half a head's items), T = 6000, per = 48: 287 / 264
+// over 1. D = 128, T = 1500, per = 48: 87 / 91 over 300, 128 / 126 over 1000; T = 1400, per = 44: 85 / 81 over 350. After an even
+// number of rounds the CUs are free together (T = 5000, per = 80: 274 / 261 over 1; D = 128, T = 2330, per = 76: 167 / 145), and at
+// D = 64 parts gained at every length measured (T = 6000, per = 48: 181 / 141 over 1).
+inline int window_long_parts(const WinMap& m, int T, long start, int D) {
     const long rem = m.per % 32;
     const double nblk = (double)(start + T / 2) / 64.0;
+    if (D > 64 && m.per / 32 % 2) {
+        const long span = T < 128 * m.rpg ? T : 128 * m.rpg, first = start + T - span;
+        if (first / 128.0 + span * (16.0 - rem) / (64.0 * m.per) < (D > 128 ? 5.1 : 4.0)) return 1;
+    }
     double best = 0.95 * 2.1 * nblk;
     int parts = 1;
     for (int p = 2; rem && p <= 8 && nblk >= 8.0 * p; ++p) {
@@ -253,7 +266,7 @@ inline int window_long_parts(const WinMap& m, int T, long start) {
     return parts;
 }
 inline size_t window_long_bytes(const WinMap& m, int T, long start, int D) {
-    const int p = window_long_parts(m, T, start);
+    const int p = window_long_parts(m, T, start, D);
     return p > 1 ? (size_t)8 * (m.per % 32) * p * 128 * (D + 4) * sizeof(float) : 0;
 }
 

@@ -529,7 +529,7 @@ static int window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64
     a.o = o; a.lse = lse;
     if (part && in_dtype == BF_DTYPE_BF16) {
         const bf::WinMap wm = bf::window_map(B, G, R, T, W, start);
-        a.split_p = long_parts ? bf::window_long_parts(wm, T, start) : bf::window_split_p(wm);
+        a.split_p = long_parts ? bf::window_long_parts(wm, T, start, D) : bf::window_split_p(wm);
         a.split_x = !long_parts ? bf::window_split_x(wm) : a.split_p > 1 ? (int)(wm.per % 32) : 0;
         a.part = part;
     }

@@ -51,3 +51,16 @@ def test_prefix_workspace_arguments():
     assert size(1, 4, 6, 96, 2048, 24576, 64, 1, ctypes.byref(n)) == -2
     assert size(1, 4, 6, 256, 2048, 2048, 1, 1, ctypes.byref(n)) == -1                            # start + T > cap
     assert lib.bf_prefix_attention(1, 4, 6, 256, 2048, 24576, 14336, 1, 256, 0, 0, 0, 256, 256, 256, 256, 1, None, 0, None) == -3
+
+
+def test_short_histories_stay_whole():
+    """After an odd number of full rounds, a last round of 12 or 16 slots is split only where the items' shortest keys pay for
+    the parts' rows; a launch of one round, one after an even number, a last round of few slots, and D = 64 are split as before."""
+    for H, G, D, T, start, parts in ((24, 4, 256, 2048, 1, False), (24, 4, 256, 2048, 300, False), (24, 4, 256, 2048, 1000, True),
+                                     (24, 4, 256, 4600, 1, False), (24, 4, 256, 4600, 1150, True), (16, 4, 256, 3000, 1, False),
+                                     (16, 4, 256, 7000, 1, False), (16, 4, 256, 2816, 1, False), (16, 4, 256, 2816, 704, True),
+                                     (32, 8, 128, 1500, 300, False), (32, 8, 128, 1500, 1000, True), (32, 8, 128, 1400, 350, True),
+                                     (32, 8, 128, 2330, 1, True), (16, 4, 256, 5000, 1, True), (8, 2, 256, 6000, 1, True),
+                                     (8, 2, 256, 2048, 1, True), (16, 4, 256, 2304, 1, True), (24, 4, 256, 2800, 1, True),
+                                     (8, 2, 64, 6000, 1, True)):
+        assert (_parts(1, G, H // G, D, T, start + T + 256, start) > 0) == parts, (H, G, D, T, start)
