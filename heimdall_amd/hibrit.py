@@ -475,7 +475,7 @@ def student(self, x, q, k, v, qr, kr, start: int, cache: Optional[dict], memory:
             qm, km, g, beta, zmix = few
         else:
             ab, zmix = _gate_logits(self, x)
-            qm, km, g, beta = _mem_inputs_bf16(self, ab, q, k, start, torch.bfloat16 if t > 1 else torch.float32)
+            qm, km, g, beta = _mem_inputs_bf16(self, ab, q, k, start, odt)
     else:
         qm, km, g, beta = self._mem_inputs(x, q, k, torch.arange(start, start + t, device=dev))
     if "ring_k" not in st:

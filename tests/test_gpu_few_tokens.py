@@ -86,3 +86,19 @@ def test_workspace_of_the_plain_layout(dev, monkeypatch, dtype, b, g, r, d, t):
         o = hibrit.student(m, *split(args, 40, 40 + t), 40, c1)
     assert any(x >= plain for x in got)
     assert rel(o, ref) < 1e-5 and rel(c1["S"], c0["S"]) < 1e-5
+
+
+@pytest.mark.parametrize("h,g,b", [(4, 2, 65), (8, 1, 66)])
+def test_memory_inputs_do_not_depend_on_the_batch(dev, h, g, b):
+    """Short chunks whose memory inputs come from the separate calls (more than 256 tokens in all) keep them in fp32 for the
+    ring, as the fused call does."""
+    from heimdall_amd import hibrit
+    t, d, w = 4, 64, 8
+    m = make_core(h, g, d, 32, window=w, sinks=2).to(dev)
+    x, q, k, v, qr, kr = to_dev(make_inputs(m, b, t, seed=5, dtype=torch.bfloat16), dev)
+    c = {}
+    with torch.no_grad():
+        hibrit.student(m, x, q, k, v, qr, kr, 0, c)
+        km = hibrit._project_bf16(k, m.fk, 1.0, torch.float32)
+    slot = torch.arange(t, device=dev) % w
+    assert torch.equal(c["ring_km"][:, slot], km)
