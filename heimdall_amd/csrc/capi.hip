@@ -561,7 +561,7 @@ int bf_prefix_attention(int B, int G, int R, int D, int T, int cap, int64_t star
     const int st = bf_prefix_attention_workspace_size(B, G, R, D, T, cap, start, dtype, &need);
     if (st) return st;
     if (!k || !v || !pos) return BF_STATUS_INVALID;
-    if (need && (!workspace || workspace_bytes < need)) return BF_STATUS_WORKSPACE;
+    if (need && (!workspace || workspace_bytes < need || ((uintptr_t)workspace & 15))) return BF_STATUS_WORKSPACE;
     const size_t off = (size_t)start * D * (dtype == BF_DTYPE_BF16 ? 2 : 4);
     const int64_t sg = (int64_t)cap * D, sb = G * sg;
     return window_fwd(B, G, R, D, T, cap, 0, start, dtype, q, q_sb, q_sh, q_st, static_cast<const char*>(k) + off, sb, sg, D,

@@ -51,6 +51,9 @@ def test_prefix_workspace_arguments():
     assert size(1, 4, 6, 96, 2048, 24576, 64, 1, ctypes.byref(n)) == -2
     assert size(1, 4, 6, 256, 2048, 2048, 1, 1, ctypes.byref(n)) == -1                            # start + T > cap
     assert lib.bf_prefix_attention(1, 4, 6, 256, 2048, 24576, 14336, 1, 256, 0, 0, 0, 256, 256, 256, 256, 1, None, 0, None) == -3
+    # partial rows are written with 16-byte stores
+    assert size(1, 4, 6, 256, 2048, 24576, 14336, 1, ctypes.byref(n)) == 0 and n.value > 0
+    assert lib.bf_prefix_attention(1, 4, 6, 256, 2048, 24576, 14336, 1, 256, 0, 0, 0, 256, 256, 256, 256, 1, 264, n.value, None) == -3
 
 
 def test_short_histories_stay_whole():
