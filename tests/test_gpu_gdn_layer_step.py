@@ -85,6 +85,22 @@ def step_cache(dev, dtype, b, hk, hv, d):
                 S=torch.randn(b, hv, d, d, device=dev, generator=gen) * 0.1)
 
 
+@pytest.mark.parametrize("b,d,inside", [(64, 128, True), (65, 128, False), (64, 64, True), (3, 256, False)])
+def test_where_the_gates_are_formed(dev, b, d, inside):
+    """The last batch with the gate logits in the step kernel, the first without, and D = 256, which never has them; each equals
+    the same step with its projections called (bf16, tolerance as above)."""
+    from heimdall_amd import gdn_layer as gl
+    print(f"gates B={b} D={d}", flush=True)
+    m = make_layer(dev, torch.bfloat16, 1, 2, d, 264)
+    u = torch.randn(b, 1, 264, device=dev).bfloat16()
+    assert gl._gates_inside(m, u) == inside
+    c0, c1 = (step_cache(dev, torch.bfloat16, b, 1, 2, d) for _ in range(2))
+    o = m(u, c0)
+    m.in_proj_b.register_forward_hook(lambda *a: None)
+    ref = m(u, c1)
+    assert rel(o, ref) < 4e-3 and rel(c0["S"], c1["S"]) < 4e-3 and torch.equal(c0["conv"], c1["conv"])
+
+
 @pytest.mark.parametrize("how", ["hook", "pre-hook", "global hook", "instance"])
 def test_step_calls_a_changed_norm(dev, how):
     """A norm with hooks or a forward of its own is called: its doubled output doubles the layer's (bf16, tolerance as above)."""
@@ -128,10 +144,10 @@ def test_step_runs_each_projection_once(dev):
         assert len(calls) == 5 and set(calls.values()) == {1}, calls
 
 
-@pytest.mark.parametrize("n", [1, 5, 64, 700, 5000])
+@pytest.mark.parametrize("n", [1, 5, 64, 700, 1400, 5000, 5440, 5441])
 def test_conv_blocks(dev, n):
-    """Token blocks of 4 .. 64 (H = 32, D = 128: 5000 tokens are the first with 64-token blocks) over packed sequences
-    give the same bits as one token at a time with the rows before it as its prefix."""
+    """Token blocks of 4, 8, 16, 32 and 64 (H = 32, D = 128: from 681, 1361, 2721 and 5441 tokens on) over packed sequences give
+    the same bits as one token at a time with the rows before it as its prefix."""
     from heimdall_amd import gdn_layer as gl
     hk = hv = 32
     d, K = 128, 4

@@ -56,3 +56,36 @@ def test_fp32_outputs(dev, lens, G, R, D, s0, out_dtype):
                 assert err < tol, (seg, i, err)
             if rs.norm() > 0:
                 assert (sf[i].cpu().double() - rs).norm() / rs.norm() < 2e-6, (seg, i)
+
+
+@pytest.mark.parametrize("lens,G,R,D", [([1], 1, 2, 64), ([129, 0, 63], 2, 3, 128), ([300, 31], 1, 2, 256), ([200], 2, 1, 128)])
+def test_fp32_outputs_in_the_scan(dev, lens, G, R, D):
+    """A workspace without room for the planes keeps the outputs in the scan (fp32 MFMAs): the same values, same tolerance."""
+    from heimdall_amd import _lib
+    gen = torch.Generator().manual_seed(sum(lens) + D)
+    N, B, H = sum(lens), len(lens), G * R
+    print(f"fp32 outputs in the scan lens={lens} G={G} R={R} D={D}", flush=True)
+    q, k = torch.randn(N, G, R, D, generator=gen), F.normalize(torch.randn(N, G, D, generator=gen), dim=-1)
+    v, g = torch.randn(N, G, D, generator=gen), -0.05 * torch.rand(N, G, generator=gen)
+    beta, s = torch.sigmoid(torch.randn(N, G, generator=gen)), torch.randn(B, G, D, D, generator=gen)
+    cu = torch.tensor([0] + lens).cumsum(0).to(torch.int32)
+    lib, n = _lib.load(), _lib.ctypes.c_size_t(0)
+    dq, dk, dv, dg, db, ds, dcu = (x.to(dev).contiguous() for x in (q, k, v, g, beta, s, cu))
+    for seg in (0, 1):
+        _lib.check(lib.bf_gdn_workspace_size(N, B, G, R, D, 0, seg, _lib.ctypes.byref(n)), "size")
+        ws = torch.empty(n.value, dtype=torch.uint8, device=dev)
+        outs = []
+        for short in (0, 1):
+            o, sf = torch.empty(N, H, D, device=dev), torch.empty(B, G, D, D, device=dev)
+            _lib.check(lib.bf_gdn_fwd(dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), dg.data_ptr(), db.data_ptr(), dcu.data_ptr(),
+                                      B, N, G, R, D, 0, 1.0, ds.data_ptr(), o.data_ptr(), 0, sf.data_ptr(), seg, ws.data_ptr(),
+                                      n.value - short, 15, torch.cuda.current_stream().cuda_stream), "bf_gdn_fwd")
+            outs.append(o)
+            for i in range(B):
+                a, e = int(cu[i]), int(cu[i + 1])
+                ro, rs = recurrence(*(x[a:e].double() for x in (q, k, v, g, beta)), s[i].double())
+                if e > a:
+                    err = (o[a:e].cpu().double().reshape(ro.shape) - ro).norm() / ro.norm()
+                    assert err < 2e-6, (seg, short, i, err)
+                assert (sf[i].cpu().double() - rs).norm() / rs.norm() < 2e-6, (seg, short, i)
+        assert N < 64 or not torch.equal(*outs)           # two routes
