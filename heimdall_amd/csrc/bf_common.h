@@ -186,35 +186,6 @@ __device__ __forceinline__ void store4<BF16>(uint16_t* p, float a, float b, floa
     *reinterpret_cast<uint2*>(p) = v;
 }
 
-// Transpose a VEC x VEC block held as VEC 16-byte row vectors (rows[i] = row i) into column vectors.
-template <class E>
-__device__ __forceinline__ void transpose_block(uint4 (&r)[E::VEC]);
-template <>
-__device__ __forceinline__ void transpose_block<F32>(uint4 (&r)[4]) {
-    uint32_t m[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) { m[i][0] = r[i].x; m[i][1] = r[i].y; m[i][2] = r[i].z; m[i][3] = r[i].w; }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = make_uint4(m[0][j], m[1][j], m[2][j], m[3][j]);
-}
-template <>
-__device__ __forceinline__ void transpose_block<BF16>(uint4 (&r)[8]) {
-    uint16_t m[8][8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const uint32_t w[4] = {r[i].x, r[i].y, r[i].z, r[i].w};
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { m[i][2 * j] = (uint16_t)(w[j] & 0xffffu); m[i][2 * j + 1] = (uint16_t)(w[j] >> 16); }
-    }
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        uint32_t w[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) w[i] = (uint32_t)m[2 * i][j] | ((uint32_t)m[2 * i + 1][j] << 16);
-        r[j] = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-}
-
 // s_waitcnt vmcnt(0): all outstanding vector-memory operations of the wave have completed. Used before a loop whose
 // first iteration consumes loads issued ahead of it, so the compiler's wait analysis at the loop header starts clean.
 __device__ __forceinline__ void wait_vmem_all() { __builtin_amdgcn_s_waitcnt(0x0F70); }

@@ -202,7 +202,7 @@ struct WinArgs {
     int split_x;              // bf16 kernel: slots per XCD split into key parts (window_split_x), 0: none
     int split_p;              // key parts per split slot (window_split_p)
     float* part;              // their partial rows [8 split_x][split_p][128][D + 4] (m, l, -, -, unnormalised o)
-    WinMap map;               // bf16 kernel: set by its launcher from window_map
+    WinMap map;               // set by the kernel's launcher (bf16: window_map)
 };
 
 // The bf16 window kernel's item map for B sequences of T queries, G KV heads of R query heads each, window W from
