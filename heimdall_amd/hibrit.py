@@ -468,8 +468,8 @@ def student(self, x, q, k, v, qr, kr, start: int, cache: Optional[dict], memory:
     if all(z.dtype == torch.bfloat16 for z in (q, k, qr, kr)):
         # fused: the gate projections, qm / km (bf16 for a chunk's scan, fp32 for the decode step and the few-token
         # memory branch), gates
-        few_t = _lib.load().bf_layer_few_tokens(c.h // c.hkv, dtype_code(compute_dtype(qr, kr, v)))
-        odt = torch.float32 if t <= max(1, few_t) else torch.bfloat16
+        few_t = _lib.FEW_TOKENS[_lib.DTYPE_BF16 if v.dtype == torch.bfloat16 else _lib.DTYPE_F32][c.h // c.hkv - 1:c.h // c.hkv]
+        odt = torch.float32 if t == 1 or few_t and t <= few_t[0] else torch.bfloat16
         few = _few_inputs(self, x, q, k, start, odt) if 1 < t and b * t <= _lib.STUDENT_INPUTS_MAX else None
         if few is not None:
             qm, km, g, beta, zmix = few

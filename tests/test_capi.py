@@ -83,9 +83,9 @@ def test_limits_match_the_library(cpu_lib):
 
 def test_few_token_line(cpu_lib):
     """Tokens up to which a chunk's memory branch runs token by token, by query heads per KV head."""
-    heads = (1, 2, 4, 5, 6, 8, 9)
-    assert [cpu_lib.bf_layer_few_tokens(r, 1) for r in heads] == [8, 8, 8, 4, 4, 4, 0]
-    assert [cpu_lib.bf_layer_few_tokens(r, 0) for r in heads] == [12] * 6 + [0]
+    from heimdall_amd import _lib
+    for dtype, line in _lib.FEW_TOKENS.items():
+        assert [cpu_lib.bf_layer_few_tokens(r, dtype) for r in range(1, 12)] == list(line) + [0] * 3
     assert cpu_lib.bf_layer_few_tokens(0, 1) == -1 and cpu_lib.bf_layer_few_tokens(1, 2) == -2
 
 
