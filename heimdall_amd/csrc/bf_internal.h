@@ -58,8 +58,10 @@ struct GdnArgs {
 
 // fp32 scans write every chunk's entry state and v_new, and the query heads' outputs are products over all chunks at once
 // (gdn_out_kernel), while those planes stay under 2 GiB. 8192 tokens, G = 4, R = 6, D = 256, forward: the scan with outputs
-// 751 us, its states 118 (87 on planes) and the outputs 296. One head per KV head gains too from D = 128 on (1 x 8192 tokens,
-// H = 4, D = 256: 552 -> 427 us; 3 x 3000, H = 4, D = 128: 201 -> 151), not at D = 64 (1 x 5000, H = 16: 126 -> 130).
+// 751 us, its states 118 (92 on planes) and the outputs 309. One head per KV head gains too from D = 128 on (1 x 8192 tokens,
+// H = 4, D = 256: 552 -> 427 us; 3 x 3000, H = 4, D = 128: 201 -> 151). At D = 64 it does at some sizes and not at others, in the
+// scan / at once: 1 x 64, H = 2: 28 / 32; 1 x 300, H = 16: 46 / 41; 1 x 3000, H = 16: 84 / 87; 1 x 5000, H = 16: 125 / 132; 3 x 10000,
+// H = 16: 915 / 832; there the scan keeps them.
 inline size_t gdn_plane_elems(long max_chunks, int G, int D) { return (size_t)max_chunks * G * (D / 16) * (D / 32 + 2) * 1536; }
 inline bool gdn_out_split(long max_chunks, int G, int R, int D, int in_dtype) {
     return in_dtype == DT_F32 && (R >= 2 || D >= 128) && 2 * gdn_plane_elems(max_chunks, G, D) <= (size_t)2 << 30;
@@ -356,7 +358,9 @@ int mem_project_dispatch(const MemProjArgs& a, hipStream_t stream);
 inline size_t mem_project32_bytes(int nh, int D) { return (size_t)nh * D * D * 6; }
 int mem_project32_dispatch(const MemProjArgs& a, uint16_t* planes, hipStream_t stream);
 
-// The memory inputs of a few tokens (student_front). Above FRONT_MAX_TOK the tiled kernels are the faster ones.
+// The memory inputs of a few tokens (student_front). A layer call with the tiled kernels' five launches / with these two, H = 24,
+// G = 4, D = 256: 64 tokens 106 / 91 us, 256 160 / 152, 400 190 / 188, 768 231 / 239; H = 32, G = 8, D = 128: 128 tokens 108 / 91, 256
+// 124 / 121, 384 144 / 144, 512 148 / 154: they cost the same at about 400 tokens.
 constexpr long FRONT_MAX_TOK = 256;
 struct FrontArgs {
     GateProjArgs gp;                // x, W, the split partials (part), n_tok; out0 / out1 unused

@@ -75,7 +75,7 @@ struct BgArgs {
 // 80 bytes: the 16 rows of a fragment hit distinct banks; a fragment is one 16-byte read), the other [k][row] (pitch an odd
 // multiple of 32 bytes; a fragment is two transposing reads). One LDS tile (46 KB at most, three workgroups per CU, which
 // fill each other's waits): the next step's loads are in flight while this one multiplies.
-// 8192 tokens, G = 4, R = 6, D = 256, forward and backward: 3102 -> 2958 us.
+// 8192 tokens, G = 4, R = 6, D = 256, forward and backward: 3102 -> 2958 us when these products went to planes.
 // EX: the epilogue extras compiled in: 0 none, 1 msc and rdo, 2 also dgc and cdo. The plain products measurably need
 // the small epilogue, and the row-scaled ones one without the per-element decay.
 template <bool AK, bool BK, int BN, int EX>

@@ -1166,7 +1166,7 @@ __attribute__((amdgpu_waves_per_eu(combine_waves<D>() / 4, combine_waves<D>() / 
 // K rows stay in their own order, since K^T is read through transposing reads of 16 consecutive dims: an A fragment of
 // K is two 8-byte reads, dims 4 lg .. and 16 + 4 lg .. of the step. The 16-byte blocks of a row are permuted by
 // 2 (row & 7) | (row >> 3 & 1): 16 rows of an 8-byte read, and 8 rows x 32 bytes of a transposing one, fall into distinct
-// banks. 8192 tokens, G = 4, R = 6, D = 256: the summary 188 -> 127 us, the states 118 -> 87.
+// banks. 8192 tokens, G = 4, R = 6, D = 256: the summary 188 -> 131 us, the states 118 -> 92.
 template <int D, bool OUT>
 __global__ __launch_bounds__((SegCfg<F32, D, OUT>::NW * 64)) void gdn_seg32_kernel(GdnArgs a) {
     using Cfg = SegCfg<F32, D, OUT>;

@@ -17,7 +17,8 @@
 // those of K_i, so each needs one tile, two barriers a block and half the registers: a piece of K is loaded where one of V was stored. Scores are
 // computed transposed (S^T = K Q^T) so each lane's softmax statistics belong to its own query column, and P feeds the P V
 // product straight from registers.
-// 4096 tokens, H = 16, G = 4, D = 256, W = 2048 + 4: 1765 us with fp32 MFMAs, now 750 us (window kernel alone).
+// 4096 tokens, H = 16, G = 4, D = 256, W = 2048 + 4: 1765 us with fp32 MFMAs, now 785 us (window kernel alone; 750 with a split
+// that cut the first plane off and made infinities NaN).
 #include "bf_common.h"
 #include "bf_internal.h"
 

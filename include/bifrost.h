@@ -79,7 +79,8 @@ const char* bf_status_string(int status);
  *     depend on it beyond rounding.
  *   phases: BF_GDN_PHASE_ALL, or PREP, SUMMARY, COMBINE, OUTPUT in separate calls (in that order) with the same
  *     arguments and workspace.
- * Chunk length is 64. Arithmetic: MFMA in in_dtype with fp32 accumulation; state, decay and the triangular
+ * Chunk length is 64. Arithmetic: MFMA in in_dtype with fp32 accumulation (in fp32 the larger products as bf16 MFMAs over three
+ * planes per operand, a product to within 3 * 2^-24; an infinite input ends as NaN); state, decay and the triangular
  * inverse in fp32; segment entry states composed in fp32 (split-bf16 MFMA for bf16 runs).
  * Workspace: bf_gdn_workspace_size bytes. For in_dtype fp32 with R >= 2 or D >= 128 its last part, unless that is over 2 GiB,
  *   is 2 (N_tok / 64 + num_seqs) G (D / 16) (D / 32 + 2) 1536 bytes, rounded up to 256, of bf16 planes: with them the outputs of
@@ -214,7 +215,8 @@ int bf_decode_fwd_noalloc(int B, int G, int R, int D, int W, int sinks, int64_t 
  * k and v over the G KV heads (e.g. q [B][H][T][D] -> strides (H*T*D, T*D, D); v [B][T][G][D] -> (T*G*D, D, G*D)).
  * ring_k/ring_v [B][G][W][D], ring_pos [W] int64, sink_k/sink_v [B][G][n_sinks][D], all in in_dtype.
  * o_mem [B][T][H][D] in o_mem_dtype (fp32 or bf16), z [B][T][H] f32, mix_lse/mem_scale [H] f32; o [B][T][H][D] in o_dtype; lse [B][H][T] f32 or
- * null. Arithmetic: MFMA in in_dtype (bf16 probabilities for bf16 inputs) with fp32 accumulation and softmax.
+ * null. Arithmetic: MFMA in in_dtype (bf16 probabilities for bf16 inputs) with fp32 accumulation and softmax; in fp32 the products
+ * as bf_mem_project_f32's.
  */
 int bf_window_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t start, int in_dtype, const void* q,
                   int64_t q_sb, int64_t q_sh, int64_t q_st, const void* k, int64_t k_sb, int64_t k_sh, int64_t k_st,
@@ -253,6 +255,8 @@ int bf_mem_project(const void* x, int64_t n_tok, int nh, int D, int64_t x_st, in
 
 /*
  * The same for fp32 rows, with no operand rounded: x, f, out fp32 (x and out 16-byte aligned, x_st and x_sh multiples of 4).
+ * Products are formed from three bf16 planes per operand, to within 3 * 2^-24 of each (fewer bits for operands below 2^-109 in
+ * size); an infinite operand gives what it gives in fp32 where the other one is at most 2^8 in size, NaN may follow past that.
  * Workspace: bf_mem_project_f32_workspace_size bytes, 16-byte aligned.
  */
 int bf_mem_project_f32_workspace_size(int nh, int D, size_t* bytes);
