@@ -58,6 +58,19 @@ def workspace(nbytes: int, dev: torch.device) -> torch.Tensor:
     return torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=dev)
 
 
+def workspace_or_min(nbytes: int, size_fn, args, dev: torch.device) -> torch.Tensor:
+    """``workspace(nbytes)``; where memory does not reach, the smallest workspace that the call accepts (``size_fn(*args)``, the
+    library's ``_min_size`` function), with which it takes a slower route."""
+    try:
+        return workspace(nbytes, dev)
+    except torch.OutOfMemoryError:
+        least = _lib.ctypes.c_size_t(0)
+        check(size_fn(*args, _lib.ctypes.byref(least)), size_fn.__name__)
+        if least.value >= nbytes:
+            raise
+    return workspace(least.value, dev)
+
+
 def gdn_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tensor, beta: torch.Tensor, *,
                 num_seqs: int, cu_seqlens: Optional[torch.Tensor] = None, initial_state: Optional[torch.Tensor] = None,
                 scale: float = 1.0, out_dtype: torch.dtype = torch.float32, phases: int = _lib.PHASE_ALL,
@@ -99,10 +112,10 @@ def gdn_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, g: torch.Tens
             raise BifrostError(f"initial_state must be [{num_seqs}, {G}, {D}, {D}], got {tuple(s0.shape)}")
     lib = _lib.load()
     nbytes = _lib.ctypes.c_size_t(0)
-    check(lib.bf_gdn_workspace_size(N, num_seqs, G, R, D, dtype_code(cdt), int(segment_chunks),
-                                    _lib.ctypes.byref(nbytes)), "bf_gdn_workspace_size")
+    size_args = (N, num_seqs, G, R, D, dtype_code(cdt), int(segment_chunks))
+    check(lib.bf_gdn_workspace_size(*size_args, _lib.ctypes.byref(nbytes)), "bf_gdn_workspace_size")
     if ws is None or ws.numel() < nbytes.value:
-        ws = workspace(nbytes.value, dev)
+        ws = workspace_or_min(nbytes.value, lib.bf_gdn_workspace_min_size, size_args, dev)
     if gated_norm is not None:
         gz, gw, geps = gated_norm
         if cdt != torch.bfloat16 or D > 128 or gz.dtype != torch.bfloat16 or gz.numel() != N * H * D:

@@ -23,6 +23,8 @@ SIGNATURES = {
     "bf_gdn_segment_chunks": (_c_int, [_c_i64, _c_int, _c_int, _c_int, _c_int]),
     "bf_gdn_workspace_size": (_c_int, [_c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                        ctypes.POINTER(_c_sz)]),
+    "bf_gdn_workspace_min_size": (_c_int, [_c_i64, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                           ctypes.POINTER(_c_sz)]),
     "bf_gdn_fwd": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _c_int, _c_i64, _c_int, _c_int, _c_int, _c_int, _fp, _vp,
                             _vp, _c_int, _vp, _c_int, _vp, _c_sz, _c_int, _vp]),
     "bf_gdn_step": (_c_int, [_vp] * 8 + [_c_int] * 4 + [_vp]),
@@ -63,6 +65,7 @@ SIGNATURES = {
     "bf_gdn_bwd": (_c_int, [_vp] * 6 + [_fp, _vp, _vp, _c_int, _c_i64, _c_int, _c_int, _c_int] + [_vp] * 7
                    + [_c_sz, _vp]),
     "bf_layer_few_tokens": (_c_int, [_c_int, _c_int]),
+    "bf_layer_prefill_workspace_min_size": (_c_int, [_c_int] * 6 + [ctypes.POINTER(_c_sz)]),
     "bf_layer_prefill_workspace_size": (_c_int, [_c_int] * 6 + [ctypes.POINTER(_c_sz)]),
     "bf_layer_prefill_fwd": (_c_int, [_c_int] * 7 + [_c_i64, _c_int, _c_int] + ([_vp, _c_i64, _c_i64, _c_i64] * 3)
                              + [_vp, _c_int, _vp, _c_int] + [_vp] * 7 + [_c_int] + [_vp] * 7 + [_c_int]

@@ -138,6 +138,13 @@ int bf_gdn_workspace_size(int64_t total_tokens, int num_seqs, int G, int R, int 
     return BF_STATUS_OK;
 }
 
+int bf_gdn_workspace_min_size(int64_t total_tokens, int num_seqs, int G, int R, int D, int in_dtype,
+                              int segment_chunks, size_t* bytes) {
+    const int st = bf_gdn_workspace_size(total_tokens, num_seqs, G, R, D, in_dtype, segment_chunks, bytes);
+    if (st == BF_STATUS_OK) *bytes = gdn_layout(total_tokens, num_seqs, G, R, D, in_dtype, segment_chunks).need;
+    return st;
+}
+
 }  // extern "C"
 
 namespace {
@@ -773,6 +780,12 @@ int bf_layer_prefill_workspace_size(int B, int G, int R, int D, int T, int in_dt
     if (!supported_dim(D) || !supported_dtype(in_dtype)) return BF_STATUS_UNSUPPORTED;
     *bytes = layer_ws(B, G, R, D, T, in_dtype).total;
     return BF_STATUS_OK;
+}
+
+int bf_layer_prefill_workspace_min_size(int B, int G, int R, int D, int T, int in_dtype, size_t* bytes) {
+    const int st = bf_layer_prefill_workspace_size(B, G, R, D, T, in_dtype, bytes);
+    if (st == BF_STATUS_OK) *bytes = layer_ws(B, G, R, D, T, in_dtype).need;
+    return st;
 }
 
 int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t start, int memory, int in_dtype,

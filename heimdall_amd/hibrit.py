@@ -24,7 +24,7 @@ import torch.nn.functional as F
 
 from . import _lib
 from ._device import (BifrostError, check, compute_dtype, dtype_code, require_device, require_no_grad, stream_ptr,
-                      workspace)
+                      workspace, workspace_or_min)
 from .teacher import set_retrieval, teacher
 
 NEW = ("fq", "fk", "ab", "mix", "mix_lse", "mem_scale", "A_log", "dt_bias")
@@ -678,9 +678,9 @@ def _prefill(self, x, qr, kr, v, qm, km, g, beta, start, st, sink_k, sink_v, mem
     sv = sink_v.to(cdt).contiguous() if ns else None
     o = torch.empty(b, t, H, D, dtype=torch.float32, device=dev)
     nbytes = _lib.ctypes.c_size_t(0)
-    check(lib.bf_layer_prefill_workspace_size(b, G, r, D, t, dtype_code(cdt), _lib.ctypes.byref(nbytes)),
-          "bf_layer_prefill_workspace_size")
-    ws = workspace(nbytes.value, dev)
+    size_args = (b, G, r, D, t, dtype_code(cdt))
+    check(lib.bf_layer_prefill_workspace_size(*size_args, _lib.ctypes.byref(nbytes)), "bf_layer_prefill_workspace_size")
+    ws = workspace_or_min(nbytes.value, lib.bf_layer_prefill_workspace_min_size, size_args, dev)
     ptr = lambda t_: t_.data_ptr() if t_ is not None else None
     check(lib.bf_layer_prefill_fwd(
         b, G, r, D, t, w, self.sinks, start, int(memory), dtype_code(cdt),

@@ -84,14 +84,16 @@ const char* bf_status_string(int status);
  * inverse in fp32; segment entry states composed in fp32 (split-bf16 MFMA for bf16 runs).
  * Workspace: bf_gdn_workspace_size bytes. For in_dtype fp32 with R >= 2 or D >= 128 its last part, unless that is over 2 GiB,
  *   is 2 (N_tok / 64 + num_seqs) G (D / 16) (D / 32 + 2) 1536 bytes, rounded up to 256, of bf16 planes: with them the outputs of
- *   all chunks are formed at once after the scan. A workspace without that part is accepted too and keeps the outputs in the
- *   scan: the same values to rounding, more slowly.
+ *   all chunks are formed at once after the scan. A workspace without that part (bf_gdn_workspace_min_size bytes) is accepted
+ *   too and keeps the outputs in the scan: the same values to rounding, more slowly.
  */
 /* Segment length (64-token chunks) that bf_gdn_fwd uses when segment_chunks is 0, or a negative status. */
 int bf_gdn_segment_chunks(int64_t total_tokens, int num_seqs, int G, int R, int D);
 
 int bf_gdn_workspace_size(int64_t total_tokens, int num_seqs, int G, int R, int D, int in_dtype,
                           int segment_chunks, size_t* bytes);
+int bf_gdn_workspace_min_size(int64_t total_tokens, int num_seqs, int G, int R, int D, int in_dtype,
+                              int segment_chunks, size_t* bytes);
 
 int bf_gdn_fwd(const void* q, const void* k, const void* v, const float* g, const float* beta,
                const int32_t* cu_seqlens, int num_seqs, int64_t total_tokens, int G, int R, int D, int in_dtype,
@@ -396,12 +398,13 @@ int bf_student_inputs(const void* x, int64_t x_st, const void* q, int64_t q_st, 
  * [B][T][G] f32; z [B][T][H] f32 (mix logits); mix_lse, mem_scale [H]; sink_k / sink_v [B][G][n_sinks][D] already
  * holding this chunk's sinks; ring_k / ring_v [B][G][W][D] in in_dtype, ring_km [B][W][G][D], ring_g / ring_beta
  * [B][W][G], ring_pos [W], state [B][G][D][D] f32 (state_valid 0: no state yet) — all updated in place. o [B][T][H][D]
- * f32, lse [B][H][T] f32 or null. Workspace from bf_layer_prefill_workspace_size, 256-byte aligned; its last part may be left
- * out as bf_gdn_fwd's (N_tok = B T, num_seqs = B).
+ * f32, lse [B][H][T] f32 or null. Workspace from bf_layer_prefill_workspace_size, 256-byte aligned, or from
+ * bf_layer_prefill_workspace_min_size without its last part, as bf_gdn_fwd's (N_tok = B T, num_seqs = B).
  */
 /* Chunks of up to this many tokens write and read the memory token by token in fp32, longer ones through bf_gdn_fwd. */
 int bf_layer_few_tokens(int R, int in_dtype);
 int bf_layer_prefill_workspace_size(int B, int G, int R, int D, int T, int in_dtype, size_t* bytes);
+int bf_layer_prefill_workspace_min_size(int B, int G, int R, int D, int T, int in_dtype, size_t* bytes);
 int bf_layer_prefill_fwd(int B, int G, int R, int D, int T, int W, int sinks, int64_t start, int memory, int in_dtype,
                          const void* qr, int64_t q_sb, int64_t q_sh, int64_t q_st, const void* kr, int64_t k_sb,
                          int64_t k_sh, int64_t k_st, const void* v, int64_t v_sb, int64_t v_sh, int64_t v_st,

@@ -76,13 +76,13 @@ def test_workspace_of_the_plain_layout(dev, monkeypatch, dtype, b, g, r, d, t):
         for c in (c0, c1):
             hibrit.student(m, *split(args, 0, 40), 0, c)
         ref = hibrit.student(m, *split(args, 40, 40 + t), 40, c0)
-        full, got = hibrit.workspace, []
+        got = []
 
-        def small(nbytes, dev_):
+        def small(nbytes, size_fn, size_args, dev_):
             got.append(nbytes)
-            return full(min(nbytes, plain) if nbytes >= plain else nbytes, dev_)
+            return hibrit.workspace(plain, dev_)
 
-        monkeypatch.setattr(hibrit, "workspace", small)
+        monkeypatch.setattr(hibrit, "workspace_or_min", small)
         o = hibrit.student(m, *split(args, 40, 40 + t), 40, c1)
     assert any(x >= plain for x in got)
     assert rel(o, ref) < 1e-5 and rel(c1["S"], c0["S"]) < 1e-5

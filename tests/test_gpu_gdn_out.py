@@ -89,3 +89,31 @@ def test_fp32_outputs_in_the_scan(dev, lens, G, R, D):
                     assert err < 2e-6, (seg, short, i, err)
                 assert (sf[i].cpu().double() - rs).norm() / rs.norm() < 2e-6, (seg, short, i)
         assert N < 64 or not torch.equal(*outs)           # two routes
+
+
+def test_planes_without_memory(dev, monkeypatch):
+    """Where memory does not reach for the planes, the calls take the smallest workspace and its route; bf16 runs have no
+    smaller one and raise."""
+    from heimdall_amd import _device
+    gen = torch.Generator().manual_seed(3)
+    N, G, R, D = 150, 2, 2, 64
+    q, k = torch.randn(N, G * R, D, generator=gen), F.normalize(torch.randn(N, G, D, generator=gen), dim=-1)
+    v, g, beta = torch.randn(N, G, D, generator=gen), -0.05 * torch.rand(N, G, generator=gen), torch.rand(N, G, generator=gen)
+    args = [x.to(dev) for x in (q, k, v, g, beta)]
+    ref = _device.gdn_forward(*args, num_seqs=1)
+    plain, asked = _device.workspace, []
+
+    def full(nbytes, dev_):
+        asked.append(nbytes)
+        if len(asked) == 1:
+            raise torch.OutOfMemoryError("no memory")
+        return plain(nbytes, dev_)
+
+    monkeypatch.setattr(_device, "workspace", full)
+    got = _device.gdn_forward(*args, num_seqs=1)
+    assert len(asked) == 2 and asked[0] - asked[1] == 2 * (N // 64 + 1) * G * (D // 16) * (D // 32 + 2) * 1536
+    for x, y in zip(got, ref):
+        assert ((x - y).norm() / y.norm()).item() < 4e-6
+    asked.clear()
+    with pytest.raises(torch.OutOfMemoryError):
+        _device.gdn_forward(*(x.bfloat16() for x in args[:3]), *args[3:], num_seqs=1)
