@@ -12,7 +12,7 @@ PHASE_PREP, PHASE_SUMMARY, PHASE_OUTPUT, PHASE_COMBINE = 1, 2, 4, 8
 PHASE_STATES, PHASE_ALL = PHASE_SUMMARY | PHASE_COMBINE, 15
 KV_MAX_K, KV_MAX_BLOCKS = 64, 16384      # bf_kv_select limits
 STUDENT_INPUTS_MAX = 256                 # bf_student_inputs_max_tokens()
-FEW_TOKENS = {DTYPE_F32: (12,) * 8, DTYPE_BF16: (8,) * 4 + (4,) * 4}    # bf_layer_few_tokens(R, dtype) for R = 1 .. 8, 0 above
+FEW_TOKENS = {DTYPE_F32: (12,) * 8, DTYPE_BF16: (8,) * 4 + (5,) * 4}    # bf_layer_few_tokens(R, dtype) for R = 1 .. 8, 0 above
 
 _c_int, _c_i64, _c_sz, _vp, _fp = ctypes.c_int, ctypes.c_int64, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_float
 
