@@ -63,8 +63,19 @@ struct GdnArgs {
 // scan / at once: 1 x 64, H = 2: 28 / 32; 1 x 300, H = 16: 46 / 41; 1 x 3000, H = 16: 84 / 87; 1 x 5000, H = 16: 125 / 132; 3 x 10000,
 // H = 16: 915 / 832; there the scan keeps them.
 inline size_t gdn_plane_elems(long max_chunks, int G, int D) { return (size_t)max_chunks * G * (D / 16) * (D / 32 + 2) * 1536; }
-inline bool gdn_out_split(long max_chunks, int G, int R, int D, int in_dtype) {
-    return in_dtype == DT_F32 && (R >= 2 || D >= 128) && 2 * gdn_plane_elems(max_chunks, G, D) <= (size_t)2 << 30;
+// With many sequences the scan's workgroups (num_seqs G of D / 128 parts) fill the chip by themselves, and the planes only cost
+// their bytes: the less so the more heads read a chunk's state and the longer the chains are. us in the scan / at once, workgroups
+// in brackets: sequences of 64 tokens, R = 1, D = 128 [96] 43 / 39, [192] 52 / 57, [1024] 395 / 578; D = 256 [192] 71 / 69, [256]
+// 83 / 90; R = 2, D = 64 [16] 25 / 24, [128] 32 / 35; R = 4, D = 64 [128] 38 / 37, [256] 44 / 47; R = 2, D = 256 [256] 105 / 101, [512]
+// 227 / 239; R = 4, D = 256 [1024] 770 / 772; R = 6 [2048] 1831 / 1566. Of 256 tokens or more, R = 1, D = 128 [192] 128 / 118, [256]
+// 154 / 169; D = 256 [192] 203 / 182, [256] 221 / 247; R = 2, D = 64 [128] 105 / 99, [256] 97 / 112; R = 2, D = 128 [384] 379 / 318, [512]
+// 444 / 454; R = 4, D = 128 [800] 1269 / 942; R = 8, D = 64 [512] 406 / 424.
+inline bool gdn_out_split(long max_chunks, int num_seqs, int G, int R, int D, int in_dtype) {
+    if (in_dtype != DT_F32 || (R < 2 && D < 128) || 2 * gdn_plane_elems(max_chunks, G, D) > (size_t)2 << 30) return false;
+    const long wgs = (long)num_seqs * G * (D > 128 ? 2 : 1);
+    const bool chains = (max_chunks - num_seqs) / num_seqs >= 4;          // (max_chunks: the tokens / 64 and one per sequence)
+    const int quarters = D < 128 ? (chains ? 4 : 2) : R == 1 ? (chains && D == 128 ? 6 : 3) : chains || (R >= 6 && D == 256) ? 6 : R >= 4 && D == 256 ? 4 : 3;
+    return 4 * wgs <= (long)quarters * R * D;
 }
 
 int gdn_prep(const GdnArgs& a, hipStream_t stream);

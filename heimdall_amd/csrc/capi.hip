@@ -98,7 +98,7 @@ GdnLayout gdn_layout(int64_t total_tokens, int num_seqs, int G, int R, int D, in
     L.n = off;    off = align256(off + ns * G * D * D * sizeof(float));
     L.sin = off;  off = align256(off + ns * G * D * D * sizeof(float));
     L.need = off;
-    const bool split = bf::gdn_out_split(L.max_chunks, G, R, D, in_dtype);
+    const bool split = bf::gdn_out_split(L.max_chunks, num_seqs, G, R, D, in_dtype);
     L.spl = split ? off : 0;
     if (split) off = align256(off + 2 * bf::gdn_plane_elems(L.max_chunks, G, D));
     L.total = off;

@@ -82,8 +82,8 @@ const char* bf_status_string(int status);
  * Chunk length is 64. Arithmetic: MFMA in in_dtype with fp32 accumulation (in fp32 the larger products as bf16 MFMAs over three
  * planes per operand, a product to within 3 * 2^-24; an infinite input ends as NaN); state, decay and the triangular
  * inverse in fp32; segment entry states composed in fp32 (split-bf16 MFMA for bf16 runs).
- * Workspace: bf_gdn_workspace_size bytes. For in_dtype fp32 with R >= 2 or D >= 128 its last part, unless that is over 2 GiB,
- *   is 2 (N_tok / 64 + num_seqs) G (D / 16) (D / 32 + 2) 1536 bytes, rounded up to 256, of bf16 planes: with them the outputs of
+ * Workspace: bf_gdn_workspace_size bytes. For in_dtype fp32 with R >= 2 or D >= 128 its last part, unless that is over 2 GiB or
+ *   the sequences are many, is 2 (N_tok / 64 + num_seqs) G (D / 16) (D / 32 + 2) 1536 bytes, rounded up to 256, of bf16 planes: with them the outputs of
  *   all chunks are formed at once after the scan. A workspace without that part (bf_gdn_workspace_min_size bytes) is accepted
  *   too and keeps the outputs in the scan: the same values to rounding, more slowly.
  */

@@ -81,6 +81,24 @@ def test_limits_match_the_library(cpu_lib):
     assert cpu_lib.bf_student_inputs_max_tokens() == _lib.STUDENT_INPUTS_MAX
 
 
+def test_planes_line(cpu_lib):
+    """fp32 scans reserve the planes (their outputs at once) while their sequences do not fill the chip, by heads and lengths."""
+    def planes(B, T, G, R, D, dtype=0):
+        n, m = ctypes.c_size_t(0), ctypes.c_size_t(0)
+        assert cpu_lib.bf_gdn_workspace_size(B * T, B, G, R, D, dtype, 0, ctypes.byref(n)) == 0
+        assert cpu_lib.bf_gdn_workspace_min_size(B * T, B, G, R, D, dtype, 0, ctypes.byref(m)) == 0
+        rest = 2 * (B * T // 64 + B) * G * (D // 16) * (D // 32 + 2) * 1536
+        assert n.value - m.value in (0, (rest + 255) // 256 * 256)
+        return n.value > m.value
+
+    for shape in ((1, 64, 4, 1, 128), (24, 64, 4, 1, 128), (48, 512, 4, 1, 128), (48, 64, 2, 1, 256), (1, 8192, 4, 6, 256), (4, 64, 4, 2, 64),
+                  (32, 256, 4, 2, 64), (64, 64, 4, 6, 256), (96, 256, 4, 2, 128)):
+        assert planes(*shape), shape
+    for shape in ((1, 64, 16, 1, 64), (48, 64, 4, 1, 128), (64, 512, 4, 1, 128), (64, 64, 2, 1, 256), (64, 512, 2, 1, 256), (32, 64, 4, 2, 64),
+                  (64, 256, 4, 2, 64), (64, 512, 8, 4, 64), (128, 256, 4, 2, 128), (3, 20000, 16, 1, 256), (1, 8192, 4, 6, 256, 1)):
+        assert not planes(*shape), shape
+
+
 def test_few_token_line(cpu_lib):
     """Tokens up to which a chunk's memory branch runs token by token, by query heads per KV head."""
     from heimdall_amd import _lib

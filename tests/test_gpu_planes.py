@@ -11,7 +11,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-N, R, D = 256, 2, 128
+N, R, D = 128, 2, 128
 
 
 def values(kind, shape, gen):
