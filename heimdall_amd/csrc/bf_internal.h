@@ -166,7 +166,7 @@ struct WinMap {
     long nrow, rpg, per;
     int R, f, rot;
 };
-__host__ __device__ inline WinMap window_map_make(int B, int G, int R, int T, int f, int rot) {
+__host__ __device__ inline WinMap window_map_make(int B, int G, int R, long T, int f, int rot) {
     WinMap m{};
     m.nrow = (long)B * G * ((T + 127) / 128);
     m.R = R;

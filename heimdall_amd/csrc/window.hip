@@ -386,8 +386,7 @@ static int launch_window(const WinArgs& args, hipStream_t stream) {
     WinArgs a = args;
     // the map counts 128-query items; 64-query ones are those of twice the length
     const int f = a.start < a.W ? 2 : 1;
-    if (a.T > (1 << 30)) return BF_STATUS_INVALID;
-    a.map = window_map_make(a.B, a.G, a.R, a.T * (8 / NW), f, 0);
+    a.map = window_map_make(a.B, a.G, a.R, a.T * (8L / NW), f, 0);
     if (8 * a.map.per > 0x7fffffffL) return BF_STATUS_INVALID;
     const dim3 grid((unsigned)(8 * a.map.per)), block(64 * NW);
     if (a.o_dtype == DT_BF16) hipLaunchKernelGGL((window_kernel<D, NW, true>), grid, block, 0, stream, a);
@@ -396,11 +395,16 @@ static int launch_window(const WinArgs& args, hipStream_t stream) {
     return e == hipSuccess ? 0 : (int)e;
 }
 
-// 64 queries per workgroup while that leaves every workgroup a CU of its own: one wave per SIMD, half the MFMAs of a block;
-// above, 128, which store each key block half as often.
+// 64 or 128 queries per workgroup: 128 store each key block half as often; 64 make twice the workgroups, each with half the
+// MFMAs of a block. 64 while every workgroup has a CU of its own (one wave per SIMD), where 128 would be half empty, and over
+// short windows at the smaller dims, whose items are mostly their first loads and their ends. us a launch, 64 / 128 queries:
+// 16 sequences of 20 queries, H = 16, D = 256, W = 2048 328 / 337; 200 of 20, D = 128, W = 64 149 / 282; 40 of 64, D = 128, W = 2048
+// 489 / 674; 4096 queries, H = 16, W = 2048 D = 256 1299 / 746, D = 128 559 / 476; H = 32, D = 64 764 / 682; 16 of 300, W = 256,
+// D = 256 319 / 256, D = 128 140 / 164, D = 64 (H = 32) 186 / 227; 3 of 2000, W = 512, D = 128 257 / 241, D = 64 (H = 8) 103 / 115.
 template <int D>
 static int launch_window_by_size(const WinArgs& a, hipStream_t stream) {
-    const bool few = (long)a.B * a.G * a.R * ((a.T + 63L) / 64) <= 256;
+    const long keys = a.start + a.T < a.W ? a.start + a.T : a.W;
+    const bool few = a.T <= 64 || (long)a.B * a.G * a.R * ((a.T + 63L) / 64) <= 256 || keys <= (D == 64 ? 1024 : D == 128 ? 256 : 0);
     return few ? launch_window<D, 4>(a, stream) : launch_window<D, 8>(a, stream);
 }
 

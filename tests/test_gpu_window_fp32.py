@@ -43,6 +43,12 @@ def reference(c):
     (3, 24, 4, 128, 300, 33, 1, 0, 0.0),
     (1, 96, 8, 64, 191, 200, 4, 150, 0.0),      # a ring that is not full
     (1, 8, 8, 64, 1, 16, 0, 40, 0.0),           # one query, no sinks
+    (40, 8, 2, 128, 64, 300, 2, 500, 0.1),      # many items of half a 128-query workgroup, and of one query more
+    (20, 8, 2, 128, 65, 300, 2, 500, 0.0),
+    (9, 16, 4, 128, 140, 256, 3, 700, 0.0),     # the last window of 64-query items, the first of 128, at either dim
+    (9, 16, 4, 128, 140, 257, 3, 700, 0.0),
+    (9, 16, 4, 64, 140, 1024, 3, 2000, 0.1),
+    (9, 16, 4, 64, 140, 1025, 3, 2000, 0.0),
 ])
 def test_window_fp32_tiles(dev, B, H, G, D, T, W, S, start, miss):
     c = make_case(B, H, G, D, T, W, S, start, seed=T + W, invalid_frac=miss, dtype=torch.float32)
