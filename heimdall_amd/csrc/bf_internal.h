@@ -391,6 +391,7 @@ struct FrontArgs {
 };
 int student_front(FrontArgs& a, bool finish, hipStream_t stream);
 int window_fa_dispatch(const WinArgs& a, hipStream_t stream);
+int window_d64_dispatch(const WinArgs& a, hipStream_t stream);
 
 struct KvArgs {
     int B, T, G, R, D, dtype;       // T queries per sequence at positions n - T .. n - 1; q, k, v dtype (f32 / bf16)

@@ -1,6 +1,7 @@
 // K2, fp32 operands: exact sliding-window + sink attention over a prefill chunk, with per-row log-sum-exp and the fused
 // gamma mix.
 //
+// (D = 64 over few queries or a short window: window_d64.hip.)
 // Reference: HybridAttention._window_fp32 (Heimdall/heimdall/hibrit.py:341-361) and the mix of :409-411.
 // Query i of the chunk sits at absolute position p = start + i. Visible keys (mask of hibrit.py:356):
 //   sinks j < n_sinks with j <= p, and window keys at positions kp with S <= kp <= p, p - kp < W, where
@@ -401,10 +402,14 @@ static int launch_window(const WinArgs& args, hipStream_t stream) {
 // 16 sequences of 20 queries, H = 16, D = 256, W = 2048 328 / 337; 200 of 20, D = 128, W = 64 149 / 282; 40 of 64, D = 128, W = 2048
 // 489 / 674; 4096 queries, H = 16, W = 2048 D = 256 1299 / 746, D = 128 559 / 476; H = 32, D = 64 764 / 682; 16 of 300, W = 256,
 // D = 256 319 / 256, D = 128 140 / 164, D = 64 (H = 32) 186 / 227; 3 of 2000, W = 512, D = 128 257 / 241, D = 64 (H = 8) 103 / 115.
+// At D = 64 the 64-query form is for 32 queries or fewer over more than 128 keys (64 sequences of 20, H = 8, W = 256: 36 us against
+// 43); otherwise the fp32 MFMAs on unsplit rows are faster (window_d64.hip).
 template <int D>
 static int launch_window_by_size(const WinArgs& a, hipStream_t stream) {
     const long keys = a.start + a.T < a.W ? a.start + a.T : a.W;
     const bool few = a.T <= 64 || (long)a.B * a.G * a.R * ((a.T + 63L) / 64) <= 256 || keys <= (D == 64 ? 1024 : D == 128 ? 256 : 0);
+    if constexpr (D == 64)
+        if (few && (a.T > 32 || keys <= 128) && a.B <= 65535 && (long)a.G * a.R <= 65535) return window_d64_dispatch(a, stream);
     return few ? launch_window<D, 4>(a, stream) : launch_window<D, 8>(a, stream);
 }
 

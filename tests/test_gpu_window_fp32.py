@@ -43,6 +43,11 @@ def reference(c):
     (3, 24, 4, 128, 300, 33, 1, 0, 0.0),
     (1, 96, 8, 64, 191, 200, 4, 150, 0.0),      # a ring that is not full
     (1, 8, 8, 64, 1, 16, 0, 40, 0.0),           # one query, no sinks
+    (1, 4, 2, 64, 33, 400, 3, 900, 0.1),        # D = 64: unsplit rows from 33 queries on, or up to 128 keys
+    (1, 4, 2, 64, 32, 400, 3, 900, 0.1),
+    (2, 4, 1, 64, 20, 128, 3, 900, 0.0),
+    (2, 4, 1, 64, 20, 129, 3, 900, 0.0),
+    (3, 4, 2, 64, 130, 70, 2, 0, 0.0),
     (40, 8, 2, 128, 64, 300, 2, 500, 0.1),      # many items of half a 128-query workgroup, and of one query more
     (20, 8, 2, 128, 65, 300, 2, 500, 0.0),
     (9, 16, 4, 128, 140, 256, 3, 700, 0.0),     # the last window of 64-query items, the first of 128, at either dim
